@@ -102,6 +102,10 @@ size_t order_temp_bytes(int n);
 hipError_t order_update(const double* rec, size_t rec_stride, int ctl_off, int n, int* prev_nst, int* bucket,
                         int* rank, int* order_out, void* temp, hipStream_t stream);
 
+// width doubles of each of `rows` records (record r at src + r stride) into a
+// dense rows x width array on the device
+hipError_t pack_rows(const double* src, size_t stride, int width, int rows, double* dst, hipStream_t stream);
+
 // guarded surrogate steps for reactor batches (all on the device)
 size_t guard_lds_bytes(const DevMech& m, int ns);
 const void* guard_kernel_ptr(int ns);

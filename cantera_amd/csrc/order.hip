@@ -13,6 +13,8 @@
 // which wavefront integrates which reactor, never a reactor's result.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "bdf.hpp"
 
 namespace cg {
@@ -83,7 +85,26 @@ __global__ void scatter_kernel(int n, const int* __restrict__ bucket, const int*
     order[offs[bucket[r]] + rank[r]] = r;
 }
 
+// One column block of consecutive reactor records into a dense array (see
+// pack_rows): one thread per value, so neighbouring threads read neighbouring
+// values of a record.
+__global__ __launch_bounds__(256) void pack_rows_kernel(const double* __restrict__ src, size_t stride, int width,
+                                                        size_t total, double* __restrict__ dst) {
+    for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < total;
+         i += static_cast<size_t>(gridDim.x) * blockDim.x) {
+        const size_t r = i / static_cast<unsigned>(width);
+        dst[i] = src[r * stride + (i - r * width)];
+    }
+}
+
 }  // namespace
+
+hipError_t pack_rows(const double* src, size_t stride, int width, int rows, double* dst, hipStream_t stream) {
+    const size_t total = static_cast<size_t>(rows) * width;
+    const unsigned grid = static_cast<unsigned>(std::min<size_t>((total + 255) / 256, 4096));
+    hipLaunchKernelGGL(pack_rows_kernel, dim3(grid), dim3(256), 0, stream, src, stride, width, total, dst);
+    return hipGetLastError();
+}
 
 size_t order_temp_bytes(int) { return 2 * kBuckets * sizeof(int); }
 
