@@ -1411,27 +1411,24 @@ struct Integrator {
 // LDS per wavefront: state broadcast, species/reaction scratch, control block,
 // then the linear-system area (LDS policy only).
 __host__ __device__ inline size_t bdf_scratch_doubles(int K, int ns) {
-    return static_cast<size_t>(kWave) * ns * 4 + (K + 1) + (K + 1) + K + 2 * K + kCtlDoubles;
+    return static_cast<size_t>(kWave) * ns * 4 + species_doubles(K) + 2 * K + kCtlDoubles;
 }
 
 template <int NS, class LS, typename MT, bool kSens = false, bool kMole = false>
 __device__ __forceinline__ void bdf_advance_body(const BdfArgs& a) {
     const DevMech& m = a.mech;
     ScratchLayout L;
-    int off = 0;
+    int off = species_doubles(m.K);
     L.yb = off;  off += kWave * NS;
     L.F = off;   off += kWave * NS;
     L.Y0 = off;  off += kWave * NS;
     L.F0 = off;  off += kWave * NS;
-    L.C = off;   off += m.K + 1;
-    L.MU = off;  off += m.K + 1;
-    L.WD = off;  off += m.K;
     L.W2 = off;  off += 2 * m.K;
     double* base = lds_base() + off;
     Ctl& c = *reinterpret_cast<Ctl*>(base);
     base += kCtlDoubles;
     Integrator<NS, LS, MT, kSens, kMole> it(m, a, c);
-    it.S = scratch_view(L);
+    it.S = scratch_view(L, kernarg_mech());
     it.L = L;
     it.lane = lane_id();
     it.N = kMole ? m.K + 1 + (m.const_volume ? 1 : 0) : m.N;

@@ -178,6 +178,28 @@ bool expand_side(const std::vector<int>& k, const std::vector<double>& order,
     return krep.size() >= 1 && krep.size() <= 3;
 }
 
+// The molecules of a side one by one, if every coefficient is a whole number;
+// returns false otherwise.
+bool expand_molecules(const std::vector<int>& k, const std::vector<double>& st, std::vector<int>& out) {
+    out.clear();
+    for (size_t n = 0; n < st.size(); n++) {
+        if (std::fmod(st[n], 1.0) != 0.0 || st[n] < 0 || st[n] > 4) return false;
+        for (int i = 0; i < st[n]; i++) out.push_back(k[n]);
+    }
+    return true;
+}
+
+// Reactions that the compact record (RxnS) describes.  A reversible reaction's
+// products must take the repeated-species multiply rules; an irreversible
+// one's only receive the rate of progress, so four of them will do.
+bool is_standard(const HostReaction& r) {
+    if (r.type == kPlog || r.type == kChebyshev || r.type == kSri || r.chem_act) return false;
+    std::vector<int> sp;
+    if (!expand_side(r.rk, r.ro, r.rs, sp)) return false;
+    if (r.rev) return expand_side(r.pk, r.ps, r.ps, sp);
+    return expand_molecules(r.pk, r.ps, sp) && sp.size() <= 4;
+}
+
 }  // namespace
 
 DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
@@ -193,24 +215,42 @@ DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
     // pass that runs the Troe code for a few lanes.  PLOG and Chebyshev
     // reactions (types 4, 5) lead: their rate constants are evaluated once per
     // state by lanes 0..63 before the reaction loop.
-    // Class order: Chebyshev, PLOG, Tsang, SRI, Troe, Lindemann, three-body, elementary.
+    // Class order: Chebyshev, PLOG, then the other reactions that need the
+    // general code (SRI, power-law orders, ...), then the standard ones: Tsang,
+    // Troe, Lindemann, three-body, elementary.
     static const int kRank[8] = {7, 6, 5, 4, 1, 0, 3, 2};   // by RxnType
-    std::stable_sort(perm_.begin(), perm_.end(),
-                     [&](int a, int b) { return kRank[h.rxn[a].type] < kRank[h.rxn[b].type]; });
+    std::vector<int> key(I);
+    for (int i = 0; i < I; i++) {
+        const int t = h.rxn[i].type;
+        key[i] = kRank[t] + ((t == kPlog || t == kChebyshev || !is_standard(h.rxn[i])) ? 0 : 8);
+    }
+    std::stable_sort(perm_.begin(), perm_.end(), [&](int a, int b) { return key[a] < key[b]; });
 
-    std::vector<double> rd(4 * static_cast<size_t>(I)), tbdef(I), fod, gend, pdd;
-    std::vector<RxnI> ri(I);
-    std::vector<int> tbk;
-    std::vector<double> tbe;
+    // every per-reaction table is filled up with null reactions to whole
+    // wavefront passes
+    const int Ip = (I + 63) / 64 * 64;
+    std::vector<double> rd(4 * static_cast<size_t>(Ip), 0.0), tbdef(Ip, 0.0), fod, gend, pdd;
+    std::vector<RxnI> ri(Ip);
+    std::vector<RxnS> rs(Ip);
+    for (int p = 0; p < Ip; p++) {
+        const unsigned short none = static_cast<unsigned short>(16 * (K + p % kDummy));
+        for (unsigned short& e : rs[p].r) e = none;
+        for (unsigned short& e : rs[p].p) e = none;
+        rs[p].flags = 0;
+        std::memset(&ri[p], 0, sizeof(RxnI));
+        ri[p].fo = ri[p].gen = -1;
+        for (int j = 0; j < kMaxSide; j++) ri[p].rk[j] = ri[p].pk[j] = static_cast<short>(K);
+    }
+    int n_gen = 0, n_nonplain = 0;
+    // the first group of the efficiency table is null: reactions without a
+    // list read it
+    std::vector<int> tbk(kTbPad, K);
+    std::vector<double> tbe(kTbPad, 0.0);
     int n_el = 0, n_tb = 0, n_fo = 0, n_pd = 0;
     for (int p = 0; p < I; p++) {
         const HostReaction& r = h.rxn[perm_[p]];
         RxnI& x = ri[p];
-        std::memset(&x, 0, sizeof x);
-        for (int j = 0; j < kMaxSide; j++) { x.rk[j] = static_cast<short>(K); x.pk[j] = static_cast<short>(K); }
         x.orig = perm_[p];
-        x.fo = -1;
-        x.gen = -1;
         // PLOG and Chebyshev reactions are mass-action reactions (type 0 on
         // the device) whose rate constant comes from their pdd record
         // SRI and Tsang are falloff reactions of the Troe form (type 3; SRI
@@ -249,7 +289,17 @@ DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
                 for (int j = 0; j < x.np; j++) x.pk[j] = static_cast<short>(r.pk[j]);
             }
         }
-        if (dtype == kElementary && !(x.flags & (64 | 128)) && !rgen && !pgen) x.flags |= 1024;
+        if (key[perm_[p]] < 8) {
+            n_gen = p + 1;
+        } else {
+            std::vector<int> sp;
+            expand_molecules(r.rk, r.rs, sp);
+            for (size_t j = 0; j < sp.size(); j++) rs[p].r[j] = static_cast<unsigned short>(16 * sp[j]);
+            expand_molecules(r.pk, r.ps, sp);
+            for (size_t j = 0; j < sp.size(); j++) rs[p].p[j] = static_cast<unsigned short>(16 * sp[j]);
+            rs[p].flags = static_cast<unsigned short>((r.rev ? 1 : 0) | (sp.size() > 3 ? 2 : 0));
+        }
+        if (dtype != kElementary) n_nonplain = p + 1;
         if (rgen || pgen) {
             x.flags |= (rgen ? 8 : 0) | (pgen ? 16 : 0);
             x.gen = static_cast<int>(gend.size() / 12);
@@ -308,39 +358,42 @@ DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
         }
         if (dtype != kElementary) {
             if (r.tbk.size() > kMaxTB) throw std::runtime_error("too many third-body efficiencies");
-            x.tbo = static_cast<int>(tbk.size());
+            x.tbo = r.tbk.empty() ? 0 : static_cast<int>(tbk.size());
             x.tbn = static_cast<int>(r.tbk.size());
             tbk.insert(tbk.end(), r.tbk.begin(), r.tbk.end());
             tbe.insert(tbe.end(), r.tbe.begin(), r.tbe.end());
+            // up to whole groups of kTbPad: species K (concentration 1) at efficiency 0
+            tbk.resize((tbk.size() + kTbPad - 1) / kTbPad * kTbPad, K);
+            tbe.resize(tbk.size(), 0.0);
         }
     }
+    fod.insert(fod.end(), 8, 0.0);
 
     std::vector<double> nasa(16 * static_cast<size_t>(K), 0.0), rmw(K);
     for (int k = 0; k < K; k++) {
-        nasa[16 * k] = h.tmid[k];
-        for (int j = 0; j < 7; j++) { nasa[16 * k + 1 + j] = h.clow[7 * k + j]; nasa[16 * k + 8 + j] = h.chigh[7 * k + j]; }
+        nasa[16 * k + 7] = h.tmid[k];
+        for (int j = 0; j < 7; j++) { nasa[16 * k + j] = h.clow[7 * k + j]; nasa[16 * k + 8 + j] = h.chigh[7 * k + j]; }
         rmw[k] = 1.0 / h.mw[k];
     }
 
     d_.K = K; d_.I = I; d_.N = K + 2; d_.E = h.E;
     d_.n_el = n_el; d_.n_tb = n_tb; d_.n_fo = n_fo;
     d_.n_pd = n_pd;
+    d_.gen_end = (n_gen + 63) / 64;
+    d_.tb_end = std::max(d_.gen_end, (n_nonplain + 63) / 64);
     if (n_pd > 64) throw std::runtime_error("mechanisms with more than 64 PLOG and Chebyshev reactions are not supported");
     d_.pref = h.pref.empty() ? 101325.0 : h.pref[0];
+    d_.rpref = 1.0 / d_.pref;
     d_.mw = upload(h.mw);
     d_.rmw = upload(rmw);
     d_.nasa = upload(nasa);
     d_.rd = upload(rd);
     d_.tbdef = upload(tbdef);
     d_.ri = upload(ri);
+    d_.rs = upload(rs);
     d_.fod = upload(fod);
     d_.gend = upload(gend);
     d_.pdd = upload(pdd);
-    // kTbPad entries of padding (species K, whose concentration slot holds 1,
-    // efficiency 0) after the last list: the first kTbPad efficiencies of any
-    // reaction are loaded without a test against its list length
-    tbk.insert(tbk.end(), kTbPad, K);
-    tbe.insert(tbe.end(), kTbPad, 0.0);
     d_.tbk = upload(tbk);
     d_.tbe = upload(tbe);
     d_.comp = upload(h.comp);

@@ -12,7 +12,8 @@ namespace cg {
 
 constexpr int kMaxSide = 4;   // species entries per reaction side on the device
 constexpr int kMaxTB = 32;    // explicit efficiencies per reaction
-constexpr int kTbPad = 8;     // padding entries after the efficiency table
+constexpr int kTbPad = 8;     // efficiency lists are padded to a multiple of this many entries
+constexpr int kDummy = 64;    // sentinel species slots K .. K+63 in the kernels' scratch
 
 enum RxnType { kElementary = 0, kThreeBody = 1, kLindemann = 2, kTroe = 3, kPlog = 4, kChebyshev = 5, kSri = 6, kTsang = 7 };
 
@@ -71,20 +72,39 @@ struct RxnI {
 };
 static_assert(sizeof(RxnI) == 48, "RxnI layout");
 
+// Compact record of a standard reaction: both sides unit-stoichiometry lists of
+// at most three molecules (four products if irreversible), a rate constant of
+// Arrhenius, three-body, Lindemann or Troe form.  Each entry is the byte offset
+// of the species' (C, mu) pair in the kernels' scratch (16 x slot).  Unused entries
+// point at the sentinel slot K + (reaction % kDummy), where C = 1 and mu = 0:
+// every sum and product runs without tests, and the lanes of a pass, which
+// hold consecutive reactions, add their unused entries to slots of their own
+// instead of serialising on one address.
+struct alignas(16) RxnS {
+    unsigned short r[3], p[4];
+    unsigned short flags;        // bit0 reversible, bit1 a fourth product
+};
+static_assert(sizeof(RxnS) == 16, "RxnS layout");
+
 // Device view of a mechanism (all pointers are device pointers).
 struct DevMech {
     int K, I, N, E;          // species, reactions, state size (K+2), elements
     int n_el, n_tb, n_fo;    // reactions of each class, in permuted order:
-                             // [Chebyshev | PLOG | Troe | Lindemann | three-body | elementary]
+                             // [Chebyshev | PLOG | other non-standard | Troe | Lindemann | three-body | elementary]
+    int gen_end, tb_end;     // wavefront passes of 64 reactions: [0, gen_end) hold the non-standard reactions
+                             // (evaluated by the general code), [gen_end, tb_end) the other falloff and
+                             // three-body ones, the rest is elementary
     int n_pd;                // PLOG + Chebyshev reactions (the first n_pd, at most 64)
-    double pref;
+    double pref, rpref;      // reference pressure and its reciprocal
     const double* mw;        // K
     const double* rmw;       // K
-    const double* nasa;      // K x 16: tmid, low[7], high[7], pad
-    const double* rd;        // I x 4: A, b, EaR, dn
-    const double* tbdef;     // I
-    const RxnI* ri;          // I
-    const double* fod;       // n_fo x 8: A0, b0, EaR0, then Troe a, 1/T3, 1/T1, T2, B (Tsang: a = A, 1/T3 = inf,
+    const double* nasa;      // K x 16: low[7], tmid, high[7], pad
+    // per-reaction tables: I entries and null reactions (A = 0, no species) up to a multiple of 64
+    const double* rd;        // 4 each: A, b, EaR, dn
+    const double* tbdef;
+    const RxnI* ri;
+    const RxnS* rs;          // valid for standard and null reactions
+    const double* fod;       // (n_fo + 1) x 8, the last all zero: A0, b0, EaR0, then Troe a, 1/T3, 1/T1, T2, B (Tsang: a = A, 1/T3 = inf,
                              // 1/T1 = 0, T2 = 0, B) or SRI a, b, c, d, e
     const double* gend;      // n_gen x 12: reactant order[4], reactant stoich[4], product stoich[4]
     const int* tbk;          // efficiency species

@@ -18,20 +18,15 @@ namespace cg {
 
 namespace {
 
-// At most 168 VGPRs, so that three wavefronts share a SIMD (latency-bound
-// kernel; without the bound the allocator settles at 169 for NS = 1).
+// At most 168 VGPRs, so that three wavefronts share a SIMD: two elementary
+// passes side by side fit without spills (three spill).
 template <int NS, bool kF32>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void rates_kernel(
     DevMech m, long n, const double* __restrict__ T, const double* __restrict__ P, const double* __restrict__ Y,
     double* __restrict__ wdot) {
-    extern __shared__ double lds_raw[];
     const int lane = lane_id();
-    double* base = lds_raw;
     WaveScratch S{};
-    S.yb = base;  base += kWave * NS;
-    S.C = base;   base += m.K + 1;
-    S.MU = base;  base += m.K + 1;
-    S.WD = base;
+    bind_species(S, kernarg_mech());
     const XcdStates xs(n);
     for (long st = xs.lo; st < xs.hi; st += xs.step) {
         const double Ts = uni(T[st]);
@@ -45,7 +40,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void ra
         GasState g;
         SpeciesRegs<NS> sr;
         species_pass<NS, true>(m, S, Ts, Ps, yk, g, sr);
-        production_rates<NS, kF32>(m, S, g, sr);
+        production_rates<NS, kF32, false, 2>(m, S, g, sr);
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             const int k = lane + kWave * s;
@@ -61,14 +56,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void ra
 template <int NS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void reactor_rates_kernel(
     DevMech m, long n, const double* __restrict__ rec, size_t stride, int cv, double* __restrict__ wdot) {
-    extern __shared__ double lds_raw[];
     const int lane = lane_id();
-    double* base = lds_raw;
     WaveScratch S{};
-    S.yb = base;  base += kWave * NS;
-    S.C = base;   base += m.K + 1;
-    S.MU = base;  base += m.K + 1;
-    S.WD = base;
+    bind_species(S, kernarg_mech());
     constexpr int NP = kWave * NS;
     const XcdStates xs(n);
     for (long st = xs.lo; st < xs.hi; st += xs.step) {
@@ -85,7 +75,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void re
         GasState g;
         SpeciesRegs<NS> sr;
         species_pass<NS, true>(m, S, Ts, cv ? 0.0 : pv, yk, g, sr, cv ? mass / pv : 0.0);
-        production_rates<NS, false>(m, S, g, sr);
+        production_rates<NS, false, false, 2>(m, S, g, sr);
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             const int k = lane + kWave * s;
@@ -116,8 +106,7 @@ const void* reactor_rates_kernel_ptr(int ns) {
 }
 
 size_t rates_lds_bytes(const DevMech& m, int ns) {
-    const size_t d = static_cast<size_t>(kWave) * rates_ns(ns) + 2 * (m.K + 1) + m.K;
-    return d * sizeof(double);
+    return static_cast<size_t>(species_doubles(m.K)) * sizeof(double);
 }
 
 hipError_t rates_launch(const DevMech& m, int ns, bool f32, long n, const double* T, const double* P,

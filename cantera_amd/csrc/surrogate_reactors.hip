@@ -122,16 +122,13 @@ __global__ __launch_bounds__(64) void guard_kernel(GuardArgs a) {
     const DevMech& m = a.m;
     const int lane = lane_id();
     ScratchLayout L;
-    int off = 0;
+    int off = species_doubles(m.K);
     L.yb = off;  off += kWave * NS;
     L.F = off;   off += kWave * NS;
     L.Y0 = off;  off += kWave * NS;
     L.F0 = off;  off += kWave * NS;
-    L.C = off;   off += m.K + 1;
-    L.MU = off;  off += m.K + 1;
-    L.WD = off;  off += m.K;
     L.W2 = off;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, kernarg_mech());
     const int N = m.N, K = m.K;
     for (int i = blockIdx.x; i < a.n; i += gridDim.x) {
         if (uni(a.elig[i]) != 1) continue;
@@ -285,7 +282,7 @@ __global__ void clear_ints_kernel(int* p, int n) {
 }  // namespace
 
 size_t guard_lds_bytes(const DevMech& m, int ns) {
-    const size_t d = static_cast<size_t>(kWave) * ns * 4 + 2 * (m.K + 1) + m.K + 2 * m.K;
+    const size_t d = static_cast<size_t>(kWave) * ns * 4 + species_doubles(m.K) + 2 * m.K;
     return d * sizeof(double);
 }
 

@@ -28,7 +28,7 @@ __device__ __forceinline__ void mat_add(double* p, double v) { unsafeAtomicAdd(p
 // bit 0 leaves out the third-body [M] terms, bit 1 the falloff d k/d[M]
 // (the rate then counts as linear in [M], BulkKinetics.cpp:761-792).
 __device__ __forceinline__ void scatter_reaction_derivs(const DevMech& m, int p, const GasState& g,
-                                                        const double* __restrict__ C, const double* __restrict__ MU,
+                                                        SpeciesColumn C, SpeciesColumn MU,
                                                         double kpd, double* A, int LD, double* acc, int skip = 0) {
     RxnRegs x;
     load_rxn(m, p, x);
@@ -295,7 +295,7 @@ __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const WaveScr
 template <int NS>
 __device__ __noinline__ void jac_call(KernargMech* mech, ScratchLayout L, double P, double* J) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     double y[NS], f0[NS];
 #pragma unroll
@@ -314,7 +314,7 @@ __device__ __noinline__ void jac_call(KernargMech* mech, ScratchLayout L, double
 template <int NS>
 __device__ __noinline__ void jac_lds_call(KernargMech* mech, ScratchLayout L, double P, int offJ, double* Jsave) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     double y[NS], f0[NS];
 #pragma unroll

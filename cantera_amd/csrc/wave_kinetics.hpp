@@ -171,35 +171,65 @@ struct XcdStates {
     }
 };
 
+// The mechanism of a kernel whose first parameter is a DevMech, or a struct
+// that begins with one, addressed in the kernel-argument segment.  Out-of-line
+// functions take this pointer rather than a reference to the kernel's copy of
+// the argument: a reference would make the kernel keep that copy in scratch
+// memory and read every field through it, while the kernel-argument segment is
+// read with scalar loads.
+using KernargMech = const __attribute__((address_space(4))) DevMech;
+__device__ __forceinline__ KernargMech* kernarg_mech() {
+    return (KernargMech*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// One member of the interleaved (C, mu) pairs of the scratch.
+struct SpeciesColumn {
+    double* p;
+    __device__ __forceinline__ double& operator[](int k) const { return p[2 * k]; }
+};
+
 // Per-wave LDS scratch for one state evaluation.
 struct WaveScratch {
+    // K + kDummy pairs at the start of dynamic LDS: C [kmol/m^3] and mu/RT at
+    // the state's pressure, (1, 0) from K on.  One 16-byte read serves a
+    // species of a reaction's product and of its equilibrium constant, at the
+    // address that the compact reaction record holds.
+    SpeciesColumn C, MU;
+    double* WD;    // K + kDummy production-rate accumulators, right behind the pairs
     double* yb;    // N (state broadcast)
-    double* C;     // K + 1 concentrations (C[K] = 1: the unused-slot sentinel of RxnI)
-    double* MU;    // K + 1 standard chemical potentials [J/kmol] (MU[K] = 0)
-    double* WD;    // K production-rate accumulators
     double* W2;    // 2K (Jacobian: wdot, D)
     double* F;     // N (right-hand side out)
     double* Y0;    // N (Jacobian expansion point)
     double* F0;    // N (right-hand side at Y0)
+    KernargMech* mech;   // for out-of-line callees
 };
+
+__host__ __device__ __forceinline__ int species_doubles(int K) { return 3 * (K + kDummy); }
 
 // The same scratch as offsets (in doubles) from the start of dynamic LDS, for
 // passing to out-of-line device functions: pointers rebuilt from the LDS base
 // inside the callee keep the LDS address space (ds_* instructions).
 struct ScratchLayout {
-    int yb, C, MU, WD, W2, F, Y0, F0;
+    int yb, W2, F, Y0, F0;
 };
 
 __device__ __forceinline__ double* lds_base() {
-    extern __shared__ double lds_raw[];
+    extern __shared__ __attribute__((aligned(16))) double lds_raw[];
     return lds_raw;
 }
 
-__device__ __forceinline__ WaveScratch scratch_view(const ScratchLayout& L) {
+__device__ __forceinline__ void bind_species(WaveScratch& S, KernargMech* mech) {
+    S.mech = mech;
+    S.C.p = lds_base();
+    S.MU.p = lds_base() + 1;
+    S.WD = lds_base() + 2 * (mech->K + kDummy);
+}
+
+__device__ __forceinline__ WaveScratch scratch_view(const ScratchLayout& L, KernargMech* mech) {
     double* b = lds_base();
     WaveScratch S;
-    S.yb = b + L.yb; S.C = b + L.C; S.MU = b + L.MU; S.WD = b + L.WD;
-    S.W2 = b + L.W2; S.F = b + L.F; S.Y0 = b + L.Y0; S.F0 = b + L.F0;
+    bind_species(S, mech);
+    S.yb = b + L.yb; S.W2 = b + L.W2; S.F = b + L.F; S.Y0 = b + L.Y0; S.F0 = b + L.F0;
     return S;
 }
 
@@ -215,7 +245,7 @@ __device__ __forceinline__ double add_mul_rn(double c, double a, double b) {
 }
 
 struct GasState {
-    double T, P, mmw, RT, dens, ctot, pressure, logT, recipT, rrt, logC0, tmp;
+    double T, P, mmw, RT, dens, ctot, pressure, logT, recipT, logC0;
 };
 
 // Values one lane keeps for the species it owns (slot s = species lane + 64 s).
@@ -226,7 +256,15 @@ struct SpeciesRegs {
 
 template <typename R>
 __device__ __forceinline__ void nasa7(const double* __restrict__ c16, double T, const double* tt, R& cp, R& h, R& s, R& g) {
-    const double* c = (T <= c16[0]) ? c16 + 1 : c16 + 8;
+    // both coefficient sets are loaded: chosen by address, the loads would wait
+    // for tmid first, a second trip to memory
+    double c[7];
+    const bool low = T <= c16[7];
+#pragma unroll
+    for (int j = 0; j < 7; j++) {
+        const double a = opaque(c16[j]), b = opaque(c16[8 + j]);
+        c[j] = low ? a : b;
+    }
     double ct0 = c[0];
     double ct1 = c[1] * tt[0];
     double ct2 = c[2] * tt[1];
@@ -267,6 +305,178 @@ __device__ __forceinline__ void load_rxn(const DevMech& m, int p, RxnRegs& x) {
     x.pk[2] = static_cast<short>(c.w & 0xffff); x.pk[3] = static_cast<short>(c.w >> 16);
 }
 
+// exp(x) without branches or special-case selects: x = n ln 2 + r, |r| <= ln(2)/2
+// (both subtractions exact to the last bit through the fused multiply-adds),
+// exp(r) = 1 + r + r^2 q(r) with q the degree-9 minimax polynomial of the
+// relative error (3.7e-18, Remez exchange), scaled by v_ldexp, which gives
+// infinity, subnormals and zero by itself.  Error below 0.63 ulp.  Arguments
+// are finite (an infinite one gives NaN) and below 1e13 in magnitude.
+constexpr double kLog2e = 1.4426950408889634;
+constexpr double kLn2Hi = 0x1.62e42fefa39efp-1, kLn2Lo = 0x1.abc9e3b39803fp-56;
+constexpr double kExpC[10] = {0x1.ad7f3cdbe6745p-26, 0x1.28ad9ef903086p-22, 0x1.71df25b30699dp-19,
+                              0x1.a01999de1245bp-16, 0x1.a01a012a0f6c4p-13, 0x1.6c16c1843a8b2p-10,
+                              0x1.1111111127d0fp-7,  0x1.5555555550834p-5,  0x1.55555555554f9p-3,
+                              0x1.000000000000ap-1};
+__device__ __forceinline__ double fast_exp(double x) {
+    const double n = rint(x * kLog2e);
+    double r = fma(n, -kLn2Hi, x);
+    r = fma(n, -kLn2Lo, r);
+    double q = kExpC[0];
+#pragma unroll
+    for (int j = 1; j < 10; j++) q = fma(q, r, kExpC[j]);
+    q = fma(q, r, 1.0);
+    q = fma(q, r, 1.0);
+    return ldexp(q, static_cast<int>(n));
+}
+
+// M exponentials side by side, the same operations as fast_exp.  One wavefront
+// per SIMD evaluates a chain of 13 dependent FMAs at its latency unless other
+// chains fill the gaps, and the scheduler, which orders for register pressure,
+// does one chain after the other (a library exp also copies each coefficient
+// into the destination, v_mov + v_fmac); written out, M chains advance together
+// with the coefficients in scalar registers.
+template <int M>
+__device__ __forceinline__ void fast_exp_n(double (&x)[M]);
+template <>
+__device__ __forceinline__ void fast_exp_n<2>(double (&x)[2]) {
+    double n[2], q[2];
+    asm(
+        "v_mul_f64 %2, %0, %4\nv_mul_f64 %3, %1, %4\n"
+        "v_rndne_f64 %2, %2\nv_rndne_f64 %3, %3\n"
+        "v_fma_f64 %0, %2, %5, %0\nv_fma_f64 %1, %3, %5, %1\n"
+        "v_fma_f64 %0, %2, %6, %0\nv_fma_f64 %1, %3, %6, %1\n"
+        : "+v"(x[0]), "+v"(x[1]),
+          "=&v"(n[0]), "=&v"(n[1])
+        : "s"(kLog2e), "s"(-kLn2Hi), "s"(-kLn2Lo));
+    asm(
+        "v_fma_f64 %0, %2, %4, %5\nv_fma_f64 %1, %3, %4, %5\n"
+        "v_fma_f64 %0, %0, %2, %6\nv_fma_f64 %1, %1, %3, %6\n"
+        "v_fma_f64 %0, %0, %2, %7\nv_fma_f64 %1, %1, %3, %7\n"
+        "v_fma_f64 %0, %0, %2, %8\nv_fma_f64 %1, %1, %3, %8\n"
+        "v_fma_f64 %0, %0, %2, %9\nv_fma_f64 %1, %1, %3, %9\n"
+        "v_fma_f64 %0, %0, %2, %10\nv_fma_f64 %1, %1, %3, %10\n"
+        "v_fma_f64 %0, %0, %2, %11\nv_fma_f64 %1, %1, %3, %11\n"
+        "v_fma_f64 %0, %0, %2, %12\nv_fma_f64 %1, %1, %3, %12\n"
+        "v_fma_f64 %0, %0, %2, %13\nv_fma_f64 %1, %1, %3, %13\n"
+        "v_fma_f64 %0, %0, %2, 1.0\nv_fma_f64 %1, %1, %3, 1.0\n"
+        "v_fma_f64 %0, %0, %2, 1.0\nv_fma_f64 %1, %1, %3, 1.0\n"
+        : "=&v"(q[0]), "=&v"(q[1])
+        : "v"(x[0]), "v"(x[1]),
+          "v"(kExpC[0]), "s"(kExpC[1]), "s"(kExpC[2]), "s"(kExpC[3]), "s"(kExpC[4]), "s"(kExpC[5]), "s"(kExpC[6]), "s"(kExpC[7]), "s"(kExpC[8]), "s"(kExpC[9]));
+#pragma unroll
+    for (int j = 0; j < 2; j++) x[j] = ldexp(q[j], static_cast<int>(n[j]));
+}
+template <>
+__device__ __forceinline__ void fast_exp_n<4>(double (&x)[4]) {
+    double n[4], q[4];
+    asm(
+        "v_mul_f64 %4, %0, %8\nv_mul_f64 %5, %1, %8\n"
+        "v_mul_f64 %6, %2, %8\nv_mul_f64 %7, %3, %8\n"
+        "v_rndne_f64 %4, %4\nv_rndne_f64 %5, %5\n"
+        "v_rndne_f64 %6, %6\nv_rndne_f64 %7, %7\n"
+        "v_fma_f64 %0, %4, %9, %0\nv_fma_f64 %1, %5, %9, %1\n"
+        "v_fma_f64 %2, %6, %9, %2\nv_fma_f64 %3, %7, %9, %3\n"
+        "v_fma_f64 %0, %4, %10, %0\nv_fma_f64 %1, %5, %10, %1\n"
+        "v_fma_f64 %2, %6, %10, %2\nv_fma_f64 %3, %7, %10, %3\n"
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]),
+          "=&v"(n[0]), "=&v"(n[1]), "=&v"(n[2]), "=&v"(n[3])
+        : "s"(kLog2e), "s"(-kLn2Hi), "s"(-kLn2Lo));
+    asm(
+        "v_fma_f64 %0, %4, %8, %9\nv_fma_f64 %1, %5, %8, %9\n"
+        "v_fma_f64 %2, %6, %8, %9\nv_fma_f64 %3, %7, %8, %9\n"
+        "v_fma_f64 %0, %0, %4, %10\nv_fma_f64 %1, %1, %5, %10\n"
+        "v_fma_f64 %2, %2, %6, %10\nv_fma_f64 %3, %3, %7, %10\n"
+        "v_fma_f64 %0, %0, %4, %11\nv_fma_f64 %1, %1, %5, %11\n"
+        "v_fma_f64 %2, %2, %6, %11\nv_fma_f64 %3, %3, %7, %11\n"
+        "v_fma_f64 %0, %0, %4, %12\nv_fma_f64 %1, %1, %5, %12\n"
+        "v_fma_f64 %2, %2, %6, %12\nv_fma_f64 %3, %3, %7, %12\n"
+        "v_fma_f64 %0, %0, %4, %13\nv_fma_f64 %1, %1, %5, %13\n"
+        "v_fma_f64 %2, %2, %6, %13\nv_fma_f64 %3, %3, %7, %13\n"
+        "v_fma_f64 %0, %0, %4, %14\nv_fma_f64 %1, %1, %5, %14\n"
+        "v_fma_f64 %2, %2, %6, %14\nv_fma_f64 %3, %3, %7, %14\n"
+        "v_fma_f64 %0, %0, %4, %15\nv_fma_f64 %1, %1, %5, %15\n"
+        "v_fma_f64 %2, %2, %6, %15\nv_fma_f64 %3, %3, %7, %15\n"
+        "v_fma_f64 %0, %0, %4, %16\nv_fma_f64 %1, %1, %5, %16\n"
+        "v_fma_f64 %2, %2, %6, %16\nv_fma_f64 %3, %3, %7, %16\n"
+        "v_fma_f64 %0, %0, %4, %17\nv_fma_f64 %1, %1, %5, %17\n"
+        "v_fma_f64 %2, %2, %6, %17\nv_fma_f64 %3, %3, %7, %17\n"
+        "v_fma_f64 %0, %0, %4, 1.0\nv_fma_f64 %1, %1, %5, 1.0\n"
+        "v_fma_f64 %2, %2, %6, 1.0\nv_fma_f64 %3, %3, %7, 1.0\n"
+        "v_fma_f64 %0, %0, %4, 1.0\nv_fma_f64 %1, %1, %5, 1.0\n"
+        "v_fma_f64 %2, %2, %6, 1.0\nv_fma_f64 %3, %3, %7, 1.0\n"
+        : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3])
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]),
+          "v"(kExpC[0]), "s"(kExpC[1]), "s"(kExpC[2]), "s"(kExpC[3]), "s"(kExpC[4]), "s"(kExpC[5]), "s"(kExpC[6]), "s"(kExpC[7]), "s"(kExpC[8]), "s"(kExpC[9]));
+#pragma unroll
+    for (int j = 0; j < 4; j++) x[j] = ldexp(q[j], static_cast<int>(n[j]));
+}
+template <>
+__device__ __forceinline__ void fast_exp_n<6>(double (&x)[6]) {
+    double n[6], q[6];
+    asm(
+        "v_mul_f64 %6, %0, %12\nv_mul_f64 %7, %1, %12\n"
+        "v_mul_f64 %8, %2, %12\nv_mul_f64 %9, %3, %12\n"
+        "v_mul_f64 %10, %4, %12\nv_mul_f64 %11, %5, %12\n"
+        "v_rndne_f64 %6, %6\nv_rndne_f64 %7, %7\n"
+        "v_rndne_f64 %8, %8\nv_rndne_f64 %9, %9\n"
+        "v_rndne_f64 %10, %10\nv_rndne_f64 %11, %11\n"
+        "v_fma_f64 %0, %6, %13, %0\nv_fma_f64 %1, %7, %13, %1\n"
+        "v_fma_f64 %2, %8, %13, %2\nv_fma_f64 %3, %9, %13, %3\n"
+        "v_fma_f64 %4, %10, %13, %4\nv_fma_f64 %5, %11, %13, %5\n"
+        "v_fma_f64 %0, %6, %14, %0\nv_fma_f64 %1, %7, %14, %1\n"
+        "v_fma_f64 %2, %8, %14, %2\nv_fma_f64 %3, %9, %14, %3\n"
+        "v_fma_f64 %4, %10, %14, %4\nv_fma_f64 %5, %11, %14, %5\n"
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]),
+          "=&v"(n[0]), "=&v"(n[1]), "=&v"(n[2]), "=&v"(n[3]), "=&v"(n[4]), "=&v"(n[5])
+        : "s"(kLog2e), "s"(-kLn2Hi), "s"(-kLn2Lo));
+    asm(
+        "v_fma_f64 %0, %6, %12, %13\nv_fma_f64 %1, %7, %12, %13\n"
+        "v_fma_f64 %2, %8, %12, %13\nv_fma_f64 %3, %9, %12, %13\n"
+        "v_fma_f64 %4, %10, %12, %13\nv_fma_f64 %5, %11, %12, %13\n"
+        "v_fma_f64 %0, %0, %6, %14\nv_fma_f64 %1, %1, %7, %14\n"
+        "v_fma_f64 %2, %2, %8, %14\nv_fma_f64 %3, %3, %9, %14\n"
+        "v_fma_f64 %4, %4, %10, %14\nv_fma_f64 %5, %5, %11, %14\n"
+        "v_fma_f64 %0, %0, %6, %15\nv_fma_f64 %1, %1, %7, %15\n"
+        "v_fma_f64 %2, %2, %8, %15\nv_fma_f64 %3, %3, %9, %15\n"
+        "v_fma_f64 %4, %4, %10, %15\nv_fma_f64 %5, %5, %11, %15\n"
+        "v_fma_f64 %0, %0, %6, %16\nv_fma_f64 %1, %1, %7, %16\n"
+        "v_fma_f64 %2, %2, %8, %16\nv_fma_f64 %3, %3, %9, %16\n"
+        "v_fma_f64 %4, %4, %10, %16\nv_fma_f64 %5, %5, %11, %16\n"
+        "v_fma_f64 %0, %0, %6, %17\nv_fma_f64 %1, %1, %7, %17\n"
+        "v_fma_f64 %2, %2, %8, %17\nv_fma_f64 %3, %3, %9, %17\n"
+        "v_fma_f64 %4, %4, %10, %17\nv_fma_f64 %5, %5, %11, %17\n"
+        "v_fma_f64 %0, %0, %6, %18\nv_fma_f64 %1, %1, %7, %18\n"
+        "v_fma_f64 %2, %2, %8, %18\nv_fma_f64 %3, %3, %9, %18\n"
+        "v_fma_f64 %4, %4, %10, %18\nv_fma_f64 %5, %5, %11, %18\n"
+        "v_fma_f64 %0, %0, %6, %19\nv_fma_f64 %1, %1, %7, %19\n"
+        "v_fma_f64 %2, %2, %8, %19\nv_fma_f64 %3, %3, %9, %19\n"
+        "v_fma_f64 %4, %4, %10, %19\nv_fma_f64 %5, %5, %11, %19\n"
+        "v_fma_f64 %0, %0, %6, %20\nv_fma_f64 %1, %1, %7, %20\n"
+        "v_fma_f64 %2, %2, %8, %20\nv_fma_f64 %3, %3, %9, %20\n"
+        "v_fma_f64 %4, %4, %10, %20\nv_fma_f64 %5, %5, %11, %20\n"
+        "v_fma_f64 %0, %0, %6, %21\nv_fma_f64 %1, %1, %7, %21\n"
+        "v_fma_f64 %2, %2, %8, %21\nv_fma_f64 %3, %3, %9, %21\n"
+        "v_fma_f64 %4, %4, %10, %21\nv_fma_f64 %5, %5, %11, %21\n"
+        "v_fma_f64 %0, %0, %6, 1.0\nv_fma_f64 %1, %1, %7, 1.0\n"
+        "v_fma_f64 %2, %2, %8, 1.0\nv_fma_f64 %3, %3, %9, 1.0\n"
+        "v_fma_f64 %4, %4, %10, 1.0\nv_fma_f64 %5, %5, %11, 1.0\n"
+        "v_fma_f64 %0, %0, %6, 1.0\nv_fma_f64 %1, %1, %7, 1.0\n"
+        "v_fma_f64 %2, %2, %8, 1.0\nv_fma_f64 %3, %3, %9, 1.0\n"
+        "v_fma_f64 %4, %4, %10, 1.0\nv_fma_f64 %5, %5, %11, 1.0\n"
+        : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3]), "=&v"(q[4]), "=&v"(q[5])
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]),
+          "v"(kExpC[0]), "s"(kExpC[1]), "s"(kExpC[2]), "s"(kExpC[3]), "s"(kExpC[4]), "s"(kExpC[5]), "s"(kExpC[6]), "s"(kExpC[7]), "s"(kExpC[8]), "s"(kExpC[9]));
+#pragma unroll
+    for (int j = 0; j < 6; j++) x[j] = ldexp(q[j], static_cast<int>(n[j]));
+}
+// 10^x, |x| moderate: x ln 10 in two parts
+__device__ __forceinline__ double fast_exp10(double x) {
+    const double h = x * 2.302585092994046;
+    const double l = fma(x, 2.302585092994046, -h) + x * -2.1707562233822494e-16;
+    const double e = fast_exp(h);
+    return fma(e, l, e);
+}
+
 // Transcendentals of the rate constants.  kF32: evaluated in FP32 (hardware
 // exp2/log2 based) on FP64 arguments rounded to FP32, widened back to FP64;
 // arguments whose result would leave the FP32 range take the FP64 function.
@@ -275,8 +485,10 @@ template <bool kF32>
 __device__ __forceinline__ double rate_exp(double arg) {
     if constexpr (kF32) {
         if (fabs(arg) < 80.0) return static_cast<double>(expf(static_cast<float>(arg)));
+        return exp(arg);
+    } else {
+        return fast_exp(arg);
     }
-    return exp(arg);
 }
 template <bool kF32>
 __device__ __forceinline__ double rate_log10(double x) {
@@ -289,8 +501,10 @@ template <bool kF32>
 __device__ __forceinline__ double rate_exp10(double x) {
     if constexpr (kF32) {
         if (fabs(x) < 35.0) return static_cast<double>(exp10f(static_cast<float>(x)));
+        return exp10(x);
+    } else {
+        return fast_exp10(x);
     }
-    return exp10(x);
 }
 
 // PLOG rate constant (PlogRate::updateFromStruct / evalFromStruct,
@@ -379,6 +593,29 @@ __device__ __noinline__ double sri_falloff(const double* __restrict__ fo, double
     return pow(w, 1.0 / (1.0 + lpr * lpr)) * (fo[6] * pow(T, fo[7]));
 }
 
+// sum_k (e_k - d) C_k over the explicit efficiencies of a reaction, in list
+// order without fused multiply-adds.  Lists are padded to whole groups of
+// kTbPad entries with efficiency 0, so a group's table loads, then its
+// concentration loads, are all in flight together with no test against the
+// list length.
+__device__ __forceinline__ double efficiency_sum(const DevMech& m, SpeciesColumn C, int tbo, int tbn) {
+    double sum = 0.0;
+    for (int j0 = 0; j0 == 0 || j0 < tbn; j0 += kTbPad) {
+        int kk[kTbPad];
+        double ee[kTbPad], cc[kTbPad];
+#pragma unroll
+        for (int b = 0; b < kTbPad; b++) {
+            kk[b] = m.tbk[tbo + j0 + b];
+            ee[b] = m.tbe[tbo + j0 + b];
+        }
+#pragma unroll
+        for (int b = 0; b < kTbPad; b++) cc[b] = opaque(C[kk[b]]);
+#pragma unroll
+        for (int b = 0; b < kTbPad; b++) sum = add_mul_rn(sum, ee[b], cc[b]);
+    }
+    return sum;
+}
+
 // Evaluate reaction p (permuted index) at the gas state; C and MU live in LDS.
 // kpd: this lane's pdep_rate_lane value (used for flags bit 6/7 only).
 // kF32: rate constants (Arrhenius, falloff centre and blending) through the
@@ -387,49 +624,14 @@ __device__ __noinline__ double sri_falloff(const double* __restrict__ fo, double
 // applied to the forward rate of progress before the reverse one is formed.
 template <bool kF32 = false>
 __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const GasState& g,
-                                              const double* __restrict__ C, const double* __restrict__ MU,
+                                              SpeciesColumn C, SpeciesColumn MU,
                                               const RxnRegs& x, double kpd, RxnVals& o, double perturb = 1.0) {
     const double4 rd = reinterpret_cast<const double4*>(m.rd)[p];
     const int type = (x.flags >> 1) & 3;
     const bool rev = x.flags & 1;
     double M = 1.0;
     if (x.flags & 32) {
-        // The first kTbPad efficiencies are loaded with no test against the
-        // list length (the table ends with kTbPad padding entries), so their
-        // table loads, then their concentration loads, are all in flight
-        // together; entries past the reaction's own list are not added.  The
-        // rest follow in groups of 4.
-        double sum = 0.0;
-        {
-            int kk[kTbPad];
-            double ee[kTbPad], cc[kTbPad];
-#pragma unroll
-            for (int b = 0; b < kTbPad; b++) {
-                kk[b] = m.tbk[x.tbo + b];
-                ee[b] = m.tbe[x.tbo + b];
-            }
-#pragma unroll
-            for (int b = 0; b < kTbPad; b++) cc[b] = opaque(C[kk[b]]);
-#pragma unroll
-            for (int b = 0; b < kTbPad; b++)
-                if (b < x.tbn) sum = add_mul_rn(sum, ee[b], cc[b]);
-        }
-        for (int j0 = kTbPad; j0 < x.tbn; j0 += 4) {
-            int kk[4];
-            double ee[4];
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const bool ok = j0 + b < x.tbn;
-                kk[b] = ok ? m.tbk[x.tbo + j0 + b] : 0;
-                ee[b] = ok ? m.tbe[x.tbo + j0 + b] : 0.0;
-            }
-            double cc[4];
-#pragma unroll
-            for (int b = 0; b < 4; b++) cc[b] = C[kk[b]];
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-                if (j0 + b < x.tbn) sum = add_mul_rn(sum, ee[b], cc[b]);
-        }
+        const double sum = efficiency_sum(m, C, x.tbo, x.tbn);
         M = add_mul_rn(sum, m.tbdef[p], g.ctot);
     }
     double kf;
@@ -442,8 +644,11 @@ __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const Gas
         double work = 0.0;
         if (type == kTroe && !sri) {
             // Troe (fo[7] = 0) and Tsang (Fcent = A + B T)
-            double Fcent = (1.0 - fo[3]) * rate_exp<kF32>(-g.T * fo[4]) + fo[3] * rate_exp<kF32>(-g.T * fo[5]);
-            if (fo[6] != 0.0) Fcent += rate_exp<kF32>(-fo[6] / g.T);
+            // (1/T3 is infinite for Tsang, and mechanisms use 1e100 for T2: the
+            // exponents are kept moderate)
+            double Fcent = (1.0 - fo[3]) * rate_exp<kF32>(fmax(-g.T * fo[4], -1e4)) +
+                           fo[3] * rate_exp<kF32>(fmax(-g.T * fo[5], -1e4));
+            if (fo[6] != 0.0) Fcent += rate_exp<kF32>(fmin(fmax(-fo[6] / g.T, -1e4), 1e4));
             Fcent += fo[7] * g.T;
             work = rate_log10<kF32>(fmax(Fcent, kSmallNumber));
         }
@@ -494,7 +699,7 @@ __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const Gas
             if (x.nr > 2) dr += MU[x.rk[2]];
             delta -= dr;
         }
-        rkcn = fmin(exp(delta * g.rrt - rd.w * g.logC0), kBigNumber);
+        rkcn = fmin(fast_exp(delta - rd.w * g.logC0), kBigNumber);
     }
     o.rkcn = rkcn;
     double ropf = kf * perturb;
@@ -552,34 +757,177 @@ __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const Gas
     o.ropr = ropr;
 }
 
-// Net rate of progress of a plain mass-action reaction (RxnI flag bit 10:
-// elementary, kRep sides of at most three entries): the same quantities as
-// eval_reaction without its tests -- unused side entries point at the
-// sentinel species (C = 1, MU = 0), which leaves every sum, product and
-// negative-concentration rule of the C1/C2/C3 cases unchanged.  pf: rate
-// multiplier of the forward rate of progress.
-template <bool kF32 = false>
-__device__ __forceinline__ double plain_ropnet(const DevMech& m, int p, const GasState& g,
-                                              const double* __restrict__ C, const double* __restrict__ MU,
-                                              const RxnRegs& x, double pf = 1.0) {
-    const double4 rd = reinterpret_cast<const double4*>(m.rd)[p];
-    const double kf = rd.x * rate_exp<kF32>(rd.y * g.logT - rd.z * g.recipT);
-    const double dr = (MU[x.rk[0]] + MU[x.rk[1]]) + MU[x.rk[2]];
-    const double dp = (MU[x.pk[0]] + MU[x.pk[1]]) + MU[x.pk[2]];
-    const double delta = dp - dr;
-    const bool rev = x.flags & 1;
-    const double rkcn = rev ? fmin(exp(delta * g.rrt - rd.w * g.logC0), kBigNumber) : 0.0;
-    double ropf = kf * pf;
-    double ropr = ropf * rkcn;
-    {
-        const double a = C[x.rk[0]], b = C[x.rk[1]], d = C[x.rk[2]];
-        ropf = ((a < 0 && (b < 0 || d < 0)) || (b < 0 && d < 0)) ? 0.0 : ropf * (a * b * d);
+// ---- standard reactions (RxnS), straight-line ---------------------------------
+//
+// One wavefront evaluates one state, so nothing but independent work in the
+// same instruction stream hides the latency of the table loads, the LDS reads
+// and the exponential's chain of dependent FMAs.  These functions therefore
+// have no branches: unused entries read the sentinel slot, selects are made on
+// values that the compiler cannot trace back to their loads (it turns a select
+// on a computed product into a branch around it, and everything after waits
+// there), and B reactions per lane are evaluated side by side.
+
+// x of two reactants/products negative: the rate of progress is 0
+// (the C1/C2/C3 rules of StoichManager.h:147-366; the sentinel's 1 is never negative)
+__device__ __forceinline__ double zero_if_two_negative(double v, double a, double b, double d) {
+    const bool na = a < 0, nb = b < 0, nd = d < 0;
+    const bool two = (na & nb) | ((na | nb) & nd);
+    v = opaque(v);
+    return two ? 0.0 : v;
+}
+
+struct StdRxn {
+    uint4 q;
+    double4 rd;     // A, b, Ea/R, dn
+    __device__ __forceinline__ void load(const DevMech& m, int p) {
+        q = reinterpret_cast<const uint4*>(m.rs)[p];
+        rd = reinterpret_cast<const double4*>(m.rd)[p];
     }
-    {
-        const double a = C[x.pk[0]], b = C[x.pk[1]], d = C[x.pk[2]];
-        ropr = rev ? (((a < 0 && (b < 0 || d < 0)) || (b < 0 && d < 0)) ? 0.0 : ropr * (a * b * d)) : 0.0;
+    __device__ __forceinline__ unsigned slot(int e) const {   // entry e: r0 r1 r2 p0 p1 p2 p3
+        const unsigned w = e < 2 ? q.x : (e < 4 ? q.y : (e < 6 ? q.z : q.w));
+        return (e & 1) ? w >> 16 : w & 0xffffu;
     }
-    return ropf - ropr;
+    __device__ __forceinline__ bool reversible() const { return q.w & 0x10000u; }
+    __device__ __forceinline__ bool four_products() const { return q.w & 0x20000u; }
+};
+
+// (C, mu/RT) of an entry
+__device__ __forceinline__ double2 species_pair(unsigned slot) {
+    return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(lds_base()) + slot);
+}
+
+// exponent of 1/K_c from the pairs of the six entries
+__device__ __forceinline__ double std_kc_arg(const StdRxn& x, double logC0, const double2 (&v)[6]) {
+    const double dr = (v[0].y + v[1].y) + v[2].y;
+    const double dp = (v[3].y + v[4].y) + v[5].y;
+    return (dp - dr) - x.rd.w * logC0;
+}
+
+// net rate of progress from the forward constant kf (perturbed, times [M] for a
+// three-body reaction) and exp(std_kc_arg)
+__device__ __forceinline__ double std_ropnet(const StdRxn& x, double kf, double ekc, const double2 (&v)[6]) {
+    const double rkcn = fmin(ekc, kBigNumber);
+    const double f = zero_if_two_negative(kf * (v[0].x * v[1].x * v[2].x), v[0].x, v[1].x, v[2].x);
+    const double r =
+        zero_if_two_negative(kf * rkcn * (v[3].x * v[4].x * v[5].x), v[3].x, v[4].x, v[5].x);
+    return f - (x.reversible() ? r : 0.0);
+}
+
+// -r to the reactants' accumulators, +r to the products' (an accumulator is
+// half a pair)
+__device__ __forceinline__ double* accumulator(double* wd, unsigned slot) {
+    return reinterpret_cast<double*>(reinterpret_cast<char*>(wd) + (slot >> 1));
+}
+__device__ __forceinline__ void std_scatter(double* wd, const StdRxn& x, double r) {
+#pragma unroll
+    for (int e = 0; e < 3; e++) atomicAdd(accumulator(wd, x.slot(e)), -r);
+#pragma unroll
+    for (int e = 3; e < 6; e++) atomicAdd(accumulator(wd, x.slot(e)), r);
+}
+
+// B passes of elementary reactions, lane entries p, p + 64, ...
+template <int B, bool kF32, bool kPert>
+__device__ __forceinline__ void plain_block(const DevMech& m, double* wd, const GasState& g, int p, int pert_rxn, double pert_v) {
+    StdRxn x[B];
+#pragma unroll
+    for (int b = 0; b < B; b++) x[b].load(m, p + kWave * b);
+    double2 v[B][6];
+    double r[B], ex[2 * B];
+#pragma unroll
+    for (int b = 0; b < B; b++)
+#pragma unroll
+        for (int e = 0; e < 6; e++) v[b][e] = species_pair(x[b].slot(e));
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        ex[b] = x[b].rd.y * g.logT - x[b].rd.z * g.recipT;
+        ex[B + b] = std_kc_arg(x[b], g.logC0, v[b]);
+    }
+    if constexpr (kF32) {
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            ex[b] = rate_exp<true>(ex[b]);
+            ex[B + b] = fast_exp(ex[B + b]);
+        }
+    } else {
+        fast_exp_n(ex);
+    }
+    bool four = false;
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        double kf = x[b].rd.x * ex[b];
+        if constexpr (kPert) kf *= (p + kWave * b == pert_rxn) ? pert_v : 1.0;
+        r[b] = std_ropnet(x[b], kf, ex[B + b], v[b]);
+        four |= x[b].four_products();
+    }
+#pragma unroll
+    for (int b = 0; b < B; b++) std_scatter(wd, x[b], r[b]);
+    if (__any(four)) {
+#pragma unroll
+        for (int b = 0; b < B; b++) atomicAdd(accumulator(wd, x[b].slot(6)), r[b]);
+    }
+}
+
+// One pass that may hold three-body, Lindemann, Troe/Tsang and elementary
+// reactions: every lane runs the same code (the falloff part only if the pass
+// has such a reaction), the type selects among the results.  The formulas are
+// eval_reaction's.
+template <bool kF32, bool kPert>
+__device__ __forceinline__ void falloff_pass(const DevMech& m, const WaveScratch& S, const GasState& g, int p,
+                                             int pert_rxn, double pert_v) {
+    StdRxn x;
+    x.load(m, p);
+    const int4* qi = reinterpret_cast<const int4*>(m.ri + p);
+    const int4 ia = qi[0], ib = qi[1];
+    const double tbdef = m.tbdef[p];
+    const int type = (ia.x >> 1) & 3;
+    const double4* f4 = reinterpret_cast<const double4*>(m.fod + 8 * (ib.y < 0 ? m.n_fo : ib.y));
+    const double4 fa = f4[0], fb = f4[1];   // A0, b0, Ea0/R, a | 1/T3, 1/T1, T2, B
+    double2 v[6];
+#pragma unroll
+    for (int e = 0; e < 6; e++) v[e] = species_pair(x.slot(e));
+    const double M = add_mul_rn(efficiency_sum(m, S.C, ia.w, ib.x), tbdef, g.ctot);
+    // the pass's six exponentials side by side (Troe exponents kept moderate:
+    // 1/T3 is infinite for Tsang, some T2 are 1e100)
+    double ex[6];
+    ex[0] = x.rd.y * g.logT - x.rd.z * g.recipT;
+    ex[1] = std_kc_arg(x, g.logC0, v);
+    ex[2] = fa.y * g.logT - fa.z * g.recipT;
+    ex[3] = fmax(-g.T * fb.x, -1e4);
+    ex[4] = fmax(-g.T * fb.y, -1e4);
+    ex[5] = fmin(fmax(-fb.z * g.recipT, -1e4), 1e4);
+    const bool falloff = __any(type >= kLindemann);
+    if constexpr (kF32) {
+        ex[1] = fast_exp(ex[1]);
+        ex[0] = rate_exp<true>(ex[0]);
+        if (falloff)
+#pragma unroll
+            for (int j = 2; j < 6; j++) ex[j] = rate_exp<true>(ex[j]);
+    } else {
+        fast_exp_n(ex);
+    }
+    double kf = x.rd.x * ex[0];
+    if (falloff) {
+        const double k0 = fa.x * ex[2];
+        double Fcent = (1.0 - fa.w) * ex[3] + fa.w * ex[4];
+        Fcent += (fb.z != 0.0) ? opaque(ex[5]) : 0.0;
+        Fcent += fb.w * g.T;
+        const double work = rate_log10<kF32>(fmax(Fcent, kSmallNumber));
+        const double pr = M * k0 / (kf + kSmallNumber);
+        const double lpr = rate_log10<kF32>(fmax(pr, kSmallNumber));
+        const double cc = -0.4 - 0.67 * work;
+        const double nn = 0.75 - 1.27 * work;
+        const double f1 = (lpr + cc) / (nn - 0.14 * (lpr + cc));
+        const double Ft = opaque(rate_exp10<kF32>(work / (1.0 + f1 * f1)));
+        const double F = (type == kTroe) ? Ft : 1.0;
+        const double kfo = opaque((pr * (F / (1.0 + pr))) * kf);
+        kf = (type >= kLindemann) ? kfo : kf;
+    }
+    if constexpr (kPert) kf *= (p == pert_rxn) ? pert_v : 1.0;
+    const double kM = opaque(kf * M);
+    kf = (type == kThreeBody) ? kM : kf;
+    const double r = std_ropnet(x, kf, ex[1], v);
+    std_scatter(S.WD, x, r);
+    if (__any(x.four_products())) atomicAdd(accumulator(S.WD, x.slot(6)), r);
 }
 
 // Gas state + per-species thermo, concentrations and chemical potentials.
@@ -602,6 +950,9 @@ __device__ __forceinline__ void species_pass(const DevMech& m, const WaveScratch
         sr.ym[s] = (k < m.K) ? yk[s] * m.rmw[k] : 0.0;
         sum += sr.ym[s];
     }
+    g.T = T;
+    g.RT = T * kGasConstant;
+    g.recipT = 1.0 / T;
     if constexpr (kSeqSum) {
 #pragma unroll
         for (int s = 0; s < NS; s++) {
@@ -610,51 +961,87 @@ __device__ __forceinline__ void species_pass(const DevMech& m, const WaveScratch
         }
         wave_sync();
         sum = 0.0;
-        for (int k = 0; k < m.K; k++) sum += S.WD[k];
+        int k = 0;
+        for (; k + 8 <= m.K; k += 8) {   // the adds are a chain, the loads are not
+            double t[8];
+#pragma unroll
+            for (int b = 0; b < 8; b++) t[b] = S.WD[k + b];
+#pragma unroll
+            for (int b = 0; b < 8; b++) sum += t[b];
+        }
+        for (; k < m.K; k++) sum += S.WD[k];
         wave_sync();
     } else {
         sum = uni(wave_sum(sum));
     }
-    g.T = T;
+    // rounded as the reference does (ThermoPhase.cpp, IdealGasPhase.h): a
+    // nearly cancelling [M] amplifies the last bits of C_tot and C_k
     g.mmw = 1.0 / sum;
-    g.RT = T * kGasConstant;
     g.dens = (rho > 0.0) ? rho : P * g.mmw / g.RT;
     g.ctot = g.dens / g.mmw;
     g.pressure = kGasConstant * g.ctot * T;
     g.P = (rho > 0.0) ? g.pressure : P;
-    g.logT = log(T);
-    g.recipT = 1.0 / T;
-    g.rrt = 1.0 / g.RT;
-    g.logC0 = log(g.pressure / g.RT);
-    g.tmp = log(g.pressure / m.pref) * g.RT;
+    // ln T, ln(P/RT) and ln(P/Pref) in one evaluation, a lane each
+    const double lg = log(lane == 0 ? T : (lane == 1 ? g.ctot : g.pressure * m.rpref));
+    g.logT = readlane_f64(lg, 0);
+    g.logC0 = readlane_f64(lg, 1);
+    const double lnp = readlane_f64(lg, 2);
     double tt[6];
     tt[0] = T;
     tt[1] = T * T;
     tt[2] = tt[1] * T;
     tt[3] = tt[2] * T;
-    tt[4] = 1.0 / T;
+    tt[4] = g.recipT;
     tt[5] = g.logT;
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         int k = lane + kWave * s;
+        sr.cpr[s] = 0.0;
+        sr.hrt[s] = 0.0;
         if (k < m.K) {
             double cp, h, sR, g0;
             nasa7(m.nasa + 16 * k, T, tt, cp, h, sR, g0);
             sr.cpr[s] = cp;
             sr.hrt[s] = h;
-            double mu = g0 * g.RT;
-            mu += g.tmp;
-            S.MU[k] = mu;
-            S.C[k] = sr.ym[s] * g.dens;
-        } else {
-            sr.cpr[s] = 0.0;
-            sr.hrt[s] = 0.0;
-            if (k == m.K) {
-                S.MU[k] = 0.0;
-                S.C[k] = 1.0;
-            }
+            *reinterpret_cast<double2*>(lds_base() + 2 * k) = double2{sr.ym[s] * g.dens, g0 + lnp};
         }
     }
+    // the sentinel slots of the compact records
+    *reinterpret_cast<double2*>(lds_base() + 2 * (m.K + lane)) = double2{1.0, 0.0};
+}
+
+// The passes of 64 reactions that hold non-standard reactions (PLOG,
+// Chebyshev, SRI, chemically activated, power-law orders): the general code,
+// out of line so that its registers and hoisted constants burden only the
+// mechanisms that have such reactions.
+template <bool kF32, bool kPert>
+__device__ __noinline__ void general_passes(KernargMech* mech, double T, double logT,
+                                            double recipT, double logC0, double ctot, double pressure, int pert_rxn,
+                                            double pert_v) {
+    const DevMech m = *(const DevMech*)mech;
+    WaveScratch S{};
+    bind_species(S, mech);
+    GasState g{};
+    g.T = T; g.logT = logT; g.recipT = recipT; g.logC0 = logC0; g.ctot = ctot; g.pressure = pressure;
+    const int lane = lane_id();
+    const double kpd = pdep_rate_lane(m, g);
+    for (int p = lane; p < min(kWave * m.gen_end, m.I); p += kWave) {
+        RxnRegs x;
+        load_rxn(m, p, x);
+        RxnVals v;
+        if constexpr (kPert) eval_reaction<kF32>(m, p, g, S.C, S.MU, x, kpd, v, p == pert_rxn ? pert_v : 1.0);
+        else eval_reaction<kF32>(m, p, g, S.C, S.MU, x, kpd, v);
+        const double r = v.ropf - v.ropr;
+        const double* gs = (x.gen >= 0) ? m.gend + 12 * x.gen : m.gend;
+        const bool rgen = x.flags & 8, pgen = x.flags & 16;
+#pragma unroll
+        for (int j = 0; j < kMaxSide; j++)
+            if (j < x.nr) atomicAdd(&S.WD[x.rk[j]], -(rgen ? gs[4 + j] : 1.0) * r);
+#pragma unroll
+        for (int j = 0; j < kMaxSide; j++)
+            if (j < x.np) atomicAdd(&S.WD[x.pk[j]], (pgen ? gs[8 + j] : 1.0) * r);
+    }
+    wave_sync();
 }
 
 // Net production rates for the species each lane owns (after species_pass).
@@ -663,7 +1050,8 @@ __device__ __forceinline__ void species_pass(const DevMech& m, const WaveScratch
 // so no second pass over a gather table is needed; the summation order of a
 // species' terms is the hardware's, not the reference's reaction order.
 // kPert: reaction pert_rxn (permuted index) runs with rate multiplier pert_v.
-template <int NS, bool kF32 = false, bool kPert = false>
+// kBlock: elementary passes evaluated side by side.
+template <int NS, bool kF32 = false, bool kPert = false, int kBlock = 3>
 __device__ __forceinline__ void production_rates(const DevMech& m, const WaveScratch& S, const GasState& g,
                                                  SpeciesRegs<NS>& sr, int pert_rxn = -1, double pert_v = 1.0) {
     const int lane = lane_id();
@@ -673,57 +1061,21 @@ __device__ __forceinline__ void production_rates(const DevMech& m, const WaveScr
         if (k < m.K) S.WD[k] = 0.0;
     }
     wave_sync();
-    const double kpd = pdep_rate_lane(m, g);
-    // Lane j takes reactions j, j + 64, ...  When the reactions of this pass
-    // and of the next one are all plain mass action (the elementary reactions
-    // come last in the permuted order), the lane evaluates both in one
-    // branch-free block -- two independent chains of loads and exponentials
-    // for the scheduler to interleave -- and the loop advances two passes.
-    for (int p = lane; p < m.I;) {
-        RxnRegs x, x1;
-        load_rxn(m, p, x);
-        const bool two = p + kWave < m.I;
-        const int p1 = two ? p + kWave : p;
-        load_rxn(m, p1, x1);
-        if (__all((x.flags & 1024) && (x1.flags & 1024))) {
-            double pf0 = 1.0, pf1 = 1.0;
-            if constexpr (kPert) {
-                pf0 = (p == pert_rxn) ? pert_v : 1.0;
-                pf1 = (p1 == pert_rxn) ? pert_v : 1.0;
-            }
-            const double r0 = plain_ropnet<kF32>(m, p, g, S.C, S.MU, x, pf0);
-            const double r1 = plain_ropnet<kF32>(m, p1, g, S.C, S.MU, x1, pf1);
-#pragma unroll
-            for (int j = 0; j < 3; j++)
-                if (j < x.nr) atomicAdd(&S.WD[x.rk[j]], -r0);
-#pragma unroll
-            for (int j = 0; j < 3; j++)
-                if (j < x.np) atomicAdd(&S.WD[x.pk[j]], r0);
-            if (two) {
-#pragma unroll
-                for (int j = 0; j < 3; j++)
-                    if (j < x1.nr) atomicAdd(&S.WD[x1.rk[j]], -r1);
-#pragma unroll
-                for (int j = 0; j < 3; j++)
-                    if (j < x1.np) atomicAdd(&S.WD[x1.pk[j]], r1);
-            }
-            p += 2 * kWave;
-        } else {
-            RxnVals v;
-            if constexpr (kPert) eval_reaction<kF32>(m, p, g, S.C, S.MU, x, kpd, v, p == pert_rxn ? pert_v : 1.0);
-            else eval_reaction<kF32>(m, p, g, S.C, S.MU, x, kpd, v);
-            const double r = v.ropf - v.ropr;
-            const double* gs = (x.gen >= 0) ? m.gend + 12 * x.gen : m.gend;
-            const bool rgen = x.flags & 8, pgen = x.flags & 16;
-#pragma unroll
-            for (int j = 0; j < kMaxSide; j++)
-                if (j < x.nr) atomicAdd(&S.WD[x.rk[j]], -(rgen ? gs[4 + j] : 1.0) * r);
-#pragma unroll
-            for (int j = 0; j < kMaxSide; j++)
-                if (j < x.np) atomicAdd(&S.WD[x.pk[j]], (pgen ? gs[8 + j] : 1.0) * r);
-            p += kWave;
+    if (m.gen_end > 0)
+        general_passes<kF32, kPert>(S.mech, g.T, g.logT, g.recipT, g.logC0, g.ctot,
+                                    g.pressure, pert_rxn, pert_v);
+    for (int q = m.gen_end; q < m.tb_end; q++) falloff_pass<kF32, kPert>(m, S, g, kWave * q + lane, pert_rxn, pert_v);
+    int q = m.tb_end;
+    const int nq = (m.I + kWave - 1) / kWave;
+    for (; q + kBlock <= nq; q += kBlock)
+        plain_block<kBlock, kF32, kPert>(m, S.WD, g, kWave * q + lane, pert_rxn, pert_v);
+    if constexpr (kBlock > 2)
+        if (q + 2 <= nq) {
+            plain_block<2, kF32, kPert>(m, S.WD, g, kWave * q + lane, pert_rxn, pert_v);
+            q += 2;
         }
-    }
+    if constexpr (kBlock > 1)
+        if (q < nq) plain_block<1, kF32, kPert>(m, S.WD, g, kWave * q + lane, pert_rxn, pert_v);
     wave_sync();
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -789,24 +1141,13 @@ __device__ __forceinline__ void reactor_rhs(const DevMech& m, const WaveScratch&
     }
 }
 
-// The mechanism of a kernel whose first parameter is a DevMech, or a struct
-// that begins with one, addressed in the kernel-argument segment.  Out-of-line
-// functions take this pointer rather than a reference to the kernel's copy of
-// the argument: a reference would make the kernel keep that copy in scratch
-// memory and read every field through it, while the kernel-argument segment is
-// read with scalar loads.
-using KernargMech = const __attribute__((address_space(4))) DevMech;
-__device__ __forceinline__ KernargMech* kernarg_mech() {
-    return (KernargMech*)__builtin_amdgcn_kernarg_segment_ptr();
-}
-
 // Out-of-line reactor RHS: state taken from S.yb (written by the caller),
 // ydot written to S.F.  One copy of the kinetics code serves every call site of
 // the integrator (smaller code, and the caller keeps little live across it).
 template <int NS>
 __device__ __noinline__ void rhs_call(KernargMech* mech, ScratchLayout L, double P) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     double y[NS], f[NS];
 #pragma unroll
@@ -831,7 +1172,7 @@ __device__ __noinline__ void rhs_call(KernargMech* mech, ScratchLayout L, double
 template <int NS>
 __device__ __noinline__ void rhs_pert_call(KernargMech* mech, ScratchLayout L, double P, int pert_rxn, double pert_v) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     double y[NS], f[NS];
 #pragma unroll
@@ -859,7 +1200,7 @@ __device__ __noinline__ void rhs_pert_call(KernargMech* mech, ScratchLayout L, d
 template <int NS>
 __device__ __noinline__ void loss_frequency_call(KernargMech* mech, ScratchLayout L, double P) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     double y[NS];
 #pragma unroll

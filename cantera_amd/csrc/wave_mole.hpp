@@ -74,7 +74,7 @@ __device__ __forceinline__ void mole_rhs(const DevMech& m, const WaveScratch& S,
 template <int NS>
 __device__ __noinline__ void mole_rhs_call(KernargMech* mech, ScratchLayout L, double P) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     const int N = m.K + 1 + (m.const_volume ? 1 : 0);
     double y[NS], f[NS];
@@ -111,7 +111,7 @@ template <int NS>
 __device__ __noinline__ void mole_jac_call(KernargMech* mech, ScratchLayout L, double P, double* __restrict__ Jd,
                                            double* __restrict__ Js, const SparseTables* sp) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L);
+    const WaveScratch S = scratch_view(L, mech);
     const int lane = lane_id();
     const int K = m.K, N = K + 1 + (m.const_volume ? 1 : 0);
     const double hshift = m.const_volume ? 1.0 : 0.0;

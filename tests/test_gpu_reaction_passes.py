@@ -1,0 +1,69 @@
+"""Rates at the edges of the wavefront passes of 64 reactions: mechanisms cut to
+reaction counts around whole passes and blocks of passes, reactions with four
+products, and non-standard reactions mixed with standard ones."""
+import numpy as np
+import pytest
+
+from conftest import mech_file
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12     # of each state's largest rate, as the other rate tests
+
+
+def cut(src, dst, keep):
+    """The mechanism with the reactions `keep` (indices, in that order)."""
+    head, rxn, n = [], [], -1
+    for line in open(src):
+        t = line.split()
+        if not t or t[0] in ("end", "reactions"):
+            continue
+        if t[0] == "R":
+            n += 1
+            rxn.append([])
+        (rxn[n] if n >= 0 else head).append(line)
+    with open(dst, "w") as f:
+        f.writelines(head)
+        f.write("reactions %d\n" % len(keep))
+        for i, k in enumerate(keep):
+            t = rxn[k][0].split()
+            f.write(" ".join([t[0], str(i)] + t[2:]) + "\n")
+            f.writelines(rxn[k][1:])
+        f.write("end\n")
+    return str(dst)
+
+
+def check(path, oracle_mod, n=5, seed=3):
+    import cantera_amd as ca
+    om, sol = oracle_mod.Mech(path), ca.Solution(path)
+    g = np.random.default_rng(seed)
+    T = g.uniform(400.0, 2500.0, n)
+    P = 101325.0 * 10.0 ** g.uniform(-1, 1.5, n)
+    Y = g.dirichlet(0.3 * np.ones(sol.n_species), n)
+    Y[0, ::5] *= -1e-6
+    w = sol.net_production_rates(T, P, Y.T)
+    for s in range(n):
+        r = om.rates(T[s], P[s], Y[s])
+        scale = max(np.abs(r["wdot"]).max(), np.abs(r["ropf"]).max(), np.abs(r["ropr"]).max(), 1e-300)
+        assert np.abs(w[:, s] - r["wdot"]).max() <= TOL * scale
+    return sol, T, P, Y
+
+
+@pytest.mark.parametrize("mech,keep", [
+    *[("gri30", range(325 - r, 325)) for r in (1, 63, 64, 65, 128, 129, 192, 193, 256, 257, 320)],
+    ("gri30", range(64)),
+    ("nDodecane", [13, 15]),                                   # four products only
+    ("nDodecane", list(range(10)) + [13] + list(range(70)) + [15]),
+])
+def test_cut_mechanisms(mech, keep, tmp_path, oracle_mod):
+    check(cut(mech_file(mech), tmp_path / "m.mech", list(keep)), oracle_mod)
+
+
+def test_nan_is_not_hidden(oracle_mod):
+    sol, T, P, Y = check(mech_file("gri30"), oracle_mod)
+    Y[2, 10] = np.nan
+    T[3] = np.nan
+    w = sol.net_production_rates(T, P, Y.T)
+    reacting = np.abs(sol.net_production_rates(T[:1], P[:1], Y[0])[:, 0]) > 0
+    assert np.isnan(w[reacting][:, 2:4]).all()
+    assert np.isfinite(w[:, [0, 1, 4]]).all()
