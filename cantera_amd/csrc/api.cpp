@@ -332,13 +332,12 @@ int32_t cg_rates_batch_device(int32_t h, int64_t n, const double* T, const doubl
         if (n <= 0) return 0;
         if (!T || !P || !Y || !wdot) throw std::runtime_error("null array");
         const DevMech& m = mo.dm->view();
-        const size_t lds = rates_lds_bytes(m, mo.ns);
-        const void* kp = rates_kernel_ptr(mo.ns, f32);
-        set_lds_limit(kp, lds);
-        const int grid = grid_for(kp, lds, 0, n);
+        const RatesPlan plan = rates_plan(m, mo.ns, f32, n);
+        set_lds_limit(plan.kernel, plan.lds);
+        const int grid = grid_for(plan.kernel, plan.lds, 0, plan.items);
         hipStream_t s = static_cast<hipStream_t>(stream);
         check(hipEventRecord(mo.e0, s), "hipEventRecord");
-        check(rates_launch(m, mo.ns, f32, n, T, P, Y, wdot, grid, lds, s), "rates kernel launch");
+        check(rates_launch(plan, m, n, T, P, Y, wdot, grid, s), "rates kernel launch");
         check(hipEventRecord(mo.e1, s), "hipEventRecord");
         return 0;
     });
@@ -1374,7 +1373,7 @@ int32_t cg_reactors_net_production_rates_device(int32_t bh, double* wdot_dev) {
         if (!wdot_dev) throw std::runtime_error("null rates array");
         if (b.mole) throw std::runtime_error("rates at the states of a mole-based batch are not available");
         const DevMech& m = b.mech->dm->view();
-        const size_t lds = rates_lds_bytes(m, b.ns);
+        const size_t lds = reactor_rates_lds_bytes(m);
         const void* kp = reactor_rates_kernel_ptr(b.ns);
         set_lds_limit(kp, lds);
         const int grid = grid_for(kp, lds, 0, b.n);

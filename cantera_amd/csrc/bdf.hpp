@@ -84,16 +84,22 @@ size_t bdf_mole_lds_bytes(const DevMech& m, int nnz);
 hipError_t bdf_mole_launch(const BdfArgs& a, int grid, size_t lds, hipStream_t stream);
 const void* bdf_mole_kernel_ptr(int N);
 
-// batched rate evaluation (species-major SoA in and out)
-size_t rates_lds_bytes(const DevMech& m, int ns);
-// f32: rate constants through FP32 transcendentals (CG_FP32)
-hipError_t rates_launch(const DevMech& m, int ns, bool f32, long n, const double* T, const double* P,
-                        const double* Y, double* wdot, int grid, size_t lds, hipStream_t stream);
-const void* rates_kernel_ptr(int ns, bool f32);
+// Batched rate evaluation (species-major SoA in and out): kernel and launch
+// shape for n states.  f32: rate constants through FP32 transcendentals.
+struct RatesPlan {
+    int wide;             // states per wavefront, 0: one at a time
+    const void* kernel;
+    size_t lds;
+    long items;           // work items that the grid strides over
+};
+RatesPlan rates_plan(const DevMech& m, int ns, bool f32, long n);
+hipError_t rates_launch(const RatesPlan& p, DevMech m, long n, const double* T, const double* P, const double* Y,
+                        double* wdot, int grid, hipStream_t stream);
 // rates at the output states of a reactor batch (records as the integrator's)
 hipError_t reactor_rates_launch(const DevMech& m, int ns, long n, const double* rec, size_t stride, int cv,
                                 double* wdot, int grid, size_t lds, hipStream_t stream);
 const void* reactor_rates_kernel_ptr(int ns);
+size_t reactor_rates_lds_bytes(const DevMech& m);
 
 // longest-first processing order for the integrator's work queue (kernels
 // only, so it can be captured in a HIP graph); prev_nst, bucket, rank and

@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
+#include <map>
 #include <numeric>
 #include <sstream>
 #include <stdexcept>
@@ -391,6 +392,16 @@ DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
     d_.tbdef = upload(tbdef);
     d_.ri = upload(ri);
     d_.rs = upload(rs);
+    for (int p = 0; p < Ip; p++) {
+        const auto wide = [&](unsigned short& e) {
+            if (e >= 16 * K) e = static_cast<unsigned short>(16 * (K + p % kDummyWide));
+        };
+        for (unsigned short& e : rs[p].r) wide(e);
+        for (unsigned short& e : rs[p].p) wide(e);
+    }
+    d_.rsw = upload(rs);
+    d_.n_gen = n_gen;
+    d_.n_nonplain = std::max(n_gen, n_nonplain);
     d_.fod = upload(fod);
     d_.gend = upload(gend);
     d_.pdd = upload(pdd);

@@ -72,6 +72,8 @@ struct RxnI {
 };
 static_assert(sizeof(RxnI) == 48, "RxnI layout");
 
+constexpr int kDummyWide = 8;  // sentinel slots where several states share a wavefront's scratch
+
 // Compact record of a standard reaction: both sides unit-stoichiometry lists of
 // at most three molecules (four products if irreversible), a rate constant of
 // Arrhenius, three-body, Lindemann or Troe form.  Each entry is the byte offset
@@ -104,6 +106,9 @@ struct DevMech {
     const double* tbdef;
     const RxnI* ri;
     const RxnS* rs;          // valid for standard and null reactions
+    const RxnS* rsw;         // the same with sentinel slots K + (reaction % kDummyWide), for scratch with
+                             // several states per wavefront
+    int n_gen, n_nonplain;   // non-standard reactions; reactions up to the last that is not elementary
     const double* fod;       // (n_fo + 1) x 8, the last all zero: A0, b0, EaR0, then Troe a, 1/T3, 1/T1, T2, B (Tsang: a = A, 1/T3 = inf,
                              // 1/T1 = 0, T2 = 0, B) or SRI a, b, c, d, e
     const double* gend;      // n_gen x 12: reactant order[4], reactant stoich[4], product stoich[4]

@@ -16,10 +16,19 @@
 
 namespace cg {
 
+// From this many states on, several states per wavefront.  Below, the tiles
+// leave SIMDs empty and one state per wavefront ends sooner (us, one state /
+// tiles: gri30 2,048 states 25 / 33, 4,096 35 / 35, 8,192 51 / 36; n-dodecane
+// 2,048 29 / 29, 4,096 42 / 32; h2o2 1,024 15 / 15, 4,096 21 / 15).
+constexpr long kRatesWideMin = 4096;
+// LDS of a wavefront with 8 states: 8 wavefronts share a CU (two per SIMD, as
+// their registers allow); larger mechanisms take 4 states
+constexpr size_t kRatesWideLds = 160 * 1024 / 8;
+
 namespace {
 
-// At most 168 VGPRs, so that three wavefronts share a SIMD: two elementary
-// passes side by side fit without spills (three spill).
+// At most 168 VGPRs, so that three wavefronts share a SIMD (latency-bound
+// kernel; without the bound the allocator settles at 169 for NS = 1).
 template <int NS, bool kF32>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void rates_kernel(
     DevMech m, long n, const double* __restrict__ T, const double* __restrict__ P, const double* __restrict__ Y,
@@ -46,6 +55,116 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void ra
             const int k = lane + kWave * s;
             if (k < m.K) wdot[static_cast<size_t>(k) * n + st] = sr.wdot[s];
         }
+        wave_sync();
+    }
+}
+
+// S states per wavefront, 64 / S lanes per state (lane = s + S j, j the lane's
+// reaction of a pass), for batches that fill the GPU.
+//
+// Evaluated one state per wavefront, 64 lanes add their rates of progress to
+// the same 53 accumulators (gri30) at once: radicals occur in a third of the
+// reactions, and LDS adds to one address take turns.  The kernel above is bound
+// by that (2.6k cycles of a CU per gri30 state), and its falloff code runs for
+// 64 lanes to serve 29.  With S = 8 only 8 lanes share an accumulator, 50
+// falloff and three-body reactions take 7 passes of 8 states instead of one of
+// each, and a tile reads and writes whole 64-byte lines.  1,048,576 gri30
+// states: 4.50 -> 2.40 ms (FP64 VALU at 60% of its issue rate: 855
+// instructions a state); S = 16 leaves room for 7 wavefronts per CU (3.02 ms),
+// S = 4 has more lanes per accumulator (2.83 ms).  30,011 n-dodecane states,
+// FP32 constants: 213 -> 138 us with S = 4, 141 us with S = 8.  1/W_bar and [M]
+// are summed in the reference's order, as in the kernel above.
+template <int S, bool kF32>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void rates_wide_kernel(
+    DevMech m, long n, const double* __restrict__ T, const double* __restrict__ P, const double* __restrict__ Y,
+    double* __restrict__ wdot) {
+    constexpr int G = 64 / S;
+    const int lane = lane_id(), s = lane % S, j = lane / S;
+    const int rows = m.K + kDummyWide;
+    LaneView<S> lv;
+    lv.pair0 = 16u * s;
+    lv.wd = lds_base() + 2 * S * rows + s;
+    const SpeciesColumn<S> C{lds_base() + 2 * s}, MU{lds_base() + 2 * s + 1};
+    const long tiles = (n + S - 1) / S;
+    for (int k = m.K + j; k < rows; k += G) {   // sentinel rows
+        C[k] = 1.0;
+        MU[k] = 0.0;
+    }
+    const XcdStates xs(tiles);
+    for (long tile = xs.lo; tile < xs.hi; tile += xs.step) {
+        const long st = tile * S + s, sc = min(st, n - 1);   // a ragged tile's spare lanes repeat the last state
+        GasState g;
+        g.T = T[sc];
+        const double Ps = P[sc];
+        for (int k = j; k < m.K; k += G) {
+            C[k] = Y[static_cast<size_t>(k) * n + sc] * m.rmw[k];
+            lv.wd[S * k] = 0.0;
+        }
+        wave_sync();
+        double sum = 0.0;
+        {
+            int k = 0;
+            for (; k + 8 <= m.K; k += 8) {
+                double t[8];
+#pragma unroll
+                for (int b = 0; b < 8; b++) t[b] = C[k + b];
+#pragma unroll
+                for (int b = 0; b < 8; b++) sum += t[b];
+            }
+            for (; k < m.K; k++) sum += C[k];
+        }
+        wave_sync();
+        // as species_pass
+        g.RT = g.T * kGasConstant;
+        g.recipT = 1.0 / g.T;
+        g.mmw = 1.0 / sum;
+        g.dens = Ps * g.mmw / g.RT;
+        g.ctot = g.dens / g.mmw;
+        g.pressure = kGasConstant * g.ctot * g.T;
+        // ln T, ln(P/RT), ln(P/Pref): one each for the first three lanes of a state
+        const double lg = log(j == 0 ? g.T : (j == 1 ? g.ctot : g.pressure * m.rpref));
+        g.logT = __shfl(lg, s);
+        g.logC0 = __shfl(lg, s + S);
+        const double lnp = __shfl(lg, s + 2 * S);
+        double tt[6];
+        tt[0] = g.T;
+        tt[1] = g.T * g.T;
+        tt[2] = tt[1] * g.T;
+        tt[3] = tt[2] * g.T;
+        tt[4] = g.recipT;
+        tt[5] = g.logT;
+        for (int k = j; k < m.K; k += G) {
+            double cp, h, sR, g0;
+            nasa7(m.nasa + 16 * k, g.T, tt, cp, h, sR, g0);
+            C[k] = C[k] * g.dens;
+            MU[k] = g0 + lnp;
+        }
+        wave_sync();
+        int q = 0;
+        for (; q < m.n_gen; q += G) {   // non-standard reactions
+            const int p = q + j;
+            if (p >= m.I) continue;
+            RxnRegs x;
+            load_rxn(m, p, x);
+            double kpd = 0.0;
+            if (x.flags & 64) kpd = plog_rate(m.pdd + x.fo, log(g.pressure), g.logT, g.recipT);
+            else if (x.flags & 128) kpd = cheb_rate(m.pdd + x.fo, log10(g.pressure), g.recipT);
+            RxnVals v;
+            eval_reaction<kF32, S>(m, p, g, C, MU, x, kpd, v);
+            const double r = v.ropf - v.ropr;
+            const double* gs = (x.gen >= 0) ? m.gend + 12 * x.gen : m.gend;
+            const bool rgen = x.flags & 8, pgen = x.flags & 16;
+#pragma unroll
+            for (int e = 0; e < kMaxSide; e++)
+                if (e < x.nr) atomicAdd(&lv.wd[S * x.rk[e]], -(rgen ? gs[4 + e] : 1.0) * r);
+#pragma unroll
+            for (int e = 0; e < kMaxSide; e++)
+                if (e < x.np) atomicAdd(&lv.wd[S * x.pk[e]], (pgen ? gs[8 + e] : 1.0) * r);
+        }
+        standard_passes<3, kF32, false, S>(m, m.rsw, lv, C, g, j, q, m.n_nonplain, m.I, -1, 1.0);
+        wave_sync();
+        if (st < n)
+            for (int k = j; k < m.K; k += G) wdot[static_cast<size_t>(k) * n + st] = lv.wd[S * k];
         wave_sync();
     }
 }
@@ -105,35 +224,36 @@ const void* reactor_rates_kernel_ptr(int ns) {
                    : reinterpret_cast<const void*>(&reactor_rates_kernel<2>);
 }
 
-size_t rates_lds_bytes(const DevMech& m, int ns) {
-    return static_cast<size_t>(species_doubles(m.K)) * sizeof(double);
+size_t reactor_rates_lds_bytes(const DevMech& m) { return static_cast<size_t>(species_doubles(m.K)) * sizeof(double); }
+
+static size_t wide_lds(int K, int S) { return static_cast<size_t>(24) * S * (K + kDummyWide); }
+
+RatesPlan rates_plan(const DevMech& m, int ns, bool f32, long n) {
+    RatesPlan p{};
+    if (n >= kRatesWideMin) {
+        p.wide = wide_lds(m.K, 8) <= kRatesWideLds ? 8 : 4;
+    }
+    if (p.wide) {
+        p.lds = wide_lds(m.K, p.wide);
+        p.items = (n + p.wide - 1) / p.wide;
+    } else {
+        p.lds = reactor_rates_lds_bytes(m);
+        p.items = n;
+    }
+    switch (p.wide ? 10 * p.wide : rates_ns(ns)) {
+        case 1: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_kernel<1, true>) : reinterpret_cast<const void*>(&rates_kernel<1, false>); break;
+        case 2: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_kernel<2, true>) : reinterpret_cast<const void*>(&rates_kernel<2, false>); break;
+        case 4: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_kernel<4, true>) : reinterpret_cast<const void*>(&rates_kernel<4, false>); break;
+        case 80: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_wide_kernel<8, true>) : reinterpret_cast<const void*>(&rates_wide_kernel<8, false>); break;
+        default: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_wide_kernel<4, true>) : reinterpret_cast<const void*>(&rates_wide_kernel<4, false>); break;
+    }
+    return p;
 }
 
-hipError_t rates_launch(const DevMech& m, int ns, bool f32, long n, const double* T, const double* P,
-                        const double* Y, double* wdot, int grid, size_t lds, hipStream_t stream) {
-    if (ns == 1 && !f32)
-        hipLaunchKernelGGL((rates_kernel<1, false>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y, wdot);
-    else if (ns == 1)
-        hipLaunchKernelGGL((rates_kernel<1, true>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y, wdot);
-    else if (ns == 2 && !f32)
-        hipLaunchKernelGGL((rates_kernel<2, false>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y, wdot);
-    else if (ns == 2)
-        hipLaunchKernelGGL((rates_kernel<2, true>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y, wdot);
-    else if (rates_ns(ns) == 4 && !f32)
-        hipLaunchKernelGGL((rates_kernel<4, false>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y, wdot);
-    else if (rates_ns(ns) == 4)
-        hipLaunchKernelGGL((rates_kernel<4, true>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y, wdot);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
-const void* rates_kernel_ptr(int ns, bool f32) {
-    if (ns == 1) return f32 ? reinterpret_cast<const void*>(&rates_kernel<1, true>)
-                            : reinterpret_cast<const void*>(&rates_kernel<1, false>);
-    if (ns == 2) return f32 ? reinterpret_cast<const void*>(&rates_kernel<2, true>)
-                            : reinterpret_cast<const void*>(&rates_kernel<2, false>);
-    return f32 ? reinterpret_cast<const void*>(&rates_kernel<4, true>)
-               : reinterpret_cast<const void*>(&rates_kernel<4, false>);
+hipError_t rates_launch(const RatesPlan& p, DevMech m, long n, const double* T, const double* P, const double* Y,
+                        double* wdot, int grid, hipStream_t stream) {
+    void* args[] = {&m, &n, &T, &P, &Y, &wdot};
+    return hipLaunchKernel(p.kernel, dim3(grid), dim3(64), args, p.lds, stream);
 }
 
 }  // namespace cg

@@ -28,7 +28,7 @@ __device__ __forceinline__ void mat_add(double* p, double v) { unsafeAtomicAdd(p
 // bit 0 leaves out the third-body [M] terms, bit 1 the falloff d k/d[M]
 // (the rate then counts as linear in [M], BulkKinetics.cpp:761-792).
 __device__ __forceinline__ void scatter_reaction_derivs(const DevMech& m, int p, const GasState& g,
-                                                        SpeciesColumn C, SpeciesColumn MU,
+                                                        SpeciesColumn<> C, SpeciesColumn<> MU,
                                                         double kpd, double* A, int LD, double* acc, int skip = 0) {
     RxnRegs x;
     load_rxn(m, p, x);

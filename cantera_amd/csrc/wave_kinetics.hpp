@@ -182,10 +182,12 @@ __device__ __forceinline__ KernargMech* kernarg_mech() {
     return (KernargMech*)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
-// One member of the interleaved (C, mu) pairs of the scratch.
+// One member of the interleaved (C, mu) pairs of the scratch, which holds S
+// states side by side (p: this lane's state).
+template <int S = 1>
 struct SpeciesColumn {
     double* p;
-    __device__ __forceinline__ double& operator[](int k) const { return p[2 * k]; }
+    __device__ __forceinline__ double& operator[](int k) const { return p[2 * S * k]; }
 };
 
 // Per-wave LDS scratch for one state evaluation.
@@ -194,7 +196,7 @@ struct WaveScratch {
     // the state's pressure, (1, 0) from K on.  One 16-byte read serves a
     // species of a reaction's product and of its equilibrium constant, at the
     // address that the compact reaction record holds.
-    SpeciesColumn C, MU;
+    SpeciesColumn<> C, MU;
     double* WD;    // K + kDummy production-rate accumulators, right behind the pairs
     double* yb;    // N (state broadcast)
     double* W2;    // 2K (Jacobian: wdot, D)
@@ -202,6 +204,21 @@ struct WaveScratch {
     double* Y0;    // N (Jacobian expansion point)
     double* F0;    // N (right-hand side at Y0)
     KernargMech* mech;   // for out-of-line callees
+};
+
+// Reactions by lanes: a wavefront evaluates S states at once, 64 / S lanes per
+// state, each lane one reaction of a pass.  State s owns column s of the
+// scratch: rows of S pairs (C, mu) per species, then rows of S accumulators.
+template <int S = 1>
+struct LaneView {
+    static constexpr int kStride = 64 / S;    // reactions per pass
+    unsigned pair0;                           // byte offset of this state's pair in a row
+    double* wd;                               // this state's accumulator in the first row
+    // (C, mu/RT) and accumulator at a record's slot (16 x species)
+    __device__ __forceinline__ double2 pair(unsigned slot) const;
+    __device__ __forceinline__ double* acc(unsigned slot) const {
+        return reinterpret_cast<double*>(reinterpret_cast<char*>(wd) + (slot * S >> 1));
+    }
 };
 
 __host__ __device__ __forceinline__ int species_doubles(int K) { return 3 * (K + kDummy); }
@@ -216,6 +233,11 @@ struct ScratchLayout {
 __device__ __forceinline__ double* lds_base() {
     extern __shared__ __attribute__((aligned(16))) double lds_raw[];
     return lds_raw;
+}
+
+template <int S>
+__device__ __forceinline__ double2 LaneView<S>::pair(unsigned slot) const {
+    return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(lds_base()) + (S == 1 ? slot : slot * S + pair0));
 }
 
 __device__ __forceinline__ void bind_species(WaveScratch& S, KernargMech* mech) {
@@ -598,7 +620,8 @@ __device__ __noinline__ double sri_falloff(const double* __restrict__ fo, double
 // kTbPad entries with efficiency 0, so a group's table loads, then its
 // concentration loads, are all in flight together with no test against the
 // list length.
-__device__ __forceinline__ double efficiency_sum(const DevMech& m, SpeciesColumn C, int tbo, int tbn) {
+template <int S>
+__device__ __forceinline__ double efficiency_sum(const DevMech& m, SpeciesColumn<S> C, int tbo, int tbn) {
     double sum = 0.0;
     for (int j0 = 0; j0 == 0 || j0 < tbn; j0 += kTbPad) {
         int kk[kTbPad];
@@ -622,9 +645,9 @@ __device__ __forceinline__ double efficiency_sum(const DevMech& m, SpeciesColumn
 // FP32 transcendentals above; everything else FP64.
 // perturb: the reaction's rate multiplier (m_perturb, Kinetics::setMultiplier),
 // applied to the forward rate of progress before the reverse one is formed.
-template <bool kF32 = false>
+template <bool kF32 = false, int S = 1>
 __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const GasState& g,
-                                              SpeciesColumn C, SpeciesColumn MU,
+                                              SpeciesColumn<S> C, SpeciesColumn<S> MU,
                                               const RxnRegs& x, double kpd, RxnVals& o, double perturb = 1.0) {
     const double4 rd = reinterpret_cast<const double4*>(m.rd)[p];
     const int type = (x.flags >> 1) & 3;
@@ -779,8 +802,8 @@ __device__ __forceinline__ double zero_if_two_negative(double v, double a, doubl
 struct StdRxn {
     uint4 q;
     double4 rd;     // A, b, Ea/R, dn
-    __device__ __forceinline__ void load(const DevMech& m, int p) {
-        q = reinterpret_cast<const uint4*>(m.rs)[p];
+    __device__ __forceinline__ void load(const DevMech& m, const RxnS* rs, int p) {
+        q = reinterpret_cast<const uint4*>(rs)[p];
         rd = reinterpret_cast<const double4*>(m.rd)[p];
     }
     __device__ __forceinline__ unsigned slot(int e) const {   // entry e: r0 r1 r2 p0 p1 p2 p3
@@ -790,11 +813,6 @@ struct StdRxn {
     __device__ __forceinline__ bool reversible() const { return q.w & 0x10000u; }
     __device__ __forceinline__ bool four_products() const { return q.w & 0x20000u; }
 };
-
-// (C, mu/RT) of an entry
-__device__ __forceinline__ double2 species_pair(unsigned slot) {
-    return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(lds_base()) + slot);
-}
 
 // exponent of 1/K_c from the pairs of the six entries
 __device__ __forceinline__ double std_kc_arg(const StdRxn& x, double logC0, const double2 (&v)[6]) {
@@ -813,30 +831,29 @@ __device__ __forceinline__ double std_ropnet(const StdRxn& x, double kf, double 
     return f - (x.reversible() ? r : 0.0);
 }
 
-// -r to the reactants' accumulators, +r to the products' (an accumulator is
-// half a pair)
-__device__ __forceinline__ double* accumulator(double* wd, unsigned slot) {
-    return reinterpret_cast<double*>(reinterpret_cast<char*>(wd) + (slot >> 1));
-}
-__device__ __forceinline__ void std_scatter(double* wd, const StdRxn& x, double r) {
+// -r to the reactants' accumulators, +r to the products'
+template <int S>
+__device__ __forceinline__ void std_scatter(const LaneView<S>& v, const StdRxn& x, double r) {
 #pragma unroll
-    for (int e = 0; e < 3; e++) atomicAdd(accumulator(wd, x.slot(e)), -r);
+    for (int e = 0; e < 3; e++) atomicAdd(v.acc(x.slot(e)), -r);
 #pragma unroll
-    for (int e = 3; e < 6; e++) atomicAdd(accumulator(wd, x.slot(e)), r);
+    for (int e = 3; e < 6; e++) atomicAdd(v.acc(x.slot(e)), r);
 }
 
-// B passes of elementary reactions, lane entries p, p + 64, ...
-template <int B, bool kF32, bool kPert>
-__device__ __forceinline__ void plain_block(const DevMech& m, double* wd, const GasState& g, int p, int pert_rxn, double pert_v) {
+// B passes of elementary reactions: this lane's are p, p + 64 / S, ...
+template <int B, bool kF32, bool kPert, int S>
+__device__ __forceinline__ void plain_block(const DevMech& m, const RxnS* rs, const LaneView<S>& lv, const GasState& g,
+                                            int p, int pert_rxn, double pert_v) {
+    constexpr int kStride = LaneView<S>::kStride;
     StdRxn x[B];
 #pragma unroll
-    for (int b = 0; b < B; b++) x[b].load(m, p + kWave * b);
+    for (int b = 0; b < B; b++) x[b].load(m, rs, p + kStride * b);
     double2 v[B][6];
     double r[B], ex[2 * B];
 #pragma unroll
     for (int b = 0; b < B; b++)
 #pragma unroll
-        for (int e = 0; e < 6; e++) v[b][e] = species_pair(x[b].slot(e));
+        for (int e = 0; e < 6; e++) v[b][e] = lv.pair(x[b].slot(e));
 #pragma unroll
     for (int b = 0; b < B; b++) {
         ex[b] = x[b].rd.y * g.logT - x[b].rd.z * g.recipT;
@@ -855,15 +872,15 @@ __device__ __forceinline__ void plain_block(const DevMech& m, double* wd, const 
 #pragma unroll
     for (int b = 0; b < B; b++) {
         double kf = x[b].rd.x * ex[b];
-        if constexpr (kPert) kf *= (p + kWave * b == pert_rxn) ? pert_v : 1.0;
+        if constexpr (kPert) kf *= (p + kStride * b == pert_rxn) ? pert_v : 1.0;
         r[b] = std_ropnet(x[b], kf, ex[B + b], v[b]);
         four |= x[b].four_products();
     }
 #pragma unroll
-    for (int b = 0; b < B; b++) std_scatter(wd, x[b], r[b]);
+    for (int b = 0; b < B; b++) std_scatter(lv, x[b], r[b]);
     if (__any(four)) {
 #pragma unroll
-        for (int b = 0; b < B; b++) atomicAdd(accumulator(wd, x[b].slot(6)), r[b]);
+        for (int b = 0; b < B; b++) atomicAdd(lv.acc(x[b].slot(6)), r[b]);
     }
 }
 
@@ -871,11 +888,12 @@ __device__ __forceinline__ void plain_block(const DevMech& m, double* wd, const 
 // reactions: every lane runs the same code (the falloff part only if the pass
 // has such a reaction), the type selects among the results.  The formulas are
 // eval_reaction's.
-template <bool kF32, bool kPert>
-__device__ __forceinline__ void falloff_pass(const DevMech& m, const WaveScratch& S, const GasState& g, int p,
-                                             int pert_rxn, double pert_v) {
+template <bool kF32, bool kPert, int S>
+__device__ __forceinline__ void falloff_pass(const DevMech& m, const RxnS* rs, const LaneView<S>& lv,
+                                             SpeciesColumn<S> C, const GasState& g, int p, int pert_rxn,
+                                             double pert_v) {
     StdRxn x;
-    x.load(m, p);
+    x.load(m, rs, p);
     const int4* qi = reinterpret_cast<const int4*>(m.ri + p);
     const int4 ia = qi[0], ib = qi[1];
     const double tbdef = m.tbdef[p];
@@ -884,8 +902,8 @@ __device__ __forceinline__ void falloff_pass(const DevMech& m, const WaveScratch
     const double4 fa = f4[0], fb = f4[1];   // A0, b0, Ea0/R, a | 1/T3, 1/T1, T2, B
     double2 v[6];
 #pragma unroll
-    for (int e = 0; e < 6; e++) v[e] = species_pair(x.slot(e));
-    const double M = add_mul_rn(efficiency_sum(m, S.C, ia.w, ib.x), tbdef, g.ctot);
+    for (int e = 0; e < 6; e++) v[e] = lv.pair(x.slot(e));
+    const double M = add_mul_rn(efficiency_sum(m, C, ia.w, ib.x), tbdef, g.ctot);
     // the pass's six exponentials side by side (Troe exponents kept moderate:
     // 1/T3 is infinite for Tsang, some T2 are 1e100)
     double ex[6];
@@ -902,8 +920,13 @@ __device__ __forceinline__ void falloff_pass(const DevMech& m, const WaveScratch
         if (falloff)
 #pragma unroll
             for (int j = 2; j < 6; j++) ex[j] = rate_exp<true>(ex[j]);
-    } else {
+    } else if (falloff) {
         fast_exp_n(ex);
+    } else {
+        double e2[2] = {ex[0], ex[1]};
+        fast_exp_n(e2);
+        ex[0] = e2[0];
+        ex[1] = e2[1];
     }
     double kf = x.rd.x * ex[0];
     if (falloff) {
@@ -926,8 +949,28 @@ __device__ __forceinline__ void falloff_pass(const DevMech& m, const WaveScratch
     const double kM = opaque(kf * M);
     kf = (type == kThreeBody) ? kM : kf;
     const double r = std_ropnet(x, kf, ex[1], v);
-    std_scatter(S.WD, x, r);
-    if (__any(x.four_products())) atomicAdd(accumulator(S.WD, x.slot(6)), r);
+    std_scatter(lv, x, r);
+    if (__any(x.four_products())) atomicAdd(lv.acc(x.slot(6)), r);
+}
+
+// The standard reactions from `first` (a whole number of passes): falloff passes
+// up to mid, elementary ones up to last, kBlock of these side by side.
+template <int kBlock, bool kF32, bool kPert, int S>
+__device__ __forceinline__ void standard_passes(const DevMech& m, const RxnS* rs, const LaneView<S>& lv,
+                                                SpeciesColumn<S> C, const GasState& g, int lane, int first, int mid,
+                                                int last, int pert_rxn, double pert_v) {
+    constexpr int kStride = LaneView<S>::kStride;
+    int q = first;
+    for (; q < mid; q += kStride) falloff_pass<kF32, kPert, S>(m, rs, lv, C, g, q + lane, pert_rxn, pert_v);
+    for (; q + (kBlock - 1) * kStride < last; q += kBlock * kStride)
+        plain_block<kBlock, kF32, kPert, S>(m, rs, lv, g, q + lane, pert_rxn, pert_v);
+    if constexpr (kBlock > 2)
+        if (q + kStride < last) {
+            plain_block<2, kF32, kPert, S>(m, rs, lv, g, q + lane, pert_rxn, pert_v);
+            q += 2 * kStride;
+        }
+    if constexpr (kBlock > 1)
+        if (q < last) plain_block<1, kF32, kPert, S>(m, rs, lv, g, q + lane, pert_rxn, pert_v);
 }
 
 // Gas state + per-species thermo, concentrations and chemical potentials.
@@ -1064,18 +1107,8 @@ __device__ __forceinline__ void production_rates(const DevMech& m, const WaveScr
     if (m.gen_end > 0)
         general_passes<kF32, kPert>(S.mech, g.T, g.logT, g.recipT, g.logC0, g.ctot,
                                     g.pressure, pert_rxn, pert_v);
-    for (int q = m.gen_end; q < m.tb_end; q++) falloff_pass<kF32, kPert>(m, S, g, kWave * q + lane, pert_rxn, pert_v);
-    int q = m.tb_end;
-    const int nq = (m.I + kWave - 1) / kWave;
-    for (; q + kBlock <= nq; q += kBlock)
-        plain_block<kBlock, kF32, kPert>(m, S.WD, g, kWave * q + lane, pert_rxn, pert_v);
-    if constexpr (kBlock > 2)
-        if (q + 2 <= nq) {
-            plain_block<2, kF32, kPert>(m, S.WD, g, kWave * q + lane, pert_rxn, pert_v);
-            q += 2;
-        }
-    if constexpr (kBlock > 1)
-        if (q < nq) plain_block<1, kF32, kPert>(m, S.WD, g, kWave * q + lane, pert_rxn, pert_v);
+    standard_passes<kBlock, kF32, kPert, 1>(m, m.rs, LaneView<1>{0u, S.WD}, S.C, g, lane, kWave * m.gen_end,
+                                            kWave * m.tb_end, m.I, pert_rxn, pert_v);
     wave_sync();
 #pragma unroll
     for (int s = 0; s < NS; s++) {
