@@ -164,11 +164,11 @@ int32_t guarded(F&& f) {
     return CG_ERR;
 }
 
-int grid_for(const void* kernel, size_t lds, int waves_per_cu, long work_items) {
+int grid_for(const void* kernel, size_t lds, int waves_per_cu, long work_items, int threads = 64) {
     int per_cu = waves_per_cu;
     if (per_cu <= 0) {
         int nb = 0;
-        check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, 64, lds), "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+        check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, lds), "hipOccupancyMaxActiveBlocksPerMultiprocessor");
         per_cu = std::max(nb, 1);
     }
     long g = static_cast<long>(per_cu) * device_cu_count();
@@ -394,13 +394,16 @@ int32_t cg_jac_batch_device(int32_t h, int64_t n, const double* T, const double*
         if (n <= 0) return 0;
         if (!T || !P || !Y || !J) throw std::runtime_error("null array");
         const DevMech& m = mo.dm->view();
-        const size_t lds = jac_lds_bytes(m, mo.ns);
-        const void* kp = jac_kernel_ptr(mo.ns, f32);
+        const JacTables& jt = mo.dm->jac();
+        const bool tile = jt.nd > 0 && jac_tile_lds_bytes(m, jt) <= kLdsPerCu;
+        const size_t lds = tile ? jac_tile_lds_bytes(m, jt) : jac_lds_bytes(m, mo.ns);
+        const void* kp = tile ? jac_tile_kernel_ptr(f32) : jac_kernel_ptr(mo.ns, f32);
         set_lds_limit(kp, lds);
-        const int grid = grid_for(kp, lds, 0, n);
+        const int grid = tile ? grid_for(kp, lds, 0, jac_tile_items(n), 256) : grid_for(kp, lds, 0, n);
         hipStream_t s = static_cast<hipStream_t>(stream);
         check(hipEventRecord(mo.j0, s), "hipEventRecord");
-        check(jac_launch(m, mo.ns, f32, n, T, P, Y, J, grid, lds, s), "Jacobian kernel launch");
+        if (tile) check(jac_tile_launch(m, jt, f32, n, T, P, Y, J, grid, lds, s), "Jacobian kernel launch");
+        else check(jac_launch(m, mo.ns, f32, n, T, P, Y, J, grid, lds, s), "Jacobian kernel launch");
         check(hipEventRecord(mo.j1, s), "hipEventRecord");
         return 0;
     });

@@ -135,6 +135,13 @@ hipError_t jac_launch(const DevMech& m, int ns, bool f32, long n, const double* 
                       void* J, int grid, size_t lds, hipStream_t stream);
 const void* jac_kernel_ptr(int ns, bool f32);
 
+// the same without atomics, for mechanisms with JacTables
+size_t jac_tile_lds_bytes(const DevMech& m, const JacTables& jt);
+const void* jac_tile_kernel_ptr(bool f32);
+long jac_tile_items(long n);
+hipError_t jac_tile_launch(const DevMech& m, const JacTables& jt, bool f32, long n, const double* T, const double* P,
+                           const double* Y, void* J, int grid, size_t lds, hipStream_t stream);
+
 // batched chemical equilibrium (hp = 1: fixed h and P; 0: fixed T and P),
 // inputs and outputs species-major; info[s] = iterations, or negative
 hipError_t equil_launch(const DevMech& m, int ns, int hp, long n, const double* T, const double* P, const double* Y,

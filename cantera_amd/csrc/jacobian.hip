@@ -8,6 +8,9 @@
 // dT/dt scale with V/m = 1/rho), so the state is taken with m = 1 kg and the m
 // row and column are zero.
 //
+// For mechanisms that jac_tile.hip does not take (more than 62 species, or
+// reactions that need the general code).
+//
 // One wavefront per state: the Jacobian assembly (two RHS evaluations, at the
 // state and with T + dT, then the per-reaction derivatives), in LDS when it
 // fits, else in the state's output block.

@@ -1,13 +1,13 @@
 #include "mech.hpp"
 
 #include <algorithm>
+#include <cctype>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
 #include <map>
 #include <numeric>
-#include <sstream>
 #include <stdexcept>
 
 namespace cg {
@@ -39,6 +39,7 @@ HostMech load_mech(const std::string& path) {
     if (!f) throw std::runtime_error("cannot open mechanism file " + path);
     HostMech m;
     std::string line;
+    std::vector<std::string> t;
     bool header = false, ended = false;
     int last_r = -1;
     while (std::getline(f, line)) {
@@ -47,10 +48,13 @@ HostMech load_mech(const std::string& path) {
             if (last_r >= 0) m.rxn[last_r].equation = line.substr(2);
             continue;
         }
-        std::istringstream is(line);
-        std::vector<std::string> t;
-        std::string w;
-        while (is >> w) t.push_back(w);
+        t.clear();
+        for (size_t i = 0; i < line.size();) {
+            while (i < line.size() && std::isspace(static_cast<unsigned char>(line[i]))) i++;
+            const size_t j = i;
+            while (i < line.size() && !std::isspace(static_cast<unsigned char>(line[i]))) i++;
+            if (i > j) t.emplace_back(line, j, i - j);
+        }
         if (t.empty()) continue;
         size_t p = 1;
         auto next = [&]() -> const std::string& {
@@ -152,14 +156,22 @@ HostMech load_mech(const std::string& path) {
 }
 
 template <class T>
-const T* DeviceMech::upload(const std::vector<T>& v) {
-    size_t bytes = std::max<size_t>(v.size(), 1) * sizeof(T);
-    void* p = nullptr;
-    hip_check(hipMalloc(&p, bytes), "hipMalloc(mechanism table)");
-    allocs_.push_back(p);
-    if (!v.empty()) hip_check(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice), "hipMemcpy(mechanism table)");
-    bytes_ += bytes;
-    return static_cast<const T*>(p);
+void DeviceMech::upload(const std::vector<T>& v, const T*& dst) {
+    const size_t off = (image_.size() + 255) & ~size_t{255};
+    image_.resize(off + std::max<size_t>(v.size(), 1) * sizeof(T));
+    if (!v.empty()) std::memcpy(image_.data() + off, v.data(), v.size() * sizeof(T));
+    fix_.emplace_back(reinterpret_cast<const void**>(&dst), off);
+}
+
+void DeviceMech::finish_upload() {
+    bytes_ = image_.size();
+    hip_check(hipMalloc(&tables_, bytes_), "hipMalloc(mechanism tables)");
+    for (const auto& [dst, off] : fix_) *dst = static_cast<const char*>(tables_) + off;
+    const hipError_t e = hipMemcpy(tables_, image_.data(), bytes_, hipMemcpyHostToDevice);
+    if (e != hipSuccess) (void)hipFree(tables_);   // the destructor does not run for a constructor that throws
+    hip_check(e, "hipMemcpy(mechanism tables)");
+    image_ = {};
+    fix_ = {};
 }
 
 namespace {
@@ -385,13 +397,13 @@ DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
     if (n_pd > 64) throw std::runtime_error("mechanisms with more than 64 PLOG and Chebyshev reactions are not supported");
     d_.pref = h.pref.empty() ? 101325.0 : h.pref[0];
     d_.rpref = 1.0 / d_.pref;
-    d_.mw = upload(h.mw);
-    d_.rmw = upload(rmw);
-    d_.nasa = upload(nasa);
-    d_.rd = upload(rd);
-    d_.tbdef = upload(tbdef);
-    d_.ri = upload(ri);
-    d_.rs = upload(rs);
+    upload(h.mw, d_.mw);
+    upload(rmw, d_.rmw);
+    upload(nasa, d_.nasa);
+    upload(rd, d_.rd);
+    upload(tbdef, d_.tbdef);
+    upload(ri, d_.ri);
+    upload(rs, d_.rs);
     for (int p = 0; p < Ip; p++) {
         const auto wide = [&](unsigned short& e) {
             if (e >= 16 * K) e = static_cast<unsigned short>(16 * (K + p % kDummyWide));
@@ -399,19 +411,139 @@ DeviceMech::DeviceMech(const HostMech& h) : h_(h) {
         for (unsigned short& e : rs[p].r) wide(e);
         for (unsigned short& e : rs[p].p) wide(e);
     }
-    d_.rsw = upload(rs);
+    upload(rs, d_.rsw);
     d_.n_gen = n_gen;
     d_.n_nonplain = std::max(n_gen, n_nonplain);
-    d_.fod = upload(fod);
-    d_.gend = upload(gend);
-    d_.pdd = upload(pdd);
-    d_.tbk = upload(tbk);
-    d_.tbe = upload(tbe);
-    d_.comp = upload(h.comp);
+    upload(fod, d_.fod);
+    upload(gend, d_.gend);
+    upload(pdd, d_.pdd);
+    upload(tbk, d_.tbk);
+    upload(tbe, d_.tbe);
+    upload(h.comp, d_.comp);
+    if (n_gen == 0 && K <= 62) build_jac();
+    finish_upload();
+}
+
+void DeviceMech::build_jac() {
+    const int K = h_.K, I = h_.I;
+    constexpr int kJacPiece = 16;
+    struct Term {
+        unsigned entry, slot;
+        double c;
+    };
+    std::vector<Term> term;   // in reaction order
+    std::vector<unsigned> rxn((static_cast<size_t>(I) + 63) / 64 * 64, 0u);
+    unsigned nd = 0;
+    std::vector<int> re, pr;
+    for (int p = 0; p < I; p++) {
+        const HostReaction& r = h_.rxn[perm_[p]];
+        expand_molecules(r.rk, r.rs, re);
+        expand_molecules(r.pk, r.ps, pr);
+        int sp[8];
+        double nu[8];
+        int ns = 0;
+        auto count = [&](int k, double v) {
+            int i = 0;
+            while (i < ns && sp[i] != k) i++;
+            if (i == ns) { sp[ns] = k; nu[ns++] = 0.0; }
+            nu[i] += v;
+        };
+        for (int k : re) count(k, -1.0);
+        for (int k : pr) count(k, 1.0);
+        const size_t np = r.rev ? pr.size() : 0;
+        const bool tb = r.type != kElementary && !r.tbk.empty();
+        rxn[p] = nd | static_cast<unsigned>(re.size()) << 16 | static_cast<unsigned>(np) << 19 | (tb ? 1u << 22 : 0u);
+        auto add = [&](int j, unsigned slot, double c) {
+            for (int i = 0; i < ns; i++)
+                if (nu[i] != 0.0) term.push_back({static_cast<unsigned>(sp[i] * K + j), slot, nu[i] * c});
+        };
+        for (int j : re) add(j, nd++, 1.0);
+        for (size_t e = 0; e < np; e++) add(pr[e], nd++, 1.0);
+        if (tb) {
+            for (size_t t = 0; t < r.tbk.size(); t++) add(r.tbk[t], nd, r.tbe[t]);
+            nd++;
+        }
+    }
+    if (nd > 0xffff) return;   // the general kernel stays
+    // lists by entry (counting sort)
+    std::vector<unsigned> start(static_cast<size_t>(K) * K + 1, 0u);
+    for (const Term& t : term) start[t.entry + 1]++;
+    for (size_t e = 0; e + 1 < start.size(); e++) start[e + 1] += start[e];
+    std::vector<Term> list(term.size());
+    {
+        std::vector<unsigned> at(start.begin(), start.end() - 1);
+        for (const Term& t : term) list[at[t.entry]++] = t;
+    }
+    std::map<double, unsigned> index;
+    std::vector<double> coef;
+    auto coef_of = [&](double c) {
+        const auto it = index.emplace(c, static_cast<unsigned>(coef.size()));
+        if (it.second) coef.push_back(c);
+        return it.first->second;
+    };
+    coef_of(0.0);
+    // pieces of at most kJacPiece terms (the diagonal entries of H and OH have
+    // over a hundred): an entry's first piece is written to the matrix, the
+    // others to the overflow area, from where they are added in order
+    struct Piece {
+        const Term* t;
+        int len;
+        unsigned pos;
+    };
+    std::vector<Piece> piece;
+    std::vector<int2> split;   // matrix position, overflow pieces (consecutive over the entries)
+    unsigned next = static_cast<unsigned>(K * K);
+    for (unsigned e = 0; e < static_cast<unsigned>(K * K); e++) {
+        const int len = static_cast<int>(start[e + 1] - start[e]);
+        const Term* t = list.data() + start[e];
+        piece.push_back({t, std::min(len, kJacPiece), e});
+        for (int o = kJacPiece; o < len; o += kJacPiece)
+            piece.push_back({t + o, std::min(len - o, kJacPiece), next++});
+        if (len > kJacPiece) split.push_back(int2{static_cast<int>(e), (len - 1) / kJacPiece});
+    }
+    {
+        std::vector<Piece> byl;
+        byl.reserve(piece.size());
+        for (int l = kJacPiece; l >= 0; l--)
+            for (const Piece& x : piece)
+                if (x.len == l) byl.push_back(x);
+        piece.swap(byl);
+    }
+    const int np = static_cast<int>(piece.size()), groups = (np + 255) / 256;
+    std::vector<int2> seg(4 * static_cast<size_t>(groups));
+    std::vector<unsigned> ell;
+    std::vector<unsigned short> pos(256 * static_cast<size_t>(groups));
+    for (int b = 0; b < 4 * groups; b++) {
+        // 64 pieces of similar length; wavefront order reversed in every other
+        // group, so that no wavefront gets the longest of each
+        const int i = b / 4, w = (i % 2) ? 3 - b % 4 : b % 4;
+        const int first = 64 * b, len = first < np ? piece[first].len : 0;
+        seg[4 * i + w] = int2{static_cast<int>(ell.size() / 64), len};
+        for (int l = 0; l < 64; l++)
+            pos[256 * i + 64 * w + l] = static_cast<unsigned short>(first + l < np ? piece[first + l].pos : 0xffff);
+        for (int t = 0; t < len; t++)
+            for (int l = first; l < first + 64; l++) {
+                const bool has = l < np && t < piece[l].len;
+                ell.push_back(has ? piece[l].t[t].slot | coef_of(piece[l].t[t].c) << 16 : nd);
+            }
+    }
+    if (next > 0xfffe) return;
+    if (coef.size() > 0xffff) return;
+    jac_.ncoef = static_cast<int>(coef.size());
+    jac_.groups = groups;
+    jac_.nsplit = static_cast<int>(split.size());
+    jac_.nover = static_cast<int>(next) - K * K;
+    upload(split, jac_.split);
+    upload(rxn, jac_.rxn);
+    upload(ell, jac_.ell);
+    upload(seg, jac_.seg);
+    upload(pos, jac_.pos);
+    upload(coef, jac_.coef);
+    jac_.nd = static_cast<int>(nd);
 }
 
 DeviceMech::~DeviceMech() {
-    for (void* p : allocs_) (void)hipFree(p);
+    if (tables_) (void)hipFree(tables_);
 }
 
 }  // namespace cg

@@ -4,6 +4,7 @@
 // src/kinetics/Kinetics.cpp:709-800) for the ideal-gas bulk path.
 #pragma once
 #include <string>
+#include <utility>
 #include <vector>
 
 #include <hip/hip_runtime.h>
@@ -120,6 +121,24 @@ struct DevMech {
                              // (the P argument is the pressure), 1 IdealGasReactor (it is the volume)
 };
 
+// Tables of the batched Jacobian without atomics (jac_tile.hip; nd = 0 if the
+// mechanism does not qualify).  Each reaction stores its derivatives in
+// consecutive slots: one per reactant, one per product if reversible, one for
+// [M] if it has explicit efficiencies.  Each entry of the K x K matrix
+// d wdot / d C is a list of (slot, coefficient), long ones cut into pieces;
+// pieces are ranked by length, 256 to a group, and the 64 lists of a wavefront
+// in a group lie interleaved in rows of 64, padded with (nd, 0), whose slot
+// holds 0.
+struct JacTables {
+    int nd, ncoef, groups, nsplit, nover;
+    const unsigned* rxn;          // per reaction (permuted, padded): slot | reactants << 16 | products << 19 | [M] << 22
+    const unsigned* ell;          // slot | coefficient index << 16
+    const int2* seg;              // per group and wavefront: first row, rows
+    const unsigned short* pos;    // per lane of a group: k K + j, K K + overflow piece, or 0xffff
+    const int2* split;            // entries in several pieces: k K + j, overflow pieces
+    const double* coef;
+};
+
 // Owns device memory for a DevMech.
 class DeviceMech {
 public:
@@ -128,6 +147,7 @@ public:
     DeviceMech(const DeviceMech&) = delete;
     DeviceMech& operator=(const DeviceMech&) = delete;
     const DevMech& view() const { return d_; }
+    const JacTables& jac() const { return jac_; }
     const HostMech& host() const { return h_; }
     const std::vector<int>& perm() const { return perm_; }   // permuted index -> mechanism index
     size_t table_bytes() const { return bytes_; }
@@ -135,10 +155,17 @@ public:
 private:
     HostMech h_;
     DevMech d_{};
-    std::vector<void*> allocs_;
+    JacTables jac_{};
+    void build_jac();
+    void* tables_ = nullptr;
     std::vector<int> perm_;
     size_t bytes_ = 0;
-    template <class T> const T* upload(const std::vector<T>& v);
+    // tables are collected in one host image and copied with one allocation
+    // (finish_upload), which then sets the pointers
+    template <class T> void upload(const std::vector<T>& v, const T*& dst);
+    void finish_upload();
+    std::vector<char> image_;
+    std::vector<std::pair<const void**, size_t>> fix_;
 };
 
 }  // namespace cg

@@ -67,3 +67,27 @@ def test_nan_is_not_hidden(oracle_mod):
     reacting = np.abs(sol.net_production_rates(T[:1], P[:1], Y[0])[:, 0]) > 0
     assert np.isnan(w[reacting][:, 2:4]).all()
     assert np.isfinite(w[:, [0, 1, 4]]).all()
+
+
+@pytest.mark.parametrize("keep,n", [(range(325), 1), (range(325), 3), (range(325), 1025), (range(64), 4),
+                                    (range(261, 325), 2), (range(40, 57), 5), ([0], 2)])
+def test_jacobian_of_cut_mechanisms(keep, n, tmp_path, oracle_mod):
+    """Jacobians at ragged tile counts, at whole passes of reactions, and with
+    falloff, three-body or elementary reactions only.  Species columns against
+    the oracle's analytic ones, as the Jacobian tests of whole mechanisms."""
+    import cantera_amd as ca
+    path = cut(mech_file("gri30"), tmp_path / "m.mech", list(keep))
+    om, sol = oracle_mod.Mech(path), ca.Solution(path)
+    g = np.random.default_rng(n)
+    T = g.uniform(600.0, 2500.0, n)
+    P = 101325.0 * 10.0 ** g.uniform(-1, 1.5, n)
+    X = 10.0 ** g.uniform(-10, 0, (n, sol.n_species))
+    Y = sol.mass_fractions_from_moles(X / X.sum(axis=1, keepdims=True))
+    J = sol.reactor_jacobians(T, P, Y.T)
+    J32 = sol.reactor_jacobians(T, P, Y.T, precision=ca.CG_FP32)
+    np.testing.assert_array_equal(J32, J.astype(np.float32))
+    assert not J[:, 0].any() and not J[:, :, 0].any()
+    for s in {0, n // 2, n - 1}:
+        Jo = om.jacobian(P[s], np.concatenate(([1.0, T[s]], Y[s])), analytic=True)
+        scale = np.abs(Jo[:, 2:]).max(axis=1, keepdims=True) + 1e-300
+        assert (np.abs(J[s][:, 2:] - Jo[:, 2:]) / scale).max() <= 1e-10
