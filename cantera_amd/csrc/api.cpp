@@ -660,7 +660,7 @@ int32_t cg_reactors_create_mole(int32_t h, int64_t n, const double* T0, const do
         // and a device copy of its tables (the internal index layout is
         // this library's, so the permutation is applied to the reaction
         // species lists of the host mechanism: reactions in mechanism order)
-        const SparseLUHost sl = sparse_lu_analyse(N, mole_pattern(hm, flags & 1, cv));
+        const SparseLUHost sl = sparse_lu_analyse(N, mole_pattern(hm, flags & 1, cv), 64 * bdf_mole_ns(N));
         auto b = std::make_unique<Batch>();
         b->mech = &mo;
         b->mole = true;
@@ -679,9 +679,24 @@ int32_t cg_reactors_create_mole(int32_t h, int64_t n, const double* T0, const do
         b->lu_stride = static_cast<size_t>(sl.nnz);
         b->piv_stride = 1;
         b->sp_updates = sl.updates();
-        // tables: diag, lptr, lslot, lrow, optr, ops, uptr, uslot, urow, iperm, srow, scol
-        std::vector<const std::vector<int>*> parts = {&sl.diag, &sl.lptr, &sl.lslot, &sl.lrow, &sl.optr, &sl.ops,
-                                                      &sl.uptr, &sl.uslot, &sl.urow, &sl.iperm, &sl.row, &sl.col};
+        // refused before any table of it is used
+        const size_t lds = bdf_mole_lds_bytes(m, N, sl.nnz);
+        if (lds > kLdsPerCu)
+            throw std::runtime_error("the preconditioner's fill pattern (" + std::to_string(sl.nnz) +
+                                     " entries) needs " + std::to_string(lds / 1024) +
+                                     " KiB of LDS per reactor, more than the " + std::to_string(kLdsPerCu / 1024) +
+                                     " KiB of a CU; skipping the third-body and falloff derivatives (flags 1 | 2) "
+                                     "makes it sparser");
+        // tables: ops (8-byte pairs, so first), fwd and bwd (two slots an int),
+        // diag, lptr, lslot, optr, iperm, row, col
+        auto packed = [](const std::vector<unsigned short>& v) {
+            std::vector<int> o(v.size() / 2);
+            std::memcpy(o.data(), v.data(), 2 * v.size());
+            return o;
+        };
+        const std::vector<int> fwd = packed(sl.fwd), bwd = packed(sl.bwd);
+        std::vector<const std::vector<int>*> parts = {&sl.ops, &fwd, &bwd, &sl.diag, &sl.lptr, &sl.lslot,
+                                                      &sl.optr, &sl.iperm, &sl.row, &sl.col};
         size_t total = 0;
         for (auto* v : parts) total += v->size() + 1;
         std::vector<int> flat;
@@ -698,9 +713,11 @@ int32_t cg_reactors_create_mole(int32_t h, int64_t n, const double* T0, const do
         const int* d = b->sp_tables;
         b->sp.nnz = sl.nnz;
         b->sp.skip = flags & 3;
-        b->sp.diag = d + off[0]; b->sp.lptr = d + off[1]; b->sp.lslot = d + off[2]; b->sp.lrow = d + off[3];
-        b->sp.optr = d + off[4]; b->sp.ops = d + off[5]; b->sp.uptr = d + off[6]; b->sp.uslot = d + off[7];
-        b->sp.urow = d + off[8]; b->sp.iperm = d + off[9]; b->sp.srow = d + off[10]; b->sp.scol = d + off[11];
+        b->sp.ops = d + off[0];
+        b->sp.fwd = reinterpret_cast<const unsigned short*>(d + off[1]);
+        b->sp.bwd = reinterpret_cast<const unsigned short*>(d + off[2]);
+        b->sp.diag = d + off[3]; b->sp.lptr = d + off[4]; b->sp.lslot = d + off[5]; b->sp.optr = d + off[6];
+        b->sp.iperm = d + off[7]; b->sp.srow = d + off[8]; b->sp.scol = d + off[9];
         check(hipMalloc(&b->rec, b->rec_stride * n * 8), "hipMalloc(records)");
         check(hipMalloc(&b->jsave, b->j_stride * n * 8), "hipMalloc(jacobians)");
         check(hipMalloc(&b->lusave, b->lu_stride * n * 8), "hipMalloc(factors)");
@@ -739,13 +756,7 @@ int32_t cg_reactors_create_mole(int32_t h, int64_t n, const double* T0, const do
             c[C_ATOL_SP] = (flags & 4) ? atol : atol * tot;
         }
         check(hipMemcpy(b->rec, rec.data(), rec.size() * 8, hipMemcpyHostToDevice), "hipMemcpy(records)");
-        b->lds = bdf_mole_lds_bytes(m, sl.nnz);
-        if (b->lds > kLdsPerCu)
-            throw std::runtime_error("the preconditioner's fill pattern (" + std::to_string(sl.nnz) +
-                                     " entries) needs " + std::to_string(b->lds / 1024) +
-                                     " KiB of LDS per reactor, more than the " + std::to_string(kLdsPerCu / 1024) +
-                                     " KiB of a CU; skipping the third-body and falloff derivatives (flags 1 | 2) "
-                                     "makes it sparser");
+        b->lds = lds;
         set_lds_limit(bdf_mole_kernel_ptr(N), b->lds);
         std::lock_guard<std::mutex> lk(g_mu);
         g_batches.push_back(std::move(b));

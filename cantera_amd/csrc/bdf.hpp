@@ -25,7 +25,8 @@ enum CtlIndex {
 struct SparseTables {
     int nnz;                                    // value slots of L + U
     int skip;                                   // bit 0: no third-body terms, bit 1: no falloff d k/d[M]
-    const int *diag, *lptr, *lslot, *lrow, *optr, *ops, *uptr, *uslot, *urow, *iperm, *srow, *scol;
+    const int *diag, *lptr, *lslot, *optr, *ops, *iperm, *srow, *scol;
+    const unsigned short *fwd, *bwd;
 };
 
 // most reaction-multiplier sensitivity parameters per reactor batch
@@ -80,7 +81,7 @@ const void* bdf_kernel_ptr(int N, bool fp32, bool global, bool sens = false);
 
 // mole-reactor integrator: state [n_0..n_{K-1}, T], N = K + 1 <= 256
 int bdf_mole_ns(int N);
-size_t bdf_mole_lds_bytes(const DevMech& m, int nnz);
+size_t bdf_mole_lds_bytes(const DevMech& m, int N, int nnz);
 hipError_t bdf_mole_launch(const BdfArgs& a, int grid, size_t lds, hipStream_t stream);
 const void* bdf_mole_kernel_ptr(int N);
 

@@ -1410,8 +1410,9 @@ struct Integrator {
 
 // LDS per wavefront: state broadcast, species/reaction scratch, control block,
 // then the linear-system area (LDS policy only).
-__host__ __device__ inline size_t bdf_scratch_doubles(int K, int ns) {
-    return static_cast<size_t>(kWave) * ns * 4 + species_doubles(K) + 2 * K + kCtlDoubles;
+// The mole reactor needs no F0 and half of W2.
+__host__ __device__ inline size_t bdf_scratch_doubles(int K, int ns, bool mole = false) {
+    return static_cast<size_t>(kWave) * ns * (mole ? 3 : 4) + species_doubles(K) + (mole ? 1 : 2) * K + kCtlDoubles;
 }
 
 template <int NS, class LS, typename MT, bool kSens = false, bool kMole = false>
@@ -1422,8 +1423,9 @@ __device__ __forceinline__ void bdf_advance_body(const BdfArgs& a) {
     L.yb = off;  off += kWave * NS;
     L.F = off;   off += kWave * NS;
     L.Y0 = off;  off += kWave * NS;
-    L.F0 = off;  off += kWave * NS;
-    L.W2 = off;  off += 2 * m.K;
+    L.F0 = off;
+    if (!kMole) off += kWave * NS;
+    L.W2 = off;  off += (kMole ? 1 : 2) * m.K;
     double* base = lds_base() + off;
     Ctl& c = *reinterpret_cast<Ctl*>(base);
     base += kCtlDoubles;

@@ -15,10 +15,9 @@ __global__ __launch_bounds__(64) void bdf_advance_mole(BdfArgs a) {
 
 int bdf_mole_ns(int N) { return N <= 64 ? 1 : (N <= 128 ? 2 : (N <= 256 ? 4 : -1)); }
 
-size_t bdf_mole_lds_bytes(const DevMech& m, int nnz) {
-    const int ns = bdf_mole_ns(m.K + 1);
-    const size_t lu = (static_cast<size_t>(nnz) + 1) & ~static_cast<size_t>(1);
-    return (bdf_scratch_doubles(m.K, ns) + lu + static_cast<size_t>(kWave) * ns + kGmDoubles) * sizeof(double);
+size_t bdf_mole_lds_bytes(const DevMech& m, int N, int nnz) {
+    const int ns = bdf_mole_ns(N);
+    return (bdf_scratch_doubles(m.K, ns, true) + SparseLdsLinSys<1>::lds_doubles(nnz, ns)) * sizeof(double);
 }
 
 const void* bdf_mole_kernel_ptr(int N) {
@@ -32,7 +31,7 @@ const void* bdf_mole_kernel_ptr(int N) {
 
 hipError_t bdf_mole_launch(const BdfArgs& a, int grid, size_t lds, hipStream_t stream) {
     hipLaunchKernelGGL(reset_mole_queue, dim3(1), dim3(1), 0, stream, a.queue);
-    switch (bdf_mole_ns(a.mech.K + 1)) {
+    switch (bdf_mole_ns(a.neq_norm)) {
         case 1: hipLaunchKernelGGL(bdf_advance_mole<1>, dim3(grid), dim3(64), lds, stream, a); break;
         case 2: hipLaunchKernelGGL(bdf_advance_mole<2>, dim3(grid), dim3(64), lds, stream, a); break;
         case 4: hipLaunchKernelGGL(bdf_advance_mole<4>, dim3(grid), dim3(64), lds, stream, a); break;

@@ -5,8 +5,8 @@
 
 namespace cg {
 
-SparseLUHost sparse_lu_analyse(int N, const std::vector<char>& pattern) {
-    if (N <= 0 || static_cast<int>(pattern.size()) != N * N) throw std::runtime_error("sparse_lu_analyse: bad pattern");
+SparseLUHost sparse_lu_analyse(int N, const std::vector<char>& pattern, int width) {
+    if (N <= 0 || N > width || static_cast<int>(pattern.size()) != N * N) throw std::runtime_error("sparse_lu_analyse: bad pattern");
     SparseLUHost s;
     s.N = N;
     // minimum-degree order on the symmetrised elimination graph (ties to the
@@ -60,29 +60,29 @@ SparseLUHost sparse_lu_analyse(int N, const std::vector<char>& pattern) {
         for (int c = 0; c < N; c++) s.pos[r * N + c] = slot[s.iperm[r] * N + s.iperm[c]];
     s.diag.resize(N);
     for (int k = 0; k < N; k++) s.diag[k] = slot[k * N + k];
+    // 16-bit slots: patterns of 65,535 entries and more are far beyond a CU's LDS
+    if (s.nnz >= 0xffff) return s;
+    s.width = width;
+    s.fwd.assign(static_cast<size_t>(N) * width, static_cast<unsigned short>(s.nnz));
+    s.bwd = s.fwd;
     s.lptr.push_back(0);
     s.optr.push_back(0);
-    s.uptr.push_back(0);
     for (int k = 0; k < N; k++) {
         for (int i = k + 1; i < N; i++)
             if (F[i * N + k]) {
                 s.lslot.push_back(slot[i * N + k]);
-                s.lrow.push_back(i);
+                s.fwd[static_cast<size_t>(k) * width + i] = static_cast<unsigned short>(slot[i * N + k]);
                 for (int j = k + 1; j < N; j++)
                     if (F[k * N + j]) {
-                        s.ops.push_back(slot[i * N + j]);
-                        s.ops.push_back(slot[i * N + k]);
+                        s.ops.push_back(static_cast<int>(static_cast<unsigned>(slot[i * N + j]) |
+                                                         static_cast<unsigned>(slot[i * N + k]) << 16));
                         s.ops.push_back(slot[k * N + j]);
                     }
             }
         for (int i = 0; i < k; i++)
-            if (F[i * N + k]) {
-                s.uslot.push_back(slot[i * N + k]);
-                s.urow.push_back(i);
-            }
+            if (F[i * N + k]) s.bwd[static_cast<size_t>(k) * width + i] = static_cast<unsigned short>(slot[i * N + k]);
         s.lptr.push_back(static_cast<int>(s.lslot.size()));
-        s.optr.push_back(static_cast<int>(s.ops.size() / 3));
-        s.uptr.push_back(static_cast<int>(s.uslot.size()));
+        s.optr.push_back(static_cast<int>(s.ops.size() / 2));
     }
     return s;
 }

@@ -24,15 +24,19 @@ struct SparseLUHost {
     std::vector<int> row, col; // value slot -> internal (row, col)
     std::vector<int> diag;     // elimination position k -> slot of (k, k)
     // factorisation step k: L entries of column k (slots), then the updates
-    // a_ij -= l_ik u_kj as (slot ij, slot ik, slot kj) triples
-    std::vector<int> lptr, lslot, lrow;   // lrow: elimination position of each L entry's row
-    std::vector<int> optr, ops;           // ops: 3 ints per update
-    // backward solve: U column k above the diagonal (slots, row positions)
-    std::vector<int> uptr, uslot, urow;
-    long updates() const { return static_cast<long>(ops.size() / 3); }
+    // a_ij -= l_ik u_kj, two ints each: slot ij | slot ik << 16, slot kj
+    std::vector<int> lptr, lslot;
+    std::vector<int> optr, ops;
+    // triangular solves: per elimination step k a row of `width` slots, one per
+    // matrix row i: that of L(i, k), i > k (fwd), or U(i, k), i < k (bwd); slot
+    // nnz, which holds 0, where there is no entry
+    int width = 0;
+    std::vector<unsigned short> fwd, bwd;
+    long updates() const { return static_cast<long>(ops.size() / 2); }
 };
 
 // pattern: N x N booleans (row-major, internal order); the diagonal is added.
-SparseLUHost sparse_lu_analyse(int N, const std::vector<char>& pattern);
+// width: lanes x slots of the solving wavefront (>= N).
+SparseLUHost sparse_lu_analyse(int N, const std::vector<char>& pattern, int width);
 
 }  // namespace cg
