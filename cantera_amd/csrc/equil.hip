@@ -14,14 +14,19 @@
 //
 // Layout: inputs and outputs species-major as the batched rates (T[n], P[n],
 // Y[k*n + s]).  One wavefront per state: lane k owns species k (slot s for
-// k = lane + 64 s); the sums of the Newton matrix are wavefront reductions,
-// the (E+2) x (E+2) system is solved by one lane in LDS.  Work per iteration
-// is O(K E^2), HBM traffic per state the state in and out (compute-bound,
-// FP64 VALU).
+// k = lane + 64 s), with its NASA coefficients and element counts in registers
+// for the whole kernel.  The Newton matrix and right-hand side are entries of
+// one contraction G = V^T diag(n) V over the species with V's columns the
+// element counts, 1, h/RT, mu/RT and cp/R (E + 4 <= 12): V goes to LDS and
+// v_mfma_f64_16x16x4f64 sums four species at a time.  The (E+2) x (E+2)
+// system is solved row per lane in registers (RegLinSys).  (As wavefront
+// sums, 36 per iteration for 5 elements, with the system eliminated by one
+// lane in LDS, 20,011 gri30 states took 3.7 ms; HBM traffic is the state in
+// and out.)
 #include <hip/hip_runtime.h>
 
 #include "bdf.hpp"
-#include "wave_kinetics.hpp"
+#include "linsys.hpp"
 
 namespace cg {
 
@@ -37,30 +42,66 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
                                                    const double* __restrict__ Pin, const double* __restrict__ Yin,
                                                    double* __restrict__ Tout, double* __restrict__ Yout,
                                                    int* __restrict__ info, int max_iter) {
-    __shared__ double As[kEqMaxNu * kEqMaxNu];
-    __shared__ double xs[kEqMaxNu];
+    // columns of V: elements 0 .. E-1, then 1, h, mu, cp; odd strides, so that
+    // a column of lanes and a row of columns are both free of bank conflicts
+    constexpr int kCols = 17;
+    __shared__ double Vs[kWave * NS * kCols];
+    __shared__ double ns[kWave * NS];
+    __shared__ double Gs[16 * kCols];
     const int lane = lane_id();
     const int K = m.K, E = m.E;
+    const int cOne = E, cH = E + 1, cMu = E + 2, cCp = E + 3;
+    const int nu = E + 1 + (hp ? 1 : 0);
+    // the lane's species
+    double cl[NS][7], ch[NS][7], tmid[NS], el[NS][kEqMaxE], rmw[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        const int k = lane + kWave * s, kc = min(k, K - 1);
+        const double* c16 = m.nasa + 16 * kc;
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            cl[s][j] = c16[j];
+            ch[s][j] = c16[8 + j];
+        }
+        tmid[s] = c16[7];
+        rmw[s] = m.rmw[kc];
+#pragma unroll
+        for (int e = 0; e < kEqMaxE; e++) el[s][e] = (k < K && e < E) ? m.comp[kc * E + e] : 0.0;
+#pragma unroll
+        for (int c = 0; c < kCols; c++) Vs[k * kCols + c] = 0.0;
+#pragma unroll
+        for (int e = 0; e < kEqMaxE; e++)
+            if (e < E) Vs[k * kCols + e] = el[s][e];
+        Vs[k * kCols + cOne] = 1.0;
+        ns[k] = 0.0;
+    }
+    wave_sync();
+    auto thermo = [&](int s, double T, double recipT, double logT, double& cp, double& h, double& g) {
+        const bool low = T <= tmid[s];
+        double c[7];
+#pragma unroll
+        for (int j = 0; j < 7; j++) c[j] = low ? cl[s][j] : ch[s][j];
+        const double ct1 = c[1] * T, ct2 = c[2] * (T * T), ct3 = c[3] * (T * T * T), ct4 = c[4] * (T * T * T * T);
+        cp = c[0] + ct1 + ct2 + ct3 + ct4;
+        h = c[0] + 0.5 * ct1 + 1.0 / 3.0 * ct2 + 0.25 * ct3 + 0.2 * ct4 + c[5] * recipT;
+        g = h - (c[0] * logT + ct1 + 0.5 * ct2 + 1.0 / 3.0 * ct3 + 0.25 * ct4 + c[6]);
+    };
     const XcdStates xst(n);
     for (long st = xst.lo; st < xst.hi; st += xst.step) {
         const double T0 = uni(Tin[st]);
         const double P = uni(Pin[st]);
-        double y[NS], tt[6];
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-            const int k = lane + kWave * s;
-            y[s] = (k < K) ? Yin[static_cast<size_t>(k) * n + st] : 0.0;
-        }
         // element amounts [kmol/kg] and specific enthalpy of the input state
-        tt[0] = T0; tt[1] = T0 * T0; tt[2] = tt[1] * T0; tt[3] = tt[2] * T0; tt[4] = 1.0 / T0; tt[5] = log(T0);
-        double hl = 0.0;
+        double hl = 0.0, ny[NS];
+        const double rT0 = 1.0 / T0, lT0 = log(T0);
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             const int k = lane + kWave * s;
+            ny[s] = 0.0;
             if (k < K) {
-                double cp, h, sR, g;
-                nasa7(m.nasa + 16 * k, T0, tt, cp, h, sR, g);
-                hl += y[s] * m.rmw[k] * h;
+                double cp, h, g;
+                ny[s] = Yin[static_cast<size_t>(k) * n + st] * rmw[s];
+                thermo(s, T0, rT0, lT0, cp, h, g);
+                hl += ny[s] * h;
             }
         }
         const double h0 = uni(wave_sum(hl)) * kGasConstant * T0;
@@ -71,10 +112,7 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
             double v = 0.0;
             if (e < E) {
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    const int k = lane + kWave * s;
-                    if (k < K) v += m.comp[k * E + e] * y[s] * m.rmw[k];
-                }
+                for (int s = 0; s < NS; s++) v += el[s][e] * ny[s];
                 v = uni(wave_sum(v));
             }
             b0[e] = v;
@@ -84,17 +122,21 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
 #pragma unroll
         for (int e = 0; e < kEqMaxE; e++)
             if (e < E && b0[e] > 1e-14 * bmax) emask |= 1u << e;
-        const int ne = __builtin_popcount(emask);
-        const int nu = ne + 1 + (hp ? 1 : 0);
+        // this lane's row of the system: element, ln n or ln T; its
+        // right-hand side b_q (elements)
+        const bool elem = lane < E && ((emask >> lane) & 1u);
+        const bool row_on = elem || lane == cOne || (hp && lane == cH);
+        double bq0 = 0.0;
+#pragma unroll
+        for (int e = 0; e < kEqMaxE; e++) bq0 = (lane == e) ? b0[e] : bq0;
         bool act[NS];
         double lnn[NS];
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            const int k = lane + kWave * s;
-            bool a = k < K;
-            if (a)
-                for (int e = 0; e < E; e++)
-                    if (!((emask >> e) & 1u) && m.comp[k * E + e] != 0.0) a = false;
+            bool a = lane + kWave * s < K;
+#pragma unroll
+            for (int e = 0; e < kEqMaxE; e++)
+                if (!((emask >> e) & 1u) && el[s][e] != 0.0) a = false;
             act[s] = a;
             lnn[s] = a ? log(0.1 / K) : 0.0;
         }
@@ -103,125 +145,73 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
         const double lnP = log(P / m.pref);
         int status = -1, it = 0;
         for (; it < max_iter; it++) {
-            tt[0] = T; tt[1] = T * T; tt[2] = tt[1] * T; tt[3] = tt[2] * T; tt[4] = 1.0 / T; tt[5] = log(T);
-            double nj[NS], mu[NS], hj[NS], cpj[NS];
-            double l_sumn = 0.0, l_sh = 0.0, l_scp = 0.0, l_shh = 0.0, l_snmu = 0.0, l_snhmu = 0.0;
+            const double recipT = 1.0 / T, logT = log(T);
+            double nj[NS], mu[NS], hj[NS];
 #pragma unroll
             for (int s = 0; s < NS; s++) {
+                double cp, h, g;
+                thermo(s, T, recipT, logT, cp, h, g);
+                hj[s] = act[s] ? h : 0.0;
+                mu[s] = act[s] ? g + (lnn[s] - lnntot) + lnP : 0.0;
+                nj[s] = act[s] ? fast_exp(lnn[s]) : 0.0;
                 const int k = lane + kWave * s;
-                nj[s] = mu[s] = hj[s] = cpj[s] = 0.0;
-                if (act[s]) {
-                    double cp, h, sR, g;
-                    nasa7(m.nasa + 16 * k, T, tt, cp, h, sR, g);
-                    hj[s] = h;
-                    cpj[s] = cp;
-                    mu[s] = g + (lnn[s] - lnntot) + lnP;
-                    nj[s] = exp(lnn[s]);
-                    l_sumn += nj[s];
-                    l_sh += nj[s] * h;
-                    l_scp += nj[s] * cp;
-                    l_shh += nj[s] * h * h;
-                    l_snmu += nj[s] * mu[s];
-                    l_snhmu += nj[s] * h * mu[s];
-                }
+                Vs[k * kCols + cH] = hj[s];
+                Vs[k * kCols + cMu] = mu[s];
+                Vs[k * kCols + cCp] = act[s] ? cp : 0.0;
+                ns[k] = nj[s];
             }
-            const double sumn = uni(wave_sum(l_sumn)), sh = uni(wave_sum(l_sh)), scp = uni(wave_sum(l_scp));
-            const double shh = uni(wave_sum(l_shh)), snmu = uni(wave_sum(l_snmu)), snhmu = uni(wave_sum(l_snhmu));
-            const double ntot = exp(lnntot);
-            // element rows: sum_j a_qj a_rj n_j, b_q, sum_j a_qj n_j h_j, sum_j a_qj n_j mu_j
-            int pq = 0;
-            for (int q = 0; q < E; q++) {
-                if (!((emask >> q) & 1u)) continue;
-                double lb = 0.0, lh = 0.0, lm = 0.0;
+            const double ntot = fast_exp(lnntot);
+            wave_sync();
+            // lane l holds V(k, l % 16), k = 4 c + l / 16, as left and, times
+            // n_k, as right operand; two accumulators break the chain
+            mfma_d4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
+            {
+                const int kq = lane >> 4, lr = lane & 15;
+                for (int k0 = 0; k0 < K; k0 += 8) {   // rows past K are zero
+                    const int ka = k0 + kq, kb = k0 + 4 + kq;
+                    const double va = Vs[ka * kCols + lr], na = ns[ka], vb = Vs[kb * kCols + lr], nb = ns[kb];
+                    acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(va, na * va, acc0, 0, 0, 0);
+                    acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(vb, nb * vb, acc1, 0, 0, 0);
+                }
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    const int k = lane + kWave * s;
-                    if (act[s]) {
-                        const double an = m.comp[k * E + q] * nj[s];
-                        lb += an;
-                        lh += an * hj[s];
-                        lm += an * mu[s];
-                    }
-                }
-                const double bq = uni(wave_sum(lb)), hq = uni(wave_sum(lh)), mq = uni(wave_sum(lm));
-                int pr = pq;
-                for (int r = q; r < E; r++) {
-                    if (!((emask >> r) & 1u)) continue;
-                    double lr = 0.0;
-#pragma unroll
-                    for (int s = 0; s < NS; s++) {
-                        const int k = lane + kWave * s;
-                        if (act[s]) lr += m.comp[k * E + q] * m.comp[k * E + r] * nj[s];
-                    }
-                    const double rqr = uni(wave_sum(lr));
-                    if (lane == 0) {
-                        As[pq * nu + pr] = rqr;
-                        As[pr * nu + pq] = rqr;
-                    }
-                    pr++;
-                }
-                if (lane == 0) {
-                    As[pq * nu + ne] = bq;
-                    As[ne * nu + pq] = bq;
-                    xs[pq] = b0[q] - bq + mq;
-                    if (hp) {
-                        As[pq * nu + ne + 1] = hq;
-                        As[(ne + 1) * nu + pq] = hq;
-                    }
-                }
-                pq++;
-            }
-            if (lane == 0) {
-                As[ne * nu + ne] = sumn - ntot;
-                xs[ne] = ntot - sumn + snmu;
-                if (hp) {
-                    As[ne * nu + ne + 1] = sh;
-                    As[(ne + 1) * nu + ne] = sh;
-                    As[(ne + 1) * nu + ne + 1] = scp + shh;
-                    xs[ne + 1] = h0 / (kGasConstant * T) - sh + snhmu;
-                }
-                // Gaussian elimination with partial pivoting (nu <= 10)
-                int sing = 0;
-                for (int c = 0; c < nu; c++) {
-                    int p = c;
-                    for (int r = c + 1; r < nu; r++)
-                        if (fabs(As[r * nu + c]) > fabs(As[p * nu + c])) p = r;
-                    if (As[p * nu + c] == 0.0) { sing = 1; break; }
-                    if (p != c) {
-                        for (int k = 0; k < nu; k++) {
-                            const double t = As[c * nu + k]; As[c * nu + k] = As[p * nu + k]; As[p * nu + k] = t;
-                        }
-                        const double t = xs[c]; xs[c] = xs[p]; xs[p] = t;
-                    }
-                    for (int r = c + 1; r < nu; r++) {
-                        const double f = As[r * nu + c] / As[c * nu + c];
-                        for (int k = c; k < nu; k++) As[r * nu + k] -= f * As[c * nu + k];
-                        xs[r] -= f * xs[c];
-                    }
-                }
-                if (!sing)
-                    for (int c = nu - 1; c >= 0; c--) {
-                        double v = xs[c];
-                        for (int k = c + 1; k < nu; k++) v -= As[c * nu + k] * xs[k];
-                        xs[c] = v / As[c * nu + c];
-                    }
-                else
-                    xs[0] = __builtin_nan("");
+                for (int r = 0; r < 4; r++) Gs[(kq + 4 * r) * kCols + lr] = acc0[r] + acc1[r];
             }
             wave_sync();
-            if (!(xs[0] == xs[0])) { status = -3; break; }
-            const double dlnN = uni(xs[ne]), dlnT = hp ? uni(xs[ne + 1]) : 0.0;
+            RegLinSys<kEqMaxNu, double> ls;
+            const int row = min(lane, nu - 1);
+            const double sumn = uni(Gs[cOne * kCols + cOne]);
+#pragma unroll
+            for (int j = 0; j < kEqMaxNu; j++) {
+                double v = Gs[row * kCols + min(j, nu - 1)];
+                if (j == lane) {
+                    v -= (lane == cOne) ? ntot : 0.0;
+                    v += (lane == cH) ? Gs[cOne * kCols + cCp] : 0.0;
+                }
+                // an element that the state lacks: 1 on the diagonal, 0 elsewhere
+                ls.a[j] = (lane < nu && j < nu) ? (row_on ? v : (j == lane ? 1.0 : 0.0)) : 0.0;
+            }
+            double x;
+            {
+                const double gmu = Gs[row * kCols + cMu], gone = Gs[row * kCols + cOne];
+                const double lead = elem ? bq0 : (lane == cOne ? ntot : h0 / (kGasConstant * T));
+                x = row_on ? lead - gone + gmu : 0.0;
+            }
+            const bool ok = ls.factor(nu);
+            if (ok) x = ls.solve(x, nu);
+            if (!ok || __any(lane < nu && !(x == x))) { status = -3; break; }
+            const double dlnN = readlane_f64(x, cOne), dlnT = hp ? readlane_f64(x, cH) : 0.0;
+            double pi[kEqMaxE];
+#pragma unroll
+            for (int e = 0; e < kEqMaxE; e++) pi[e] = readlane_f64(x, e);
             double d[NS];
             double l_big = 0.0, l_conv = 0.0, l_lam2 = 1.0;
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                const int k = lane + kWave * s;
                 d[s] = 0.0;
                 if (act[s]) {
                     double v = -mu[s] + dlnN + hj[s] * dlnT;
-                    int p = 0;
-                    for (int e = 0; e < E; e++)
-                        if ((emask >> e) & 1u) v += m.comp[k * E + e] * xs[p++];
+#pragma unroll
+                    for (int e = 0; e < kEqMaxE; e++) v += (e < E) ? el[s][e] * pi[e] : 0.0;
                     d[s] = v;
                     const double lnx = lnn[s] - lnntot;
                     if (lnx > -kSize) {
@@ -242,14 +232,13 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
             for (int s = 0; s < NS; s++)
                 if (act[s]) lnn[s] += lam * d[s];
             lnntot += lam * dlnN;
-            if (hp) T = fmin(fmax(T * exp(lam * dlnT), 200.0), 6000.0);
+            if (hp) T = fmin(fmax(T * fast_exp(lam * dlnT), 200.0), 6000.0);
             if (lam == 1.0 && conv < 1e-12) { status = 0; it++; break; }
         }
         double yo[NS], ysum = 0.0;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            const int k = lane + kWave * s;
-            yo[s] = act[s] ? exp(lnn[s]) / m.rmw[k] : 0.0;
+            yo[s] = act[s] ? exp(lnn[s]) / rmw[s] : 0.0;
             ysum += yo[s];
         }
         ysum = uni(wave_sum(ysum));
