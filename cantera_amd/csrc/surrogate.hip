@@ -18,24 +18,36 @@ namespace {
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0;   // NaN
-    u += 0x7fffu + ((u >> 16) & 1u);                        // round to nearest even
-    return static_cast<uint16_t>(u >> 16);
-}
+// round to nearest even (v_cvt_pk_bf16_f32); NaN stays NaN
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(static_cast<uint32_t>(h) << 16); }
 
 // GELU, tanh form (Hendrycks & Gimpel 2016), and its derivative.
 constexpr float kGeluC = 0.7978845608028654f;   // sqrt(2/pi)
 constexpr float kGeluA = 0.044715f;
+// 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)): one hardware exponential and one
+// reciprocal (1 ulp each) instead of tanhf's ~30 instructions, which took
+// longer than a 256-wide layer's matrix products.  With t = exp(-2|u|) and
+// r = 1 / (1 + t), gelu(z) = max(z, 0) - |z| t r and the derivative of the
+// gate is t r^2 times that of 2u, both without cancellation.  Over |z| <= 12,
+// exponential and reciprocal each off by an ulp,
+// the largest errors against 64 bits are 2.4e-7 and 3.8e-7 (with tanhf 4.7e-7
+// and 1.2e-6), the RMS errors 4e-8 and 1e-7 (6e-8 and 1.9e-7).
+constexpr float kGelu1 = 2.0f * kGeluC, kGelu3 = 2.0f * kGeluC * kGeluA, kLog2e = 1.4426950408889634f;
+struct Gate { float t, r; };
+__device__ __forceinline__ Gate gelu_gate(float z) {
+    const float w = fabsf(z) * fmaf(z * z, kGelu3 * kLog2e, kGelu1 * kLog2e);   // 2|u| log2(e)
+    const float t = __builtin_amdgcn_exp2f(-w);
+    return {t, __builtin_amdgcn_rcpf(1.0f + t)};
+}
 __device__ __forceinline__ float gelu(float z) {
-    const float t = tanhf(kGeluC * (z + kGeluA * z * z * z));
-    return 0.5f * z * (1.0f + t);
+    const Gate g = gelu_gate(z);
+    return fmaf(-fminf(fabsf(z), 1e30f), g.t * g.r, fmaxf(z, 0.0f));   // 1e30: no inf * 0
 }
 __device__ __forceinline__ float gelu_grad(float z) {
-    const float t = tanhf(kGeluC * (z + kGeluA * z * z * z));
-    return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * kGeluC * (1.0f + 3.0f * kGeluA * z * z);
+    const Gate g = gelu_gate(z);
+    const float tr = g.t * g.r;
+    return fmaf(z * (tr * g.r), fmaf(z * z, 3.0f * kGelu3, kGelu1), z >= 0.0f ? g.r : tr);
 }
 
 enum Epi { kFwdGelu = 0, kFwdLinear = 1, kStoreF32 = 2, kBwdGelu = 3 };
@@ -273,111 +285,149 @@ __global__ void to_bf16_kernel(size_t n, const float* __restrict__ w, uint16_t* 
 // D_k = max(|Y0_k|, |Y0_k + dY_k|) + 1e-12, dY <- dY - D B^T (B D B^T)^-1 B dY,
 // the correction of least D^-1-weighted norm, so species near zero hardly move
 // and sum_k dY_k = 0 follows from element conservation.
-// One wavefront per row, lanes over species: the E x E Gram matrix B D B^T and
-// B dY are wavefront sums; every lane then solves the (symmetric positive
-// definite) system by elimination; an element absent from the mechanism's
-// species has a zero row and gets lambda = 0.
-constexpr int kMaxK = 128, kMaxE = 8, kSlots = kMaxK / 64;
+//
+// A wavefront takes 32 rows, two lanes per row, each with every other species:
+// the E x E Gram matrix B D B^T and B dY are sums in the lane's registers, the
+// two halves are added once, and each lane solves its row's (symmetric positive
+// definite) system by elimination (an element absent from the mechanism's
+// species has a zero row and gets lambda = 0).  Rows of y0 and of the output go
+// through LDS, so HBM sees whole lines; the network output is FP32, so the
+// decode is too (sinhf), the increments and the projection are FP64.  (One row
+// per wavefront with E (E + 3) / 2 wavefront sums and the elimination repeated
+// by all 64 lanes took 217 us per 65,536 gri30 rows; this takes 65, of which the
+// 90 MB of rows are 18 at a copy's rate and the rest the FP64 sums and sinhf at
+// a few wavefronts per SIMD.)
+constexpr int kMaxK = 128, kMaxE = 8, kApplyRows = 32;
+template <int EM>   // elements, padded with zero rows
 __global__ __launch_bounds__(64) void apply_kernel(int rows, int N, int K, const double* __restrict__ y0,
                                                    const float* __restrict__ out, const double* __restrict__ norm,
                                                    int in_p, int out_p, const double* __restrict__ comp,
                                                    const double* __restrict__ rmw, int E, double* __restrict__ y1) {
-    const int r = blockIdx.x;
-    if (r >= rows) return;
-    const int lane = threadIdx.x;
-    const double* mu = norm + 2 * in_p;
-    const double* sd = mu + out_p;
-    const double* sc = sd + out_p;
-    const double* y0r = y0 + static_cast<size_t>(r) * N;
-    double* y1r = y1 + static_cast<size_t>(r) * N;
-    const float* o = out + static_cast<size_t>(r) * out_p;
-    // j = 0 (mass) and j = 1 (T)
-    if (lane == 0) y1r[0] = y0r[0];
-    // the network output is FP32, so the decode is too (sinhf); the increments
-    // and the projection below are FP64
-    if (lane == 1) y1r[1] = y0r[1] + sc[0] * static_cast<double>(sinhf(static_cast<float>(o[0] * sd[0] + mu[0])));
-    double dY[kSlots], D[kSlots];
-#pragma unroll
-    for (int t = 0; t < kSlots; t++) {
-        const int k = lane + 64 * t;
-        dY[t] = 0.0;
-        D[t] = 0.0;
-        if (k < K) {
-            dY[t] = sc[1 + k] * static_cast<double>(sinhf(static_cast<float>(o[1 + k] * sd[1 + k] + mu[1 + k])));
-            D[t] = fmax(fabs(y0r[2 + k]), fabs(y0r[2 + k] + dY[t])) + 1e-12;
-        }
-    }
+    extern __shared__ __attribute__((aligned(16))) double apply_lds[];
+    const int os = out_p + 1;                      // odd row stride
+    double* const ly = apply_lds;                  // rows of y0
+    double* const lB = ly + kApplyRows * N;        // B_ek, species-major, EM each
+    double* const ld = lB + EM * K;                // mu, sd, sc of each output
+    float* const lo = reinterpret_cast<float*>(ld + 3 * (K + 1));
+    const int lane = threadIdx.x, half = lane / kApplyRows;
+    const int r0 = blockIdx.x * kApplyRows, nr = min(kApplyRows, rows - r0);
     const bool project = comp && E >= 1 && E <= kMaxE;
-    double lam[kMaxE];
+    // everything through LDS, 8 loads per lane in flight
+    auto stage = [&](int count, auto&& load, auto&& store) {
+        for (int i = lane; i < count; i += 8 * 64) {
+            decltype(load(0)) v[8];
 #pragma unroll
-    for (int a = 0; a < kMaxE; a++) lam[a] = 0.0;
-    // B_ek of the lane's species
-    double Bk[kSlots][kMaxE];
+            for (int b = 0; b < 8; b++) v[b] = load(min(i + 64 * b, count - 1));
 #pragma unroll
-    for (int t = 0; t < kSlots; t++) {
-        const int k = lane + 64 * t;
+            for (int b = 0; b < 8; b++)
+                if (i + 64 * b < count) store(i + 64 * b, v[b]);
+        }
+    };
+    const double* yr = y0 + static_cast<size_t>(r0) * N;
+    const float* orow = out + static_cast<size_t>(r0) * out_p;
+    stage(nr * N, [&](int i) { return yr[i]; }, [&](int i, double v) { ly[i] = v; });
+    stage(nr * out_p, [&](int i) { return orow[i]; },
+          [&](int i, float v) { lo[i / out_p * os + i % out_p] = v; });
+    const double* par = norm + 2 * in_p;           // mu, sd, sc
+    stage(3 * (K + 1), [&](int i) { return par[(i % 3) * out_p + i / 3]; }, [&](int i, double v) { ld[i] = v; });
+    if (project)
+        stage(K * EM, [&](int i) { return i % EM < E ? comp[i / EM * E + i % EM] * rmw[i / EM] : 0.0; },
+              [&](int i, double v) { lB[i] = v; });
+    __syncthreads();
+    const int row = min(lane % kApplyRows, nr - 1);   // spare lanes repeat the last row
+    double* const y = ly + row * N;
+    float* const o = lo + row * os;
+    double G[EM][EM + 1];
 #pragma unroll
-        for (int a = 0; a < kMaxE; a++) Bk[t][a] = (project && k < K && a < E) ? comp[k * E + a] * rmw[k] : 0.0;
+    for (int a = 0; a < EM; a++)
+#pragma unroll
+        for (int b = 0; b <= EM; b++) G[a][b] = 0.0;
+    // output j = 0 is T, 1 + k species k; half 0 takes the even ones
+    for (int j = half; j <= K; j += 2) {
+        const float sh = sinhf(static_cast<float>(o[j] * ld[3 * j + 1] + ld[3 * j]));
+        o[j] = sh;
+        if (j == 0 || !project) continue;
+        const int k = j - 1;
+        const double dY = ld[3 * j + 2] * static_cast<double>(sh);
+        const double D = fmax(fabs(y[2 + k]), fabs(y[2 + k] + dY)) + 1e-12;
+        double B[EM];
+#pragma unroll
+        for (int a = 0; a < EM; a++) B[a] = lB[k * EM + a];
+#pragma unroll
+        for (int a = 0; a < EM; a++) {
+            const double bd = B[a] * D;
+#pragma unroll
+            for (int b = a; b < EM; b++) G[a][b] += bd * B[b];
+            G[a][EM] += B[a] * dY;
+        }
     }
+    double lam[EM];
+#pragma unroll
+    for (int a = 0; a < EM; a++) lam[a] = 0.0;
     if (project) {
-        double G[kMaxE][kMaxE + 1];
 #pragma unroll
-        for (int a = 0; a < kMaxE; a++) {
+        for (int a = 0; a < EM; a++)
 #pragma unroll
-            for (int b = 0; b <= kMaxE; b++) G[a][b] = 0.0;
-        }
-#pragma unroll
-        for (int a = 0; a < kMaxE; a++) {
-            if (a >= E) continue;
-#pragma unroll
-            for (int b = a; b < kMaxE; b++) {
-                if (b >= E) continue;
-                double part = 0.0;
-#pragma unroll
-                for (int t = 0; t < kSlots; t++) part += Bk[t][a] * D[t] * Bk[t][b];
-                G[a][b] = G[b][a] = wave_sum(part);
+            for (int b = a; b <= EM; b++) {
+                G[a][b] += __shfl_xor(G[a][b], kApplyRows);
+                if (b < EM) G[b][a] = G[a][b];
             }
-            double v = 0.0;
-#pragma unroll
-            for (int t = 0; t < kSlots; t++) v += Bk[t][a] * dY[t];
-            G[a][kMaxE] = wave_sum(v);
-        }
         // elimination without pivoting (SPD); zero rows give lambda = 0
-        bool live[kMaxE];
-        double rp[kMaxE];
+        double rp[EM];
 #pragma unroll
-        for (int c = 0; c < kMaxE; c++) {
-            live[c] = c < E && G[c][c] > 1e-300;
-            rp[c] = live[c] ? 1.0 / G[c][c] : 0.0;
-            if (!live[c]) continue;
+        for (int c = 0; c < EM; c++) {
+            rp[c] = G[c][c] > 1e-300 ? 1.0 / G[c][c] : 0.0;
 #pragma unroll
-            for (int a = c + 1; a < kMaxE; a++) {
-                if (a >= E) continue;
+            for (int a = c + 1; a < EM; a++) {
                 const double f = G[a][c] * rp[c];
 #pragma unroll
-                for (int b = c; b <= kMaxE; b++)
-                    if (b < E || b == kMaxE) G[a][b] -= f * G[c][b];
+                for (int b = c; b <= EM; b++) G[a][b] -= f * G[c][b];
             }
         }
 #pragma unroll
-        for (int c = kMaxE - 1; c >= 0; c--) {
-            if (!live[c]) continue;
-            double v = G[c][kMaxE];
+        for (int c = EM - 1; c >= 0; c--) {
+            double v = G[c][EM];
 #pragma unroll
-            for (int b = c + 1; b < kMaxE; b++)
-                if (b < E) v -= G[c][b] * lam[b];
+            for (int b = c + 1; b < EM; b++) v -= G[c][b] * lam[b];
             lam[c] = v * rp[c];
         }
     }
+    __syncthreads();   // the spare lanes have read the last row
+    if (lane % kApplyRows < nr)
+        for (int j = half; j <= K; j += 2) {
+            const double d = ld[3 * j + 2] * static_cast<double>(o[j]);
+            if (j == 0) {
+                y[1] += d;
+                continue;
+            }
+            const int k = j - 1;
+            double c = 0.0;
+            if (project) {
 #pragma unroll
-    for (int t = 0; t < kSlots; t++) {
-        const int k = lane + 64 * t;
-        if (k >= K) continue;
-        double c = 0.0;
-#pragma unroll
-        for (int a = 0; a < kMaxE; a++) c += Bk[t][a] * lam[a];
-        y1r[2 + k] = y0r[2 + k] + (dY[t] - D[t] * c);
-    }
+                for (int a = 0; a < EM; a++) c += lB[k * EM + a] * lam[a];
+            }
+            const double D = fmax(fabs(y[2 + k]), fabs(y[2 + k] + d)) + 1e-12;
+            y[2 + k] += d - D * c;
+        }
+    __syncthreads();
+    double* const yo = y1 + static_cast<size_t>(r0) * N;
+    for (int i = lane; i < nr * N; i += 64) yo[i] = ly[i];
+}
+
+void launch_apply(int rows, int N, int K, const double* y0, const float* out, const double* norm, int in_p, int out_p,
+                  const double* comp, const double* rmw, int E, double* y1, hipStream_t st) {
+    const int em = E <= 5 ? 5 : kMaxE;
+    const size_t lds = static_cast<size_t>(kApplyRows * N + em * K + 3 * (K + 1)) * sizeof(double) +
+                       static_cast<size_t>(kApplyRows) * (out_p + 1) * sizeof(float);
+    const dim3 grid((rows + kApplyRows - 1) / kApplyRows);
+    if (em == 5)
+        hipLaunchKernelGGL(apply_kernel<5>, grid, dim3(64), lds, st, rows, N, K, y0, out, norm, in_p, out_p, comp, rmw,
+                           E, y1);
+    else
+        hipLaunchKernelGGL(apply_kernel<kMaxE>, grid, dim3(64), lds, st, rows, N, K, y0, out, norm, in_p, out_p, comp, rmw,
+                           E, y1);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) throw std::runtime_error(std::string("surrogate apply: ") + hipGetErrorString(e));
 }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -460,6 +510,149 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16(int M, int N, int K, const u
                     e.zf[o] = v + e.bias[n];
                 }
             }
+}
+
+// Inference in one kernel: features, hidden layers and output layer for 64 rows
+// per workgroup, with the activations (BF16) in LDS from layer to layer.
+//
+// Layer by layer through HBM, a 65,536 x 256 layer moved 100 MB for 8.6 GFLOP
+// (50 us with its epilogue).  Here HBM sees the states once and the FP32
+// outputs; the weights (450 KB for 55 -> 4 x 256 -> 54) are read by every
+// workgroup through L2, each element by one wavefront only, straight into the
+// B operand's lanes (16 bytes per lane and 16 x 32 tile), four k-steps ahead.
+// Wavefront w computes columns 16 HT w .. of all rows: 4 x HT tiles of
+// v_mfma_f32_16x16x32_bf16 (layouts as gemm_nt_bf16).  A layer's results stay
+// in the accumulators until every wavefront has read its input, then replace it.
+// hidden = 64 HT <= 256: 128 rows would need 128 accumulator registers and
+// spill.  65,536 rows of the net above: 109 us against 255 us layer by layer
+// (30 GFLOP: 26 us at a large product's rate); what is left over that is GELU,
+// the FP64 logarithms of the features and the waits between layers.
+struct MlpArgs {
+    int rows, N, K, in_p, out_p, depth;
+    const double* y;
+    const double* P;
+    const double* norm;
+    const uint16_t* W;     // BF16 weights
+    const float* par;      // FP32 parameters (biases)
+    float* out;            // rows x out_p
+    int oW[17], oB[17];
+};
+
+constexpr int kMlpRows = 64;
+
+// KC k-steps of weights at a time, the next KC loaded while these are multiplied
+template <int NT, int KC>
+__device__ __forceinline__ void mlp_steps(const uint16_t* __restrict__ act, int ls, const uint16_t* __restrict__ W,
+                                          int fi, int n0, f32x4 (&acc)[kMlpRows / 16][NT]) {
+    const int lane = threadIdx.x & 63, lr = lane & 15, ko = 8 * (lane >> 4);
+    const uint16_t* w = W + static_cast<size_t>(n0 + lr) * fi + ko;
+    bf16x8 b[KC][NT];
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) b[c][j] = *reinterpret_cast<const bf16x8*>(w + static_cast<size_t>(16 * j) * fi + 32 * c);
+    for (int k0 = 0; k0 < fi; k0 += 32 * KC) {
+        bf16x8 nb[KC][NT];
+        const int kn = min(k0 + 32 * KC, fi - 32 * KC);
+#pragma unroll
+        for (int c = 0; c < KC; c++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                nb[c][j] = *reinterpret_cast<const bf16x8*>(w + static_cast<size_t>(16 * j) * fi + kn + 32 * c);
+#pragma unroll
+        for (int c = 0; c < KC; c++)
+#pragma unroll
+            for (int i = 0; i < kMlpRows / 16; i++) {
+                const bf16x8 a = *reinterpret_cast<const bf16x8*>(act + (16 * i + lr) * ls + k0 + 32 * c + ko);
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[c][j], acc[i][j], 0, 0, 0);
+            }
+#pragma unroll
+        for (int c = 0; c < KC; c++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) b[c][j] = nb[c][j];
+    }
+}
+
+template <int NT>
+__device__ __forceinline__ void mlp_layer(const uint16_t* __restrict__ act, int ls, const uint16_t* __restrict__ W,
+                                          int fi, int n0, f32x4 (&acc)[kMlpRows / 16][NT]) {
+#pragma unroll
+    for (int i = 0; i < kMlpRows / 16; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (fi % 128 == 0) mlp_steps<NT, 4>(act, ls, W, fi, n0, acc);
+    else mlp_steps<NT, 2>(act, ls, W, fi, n0, acc);   // a multiple of 64
+}
+
+template <int HT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mlp_kernel(MlpArgs g) {
+    extern __shared__ __attribute__((aligned(16))) double apply_lds[];
+    uint16_t* const act = reinterpret_cast<uint16_t*>(apply_lds);
+    constexpr int H = 64 * HT;
+    const int ls = max(H, g.in_p) + 8;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, lr = lane & 15, lq = lane >> 4;
+    const int r0 = blockIdx.x * kMlpRows;
+    // features (see features_kernel): column c of a state gives feature 0 (T,
+    // c = 1), 1 (ln P, in the place of the mass) or c; rows past the end repeat
+    // the last one
+    const int total = kMlpRows * g.N;
+    for (int e0 = t; e0 < total; e0 += 4 * 256) {
+        double x[4];
+        int row[4], col[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const int e = min(e0 + 256 * b, total - 1);
+            row[b] = e / g.N;
+            const int c = e - row[b] * g.N;
+            col[b] = c < 2 ? 1 - c : c;
+            const size_t s = static_cast<size_t>(min(r0 + row[b], g.rows - 1));
+            x[b] = c == 0 ? g.P[s] : g.y[s * g.N + c];
+        }
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const double lx = log(col[b] == 1 ? x[b] : fmax(x[b], 1e-30));
+            const double f = col[b] == 0 ? x[b] : lx;
+            const double z = (f - g.norm[col[b]]) / g.norm[g.in_p + col[b]];
+            act[row[b] * ls + col[b]] = f2bf(static_cast<float>(fmin(fmax(z, -8.0), 8.0)));
+        }
+    }
+    for (int i = t; i < kMlpRows * (g.in_p - g.N); i += 256) {
+        const int r = i / (g.in_p - g.N), c = i - r * (g.in_p - g.N);
+        act[r * ls + g.N + c] = 0;
+    }
+    __syncthreads();
+    for (int l = 0; l < g.depth; l++) {
+        f32x4 acc[kMlpRows / 16][HT];
+        const int n0 = 16 * HT * w;
+        mlp_layer<HT>(act, ls, g.W + g.oW[l], l == 0 ? g.in_p : H, n0, acc);
+        const float* bias = g.par + g.oB[l] + n0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < HT; j++) {
+            const float bj = bias[16 * j + lr];
+#pragma unroll
+            for (int i = 0; i < kMlpRows / 16; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    act[(16 * i + 4 * lq + r) * ls + n0 + 16 * j + lr] = f2bf(gelu(acc[i][j][r] + bj));
+        }
+        __syncthreads();
+    }
+    for (int c = 0; c < g.out_p; c += 64) {   // output layer, 16 columns per wavefront
+        f32x4 acc[kMlpRows / 16][1];
+        const int n0 = c + 16 * w;
+        mlp_layer<1>(act, ls, g.W + g.oW[g.depth], H, n0, acc);
+        const float bj = g.par[g.oB[g.depth] + n0 + lr];
+#pragma unroll
+        for (int i = 0; i < kMlpRows / 16; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = r0 + 16 * i + 4 * lq + r;
+                if (row < g.rows) g.out[static_cast<size_t>(row) * g.out_p + n0 + lr] = acc[i][0][r] + bj;
+            }
+    }
 }
 
 void check(hipError_t e, const char* what) {
@@ -742,19 +935,46 @@ double SurrogateNet::loss_grad(long n, const double* y0, const double* P, const 
     return loss;
 }
 
+// The fused kernel for hidden widths of 64, 128, 192 and 256 (weights 16-byte
+// aligned: every width and offset is a multiple of 8 elements); false: not taken.
+bool SurrogateNet::infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t st) const {
+    if (s_.hidden % 64 || s_.hidden > 256 || reinterpret_cast<uintptr_t>(wb_) % 16) return false;
+    MlpArgs g{};
+    g.rows = rows; g.N = s_.K + 2; g.K = s_.K; g.in_p = s_.in_p; g.out_p = s_.out_p; g.depth = s_.depth;
+    g.y = y0; g.P = P; g.norm = norm_; g.W = wb_; g.par = par_; g.out = out;
+    for (int l = 0; l <= s_.depth; l++) {
+        g.oW[l] = static_cast<int>(oW_[l]);
+        g.oB[l] = static_cast<int>(oB_[l]);
+    }
+    const size_t lds = static_cast<size_t>(kMlpRows) * (std::max(s_.hidden, s_.in_p) + 8) * 2;
+    const void* kp = nullptr;
+    switch (s_.hidden / 64) {
+        case 1: kp = reinterpret_cast<const void*>(&mlp_kernel<1>); break;
+        case 2: kp = reinterpret_cast<const void*>(&mlp_kernel<2>); break;
+        case 3: kp = reinterpret_cast<const void*>(&mlp_kernel<3>); break;
+        default: kp = reinterpret_cast<const void*>(&mlp_kernel<4>);
+    }
+    if (lds > 65536)
+        check(hipFuncSetAttribute(kp, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
+              "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
+    void* args[] = {&g};
+    check(hipLaunchKernel(kp, dim3((rows + kMlpRows - 1) / kMlpRows), dim3(256), args, lds, st), "surrogate MLP launch");
+    return true;
+}
+
 void SurrogateNet::predict(long n, const double* y0, const double* P, double* y1, hipStream_t st) {
     const int N = s_.K + 2;
     const long chunk = 65536;
     for (long c0 = 0; c0 < n; c0 += chunk) {
         const int rows = static_cast<int>(std::min(chunk, n - c0));
         ensure_batch(rows);
-        hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0 + c0 * N, P + c0,
-                           norm_, s_.in_p, act_);
-        check(hipGetLastError(), "surrogate features");
-        forward(rows, st);
-        hipLaunchKernelGGL(apply_kernel, dim3(rows), dim3(64), 0, st, rows, N, s_.K, y0 + c0 * N, out_, norm_,
-                           s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N);
-        check(hipGetLastError(), "surrogate apply");
+        if (!infer_fused(rows, y0 + c0 * N, P + c0, out_, st)) {
+            hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0 + c0 * N,
+                               P + c0, norm_, s_.in_p, act_);
+            check(hipGetLastError(), "surrogate features");
+            forward(rows, st);
+        }
+        launch_apply(rows, N, s_.K, y0 + c0 * N, out_, norm_, s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N, st);
     }
 }
 
@@ -812,12 +1032,15 @@ void SurrogateNet::predict_noalloc(long n, const double* y0, const double* P, do
     const int N = s_.K + 2;
     for (long c0 = 0; c0 < n; c0 += R) {
         const int rows = static_cast<int>(std::min<long>(R, n - c0));
-        hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0 + c0 * N, P + c0,
-                           norm_, s_.in_p, feat);
-        check(hipGetLastError(), "surrogate features");
+        const bool fused = infer_fused(rows, y0 + c0 * N, P + c0, out, st);
+        if (!fused) {
+            hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0 + c0 * N,
+                               P + c0, norm_, s_.in_p, feat);
+            check(hipGetLastError(), "surrogate features");
+        }
         const uint16_t* H = feat;
         uint16_t* next = ha;
-        for (int l = 0; l <= s_.depth; l++) {
+        for (int l = 0; !fused && l <= s_.depth; l++) {
             const int fi = s_.fan_in(l), fo = s_.fan_out(l);
             EpiArgs e{};
             e.bias = par_ + oB_[l];
@@ -833,9 +1056,7 @@ void SurrogateNet::predict_noalloc(long n, const double* y0, const double* P, do
                 gemm<false, false, kFwdLinear>(rows, fo, fi, H, fi, wb_ + oW_[l], fi, e, st);
             }
         }
-        hipLaunchKernelGGL(apply_kernel, dim3(rows), dim3(64), 0, st, rows, N, s_.K, y0 + c0 * N, out, norm_,
-                           s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N);
-        check(hipGetLastError(), "surrogate apply");
+        launch_apply(rows, N, s_.K, y0 + c0 * N, out, norm_, s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N, st);
     }
 }
 

@@ -76,6 +76,7 @@ public:
 private:
     void ensure_batch(int rows);
     void forward(int rows, hipStream_t stream);
+    bool infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t stream) const;
     double backward_and_loss(int rows, bool update, double lr, hipStream_t stream);
     void sync_bf16(hipStream_t stream);
 

@@ -1,0 +1,70 @@
+"""Surrogate.predict at the edges of its row tiles and at widths on either side
+of the fused kernel's range (a multiple of 64 up to 256; 48 and 320 go layer by
+layer), against a float64 numpy restatement that rounds to BF16 where the
+device does.
+
+An activation within FP32 summation error of a BF16 rounding boundary may round
+the other way: 2^-8 of one of `hidden` inputs of the next layer.  With a few of
+them per row, |h| <= 2 and |w| <= 1 / sqrt(hidden) <= 1 / 6.9, an output moves by
+less than 4e-3; the increments follow through sinh, and the projection does not
+enlarge an error in its own norm (factor 2: its weights depend on the
+increments)."""
+import numpy as np
+import pytest
+
+from conftest import mech_file
+from test_gpu_surrogate import bf16, gelu, pad, synthetic_pairs
+
+pytestmark = pytest.mark.gpu
+
+
+def network_output(params, norm, K, hidden, depth, y0, P):
+    ip, op = pad(K + 2), pad(K + 1)
+    f = np.zeros((len(y0), ip))
+    f[:, 0] = y0[:, 1]
+    f[:, 1] = np.log(P)
+    f[:, 2:K + 2] = np.log(np.maximum(y0[:, 2:], 1e-30))
+    z = np.clip((f - norm[:ip]) / norm[ip:2 * ip], -8, 8)
+    z[:, K + 2:] = 0
+    h, off = bf16(z).astype(np.float64), 0
+    widths = [ip] + [hidden] * depth + [op]
+    for l in range(depth + 1):
+        fi, fo = widths[l], widths[l + 1]
+        W = bf16(params[off:off + fo * fi]).astype(np.float64).reshape(fo, fi)
+        v = (h @ W.T).astype(np.float32) + params[off + fo * fi:off + fo * fi + fo]
+        off += fo * fi + fo
+        h = bf16(gelu(v)).astype(np.float64) if l < depth else v
+    return h[:, :K + 1].astype(np.float64)
+
+
+@pytest.mark.parametrize("mech,hidden,depth,rows", [
+    ("h2o2", 64, 1, 1), ("h2o2", 48, 2, 33), ("h2o2", 128, 2, 64), ("gri30", 192, 3, 65),
+    ("gri30", 256, 4, 31), ("gri30", 256, 1, 129), ("gri30", 320, 2, 97), ("nDodecane", 64, 2, 1000)])
+def test_predict_matches_reference(mech, hidden, depth, rows):
+    import cantera_amd as ca
+    from cantera_amd.surrogate import Surrogate
+    from cantera_amd.workloads import MechInfo
+    info = MechInfo(mech_file(mech))
+    sol = ca.Solution(mech)
+    K = sol.n_species
+    sur = Surrogate(sol, dt=1e-6, hidden=hidden, depth=depth, seed=hidden + depth)
+    y0, P, y1 = synthetic_pairs(info, max(rows, 256), 11)
+    sur.fit_normalization(y0, P, y1)
+    y0, P = y0[:rows], P[:rows]
+    norm = sur.normalization
+    ip, op = pad(K + 2), pad(K + 1)
+    mu, sd, sc = (norm[2 * ip + i * op:2 * ip + i * op + K + 1] for i in range(3))
+    arg = network_output(sur.params, norm, K, hidden, depth, y0, P) * sd + mu
+    d, tol = sc * np.sinh(arg), sc * np.cosh(arg) * sd * 4e-3
+    got = sur.predict(y0, P)
+    assert np.array_equal(got[:, 0], y0[:, 0])
+    # a rounding of T1 itself on top of the network's tolerance
+    assert np.all(np.abs(got[:, 1] - (y0[:, 1] + d[:, 0])) <= tol[:, 0] + 1e-12 * y0[:, 1])
+    B = info.composition / info.molecular_weights[:, None]
+    B = B[:, B.any(axis=0)]
+    for r in range(rows):
+        dY = d[r, 1:]
+        D = np.maximum(np.abs(y0[r, 2:]), np.abs(y0[r, 2:] + dY)) + 1e-12
+        lam = np.linalg.solve(B.T @ (B * D[:, None]), B.T @ dY)
+        e = got[r, 2:] - (y0[r, 2:] + dY - D * (B @ lam))
+        assert np.linalg.norm(e / np.sqrt(D)) <= 2 * np.linalg.norm(tol[r, 1:] / np.sqrt(D)) + 1e-12
