@@ -50,11 +50,11 @@ __device__ __forceinline__ float gelu_grad(float z) {
     return fmaf(z * (tr * g.r), fmaf(z * z, 3.0f * kGelu3, kGelu1), z >= 0.0f ? g.r : tr);
 }
 
-enum Epi { kFwdGelu = 0, kFwdLinear = 1, kStoreF32 = 2, kBwdGelu = 3 };
+enum Epi { kFwdGelu, kFwdLinear, kBwdGelu };
 
 struct EpiArgs {
     const float* bias;   // kFwdGelu / kFwdLinear: [N]
-    float* zf;           // kFwdGelu: pre-activation out; kFwdLinear / kStoreF32: fp32 out
+    float* zf;           // kFwdGelu: pre-activation out; kFwdLinear: fp32 out
     uint16_t* hb;        // kFwdGelu: gelu(z) as bf16; kBwdGelu: acc * gelu'(zin) as bf16
     const float* zin;    // kBwdGelu: pre-activation of the layer below
     int ldc;
@@ -63,15 +63,15 @@ struct EpiArgs {
 constexpr int kTM = 64, kTN = 64, kTK = 32, kLdsK = kTK + 8;
 
 // C(m, n) = sum_k A(m, k) B(n, k) over BF16 operands, FP32 accumulation.
-// A(m, k) = TA ? A[k * lda + m] : A[m * lda + k];  B(n, k) = TB ? B[k * ldb + n] : B[n * ldb + k].
+// A(m, k) = A[m * K + k];  B(n, k) = B[n * K + k], for kBwdGelu B[k * N + n].
+// Any size: the layers that gemm_direct and gemm_nt_bf16 do not take.
 // 256 threads: a 64 x 64 tile of C per workgroup, 32 x 32 per wavefront as
 // 2 x 2 MFMA 16x16x16 tiles; K staged through LDS in steps of 32.  Out-of-range
 // rows / columns / k read as zero and are not stored.
-// kStoreF32 may split K over gridDim.z (chunks of kchunk, a multiple of kTK):
-// each split adds its partial sums to the cleared output with FP32 atomics.
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void gemm_bf16(int M, int N, int K, const uint16_t* __restrict__ A, int lda,
-                                                 const uint16_t* __restrict__ B, int ldb, EpiArgs e, int kchunk) {
+template <int EPI>
+__global__ __launch_bounds__(256) void gemm_bf16(int M, int N, int K, const uint16_t* __restrict__ A,
+                                                 const uint16_t* __restrict__ B, EpiArgs e) {
+    constexpr bool TB = EPI == kBwdGelu;
     __shared__ uint16_t As[kTM][kLdsK];
     __shared__ uint16_t Bs[kTN][kLdsK];
     const int t = threadIdx.x;
@@ -83,24 +83,15 @@ __global__ __launch_bounds__(256) void gemm_bf16(int M, int N, int K, const uint
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kbeg = blockIdx.z * kchunk, kend = min(K, kbeg + kchunk);
-    for (int k0 = kbeg; k0 < kend; k0 += kTK) {
+    for (int k0 = 0; k0 < K; k0 += kTK) {
         // stage A (64 x 32) and B (64 x 32), 8 elements per thread each
-        if (!TA) {
+        {
             const int r = t >> 2, kk = (t & 3) * 8;
             const int m = m0 + r;
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 const int k = k0 + kk + q;
-                As[r][kk + q] = (m < M && k < K) ? A[static_cast<size_t>(m) * lda + k] : 0;
-            }
-        } else {
-            const int kk = t >> 3, rr = (t & 7) * 8;
-            const int k = k0 + kk;
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const int m = m0 + rr + q;
-                As[rr + q][kk] = (m < M && k < K) ? A[static_cast<size_t>(k) * lda + m] : 0;
+                As[r][kk + q] = (m < M && k < K) ? A[static_cast<size_t>(m) * K + k] : 0;
             }
         }
         if (!TB) {
@@ -109,7 +100,7 @@ __global__ __launch_bounds__(256) void gemm_bf16(int M, int N, int K, const uint
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 const int k = k0 + kk + q;
-                Bs[r][kk + q] = (n < N && k < K) ? B[static_cast<size_t>(n) * ldb + k] : 0;
+                Bs[r][kk + q] = (n < N && k < K) ? B[static_cast<size_t>(n) * K + k] : 0;
             }
         } else {
             const int kk = t >> 3, rr = (t & 7) * 8;
@@ -117,7 +108,7 @@ __global__ __launch_bounds__(256) void gemm_bf16(int M, int N, int K, const uint
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 const int n = n0 + rr + q;
-                Bs[rr + q][kk] = (n < N && k < K) ? B[static_cast<size_t>(k) * ldb + n] : 0;
+                Bs[rr + q][kk] = (n < N && k < K) ? B[static_cast<size_t>(k) * N + n] : 0;
             }
         }
         __syncthreads();
@@ -159,9 +150,6 @@ __global__ __launch_bounds__(256) void gemm_bf16(int M, int N, int K, const uint
                     e.hb[o] = f2bf(gelu(z));
                 } else if (EPI == kFwdLinear) {
                     e.zf[o] = v + e.bias[n];
-                } else if (EPI == kStoreF32) {
-                    if (gridDim.z > 1) atomicAdd(&e.zf[o], v);
-                    else e.zf[o] = v;
                 } else {
                     e.hb[o] = f2bf(v * gelu_grad(e.zin[o]));
                 }
@@ -191,40 +179,31 @@ __global__ void features_kernel(int rows, const int* __restrict__ idx, int N, in
     }
 }
 
-// Targets: the increments d = (T1 - T0, Y1_k - Y0_k), compressed as asinh(d / s)
-// (linear below the scale s, logarithmic above, so small and large increments
-// get comparable relative accuracy), then standardised.
-__global__ void targets_kernel(int rows, const int* __restrict__ idx, int N, int K, const double* __restrict__ y0,
-                               const double* __restrict__ y1, const double* __restrict__ norm, int in_p, int out_p,
-                               float* __restrict__ T) {
-    const int r = blockIdx.x;
-    if (r >= rows) return;
-    const long s = idx ? idx[r] : r;
-    const double* mu = norm + 2 * in_p;
-    const double* sd = mu + out_p;
-    const double* sc = sd + out_p;
-    for (int j = threadIdx.x; j < out_p; j += blockDim.x) {
-        float v = 0.f;
-        if (j <= K) {
-            const double d = y1[s * N + 1 + j] - y0[s * N + 1 + j];
-            v = static_cast<float>((asinh(d / sc[j]) - mu[j]) / sd[j]);
-        }
-        T[static_cast<size_t>(r) * out_p + j] = v;
-    }
-}
-
-// Mean-squared error over the n_out valid outputs; gradient as BF16 operand.
-__global__ void loss_kernel(int rows, int n_out, int out_p, const float* __restrict__ out,
-                            const float* __restrict__ tgt, uint16_t* __restrict__ g, double* __restrict__ loss) {
+// Mean-squared error over the n_out valid outputs, gradient as BF16 operand.
+// Targets are the increments d = (T1 - T0, Y1_k - Y0_k), compressed as
+// asinh(d / s) (linear below the scale s, logarithmic above, so small and large
+// increments get comparable relative accuracy), then standardised.  Each block
+// leaves its part of the loss in loss[1 + block]; grad_sum_kernel adds them.
+constexpr int kLossBlocks = 256;
+__global__ __launch_bounds__(256) void loss_kernel(int rows, const int* __restrict__ idx, int N, int n_out, int in_p,
+                                                   int out_p, const double* __restrict__ y0,
+                                                   const double* __restrict__ y1, const double* __restrict__ norm,
+                                                   const float* __restrict__ out, uint16_t* __restrict__ g,
+                                                   double* __restrict__ loss) {
     __shared__ double part[256];
     double acc = 0.0;
     const double scale = 1.0 / (static_cast<double>(rows) * n_out);
+    const double* mu = norm + 2 * in_p;
+    const double* sd = mu + out_p;
+    const double* sc = sd + out_p;
     const size_t total = static_cast<size_t>(rows) * out_p;
     for (size_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += static_cast<size_t>(gridDim.x) * blockDim.x) {
         const int j = static_cast<int>(i % out_p);
         float gv = 0.f;
         if (j < n_out) {
-            const float d = out[i] - tgt[i];
+            const size_t r = i / out_p, e = (idx ? idx[r] : r) * N + 1 + j;
+            const float tgt = static_cast<float>((asinh((y1[e] - y0[e]) / sc[j]) - mu[j]) / sd[j]);
+            const float d = out[i] - tgt;
             acc += static_cast<double>(d) * d;
             gv = static_cast<float>(2.0 * scale) * d;
         }
@@ -236,26 +215,7 @@ __global__ void loss_kernel(int rows, int n_out, int out_p, const float* __restr
         if (threadIdx.x < s) part[threadIdx.x] += part[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(loss, part[0] * scale);
-}
-
-// Column sums of a BF16 gradient operand: bias gradient.
-// db[c] += sum over a block of 64 rows of g[r][c] (db cleared by the caller):
-// 256 threads as 4 row groups x 64 columns, coalesced 128-byte row segments,
-// partial sums combined in LDS and added with one atomic per column and block.
-constexpr int kColsumRows = 64;
-__global__ __launch_bounds__(256) void colsum_kernel(int rows, int cols, const uint16_t* __restrict__ g,
-                                                     float* __restrict__ db) {
-    __shared__ float part[4][64];
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int rg = threadIdx.x >> 6;
-    const int r0 = blockIdx.y * kColsumRows;
-    float s = 0.f;
-    if (c < cols)
-        for (int r = r0 + rg; r < min(rows, r0 + kColsumRows); r += 4) s += bf2f(g[static_cast<size_t>(r) * cols + c]);
-    part[rg][threadIdx.x & 63] = s;
-    __syncthreads();
-    if (rg == 0 && c < cols) atomicAdd(&db[c], (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]));
+    if (threadIdx.x == 0) loss[1 + blockIdx.x] = part[0] * scale;
 }
 
 // Adam (Kingma & Ba 2015) with bias correction, then the BF16 weight copy.
@@ -512,6 +472,220 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16(int M, int N, int K, const u
             }
 }
 
+// Four neighbouring columns of 8 rows of a row-major BF16 matrix as B operands
+// (or A operands of a transposed product): each lane loads its own 8 rows
+// (8 (lane / 16) ..) and columns (4 (lane % 16) ..), 8 bytes a row, and
+// transposes the 8 x 4 block in registers with 16 byte permutes, so no LDS is
+// needed.  Operand j then holds the columns 4 (lane % 16) + j of the tile.
+struct Rows8 { uint2 r[8]; };
+__device__ __forceinline__ bf16x8 column(const Rows8& v, int j) {
+    union { uint32_t u[4]; bf16x8 b; } o;
+    const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        o.u[q] = j < 2 ? __builtin_amdgcn_perm(v.r[2 * q + 1].x, v.r[2 * q].x, sel)
+                       : __builtin_amdgcn_perm(v.r[2 * q + 1].y, v.r[2 * q].y, sel);
+    return o.b;
+}
+
+// Training's products over one batch, C = A B^T (kBwdGelu: A B): a 64 x 64 tile
+// per workgroup, 16 rows x 64 columns per wavefront, operands straight from
+// global memory into the MFMA lanes (layouts as above; column 4 (lane % 16) + j
+// in operand j, so that results are stored 4 columns at a time).  A 4,096-row
+// batch is 64 tiles of 128 x 128 for 256 CUs and only 8 k-steps long: one
+// memory latency per k-step (20 us per layer) against one per KC k-steps here,
+// all loads of the next KC in flight under the products of these (9 us forward
+// and 7 us backward, where a tile's k-major operand was read 2 bytes at a time).
+// Requires K % (32 KC) == 0, N % 16 == 0.
+template <int KC, int EPI>
+__global__ __launch_bounds__(256) void gemm_direct(int M, int N, int K, const uint16_t* __restrict__ A,
+                                                   const uint16_t* __restrict__ B, EpiArgs e) {
+    constexpr bool kTB = EPI == kBwdGelu;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+    const int m0 = blockIdx.x * 64 + 16 * w, n = blockIdx.y * 64 + 4 * lr;
+    if (m0 >= M) return;
+    const bool nok = n < N;
+    const int nc = nok ? n : 0;
+    const uint16_t* pa = A + static_cast<size_t>(min(m0 + lr, M - 1)) * K + 8 * lq;
+    const uint16_t* pb = kTB ? B + static_cast<size_t>(8 * lq) * N + nc : B + static_cast<size_t>(nc) * K + 8 * lq;
+    union Bk { Rows8 t; bf16x8 d[4]; };
+    auto load = [&](int k0, bf16x8 (&a)[KC], Bk (&b)[KC]) {
+#pragma unroll
+        for (int c = 0; c < KC; c++) {
+            const int k = k0 + 32 * c;
+            a[c] = *reinterpret_cast<const bf16x8*>(pa + k);
+            if constexpr (kTB) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) b[c].t.r[i] = *reinterpret_cast<const uint2*>(pb + static_cast<size_t>(k + i) * N);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) b[c].d[j] = *reinterpret_cast<const bf16x8*>(pb + static_cast<size_t>(j) * K + k);
+            }
+        }
+    };
+    bf16x8 a[KC];
+    Bk b[KC];
+    load(0, a, b);
+    float4 z[4];   // kBwdGelu: pre-activations; otherwise the bias
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if constexpr (kTB)
+            z[r] = *reinterpret_cast<const float4*>(e.zin + static_cast<size_t>(min(m0 + 4 * lq + r, M - 1)) * N + nc);
+        else
+            z[r] = *reinterpret_cast<const float4*>(e.bias + nc);
+    f32x4 acc[4] = {};
+    for (int k0 = 0; k0 < K; k0 += 32 * KC) {
+        bf16x8 an[KC];
+        Bk bn[KC];
+        load(min(k0 + 32 * KC, K - 32 * KC), an, bn);
+#pragma unroll
+        for (int c = 0; c < KC; c++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                bf16x8 bj;
+                if constexpr (kTB) bj = column(b[c].t, j);
+                else bj = b[c].d[j];
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], bj, acc[j], 0, 0, 0);
+            }
+#pragma unroll
+        for (int c = 0; c < KC; c++) { a[c] = an[c]; b[c] = bn[c]; }
+    }
+    if (!nok) return;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int m = m0 + 4 * lq + r;
+        if (m >= M) continue;
+        const size_t o = static_cast<size_t>(m) * N + n;
+        float v[4] = {acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+        const float zz[4] = {z[r].x, z[r].y, z[r].z, z[r].w};
+        union { uint16_t h[4]; uint2 u; } h;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (kTB) v[j] *= gelu_grad(zz[j]);
+            else v[j] += zz[j];
+            h.h[j] = f2bf(EPI == kFwdGelu ? gelu(v[j]) : v[j]);
+        }
+        if (!kTB && e.zf) *reinterpret_cast<float4*>(e.zf + o) = make_float4(v[0], v[1], v[2], v[3]);
+        if (EPI != kFwdLinear) *reinterpret_cast<uint2*>(e.hb + o) = h.u;
+    }
+}
+
+// Weight and bias gradients of every layer in one launch: dW = G^T H (fo x fi)
+// and the column sums of G, over the rows [chunk z, chunk (z + 1)) of the batch,
+// into split z's own copy of the parameters (grad_sum_kernel adds the copies).
+// A 64 x 64 tile of one layer per workgroup; its wavefronts take every fourth
+// 32 rows and are added through LDS.  Both operands are transposed in registers
+// (Rows8), the next 32 rows loaded while these are multiplied.  Bias: the
+// product with a column of ones, by the tiles of the first columns.
+// (Layer by layer with atomics onto cleared gradients this was 20 launches and
+// 160 us for 4,096 rows of 55 -> 4 x 256 -> 54, more than half of it 2-byte
+// loads, the rest clears and column sums; now 16 us and 6 for the sum.)
+constexpr int kGradTiles = 512;   // workgroups aimed at
+struct GradArgs {
+    int rows, chunk;
+    size_t n_par;
+    float* part;
+    int first[18];                     // first tile of each layer, and their number
+    int fo[17], fi[17];
+    size_t oW[17], oB[17];
+    const uint16_t* G[17];
+    const uint16_t* H[17];
+};
+__global__ __launch_bounds__(256) void wgrad_kernel(GradArgs g) {
+    __shared__ float sum[4][16][64];   // one row of tiles of each wavefront
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+    int l = 0;
+    while (static_cast<int>(blockIdx.x) >= g.first[l + 1]) l++;
+    const int fo = g.fo[l], fi = g.fi[l], tile = blockIdx.x - g.first[l], tn = (fi + 63) / 64;
+    const int m0 = tile / tn * 64, n0 = tile % tn * 64, m = m0 + 4 * lr, n = n0 + 4 * lr;
+    const uint16_t* pg = g.G[l] + (m < fo ? m : 0);
+    const uint16_t* ph = g.H[l] + (n < fi ? n : 0);
+    const int r0 = blockIdx.y * g.chunk, r1 = min(g.rows, r0 + g.chunk);
+    auto load = [&](int r, Rows8& a, Rows8& b) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int row = r + 8 * lq + i;
+            const size_t q = min(row, g.rows - 1);
+            a.r[i] = *reinterpret_cast<const uint2*>(pg + q * fo);
+            b.r[i] = *reinterpret_cast<const uint2*>(ph + q * fi);
+            if (row >= r1) a.r[i] = b.r[i] = make_uint2(0u, 0u);
+        }
+    };
+    f32x4 acc[4][4] = {}, bias[4] = {};
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; i++) ones[i] = static_cast<__bf16>(1.0f);
+    Rows8 a, b;
+    load(r0 + 32 * w, a, b);
+    for (int r = r0 + 32 * w; r < r1; r += 128) {
+        Rows8 an, bn;
+        load(r + 128, an, bn);
+        bf16x8 bj[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) bj[j] = column(b, j);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const bf16x8 ai = column(a, i);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ai, bj[j], acc[i][j], 0, 0, 0);
+            if (n0 == 0) bias[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ai, ones, bias[i], 0, 0, 0);
+        }
+        a = an;
+        b = bn;
+    }
+    float* const part = g.part + static_cast<size_t>(blockIdx.y) * g.n_par;
+    auto reduce = [&](const f32x4 (&v)[4], float (&o)[4]) {   // wavefront w: o[j] of register w
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) sum[w][4 * r + j][lane] = v[j][r];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            o[j] = (sum[0][4 * w + j][lane] + sum[1][4 * w + j][lane]) + (sum[2][4 * w + j][lane] + sum[3][4 * w + j][lane]);
+    };
+    // operand i, register r of row group lq is row 4 (4 lq + r) + i of the tile
+    const int mr = m0 + 4 * (4 * lq + w);
+    float o[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        reduce(acc[i], o);
+        if (mr < fo && n < fi)
+            *reinterpret_cast<float4*>(part + g.oW[l] + static_cast<size_t>(mr + i) * fi + n) =
+                make_float4(o[0], o[1], o[2], o[3]);
+    }
+    if (n0 == 0) {
+        reduce(bias, o);
+        if (mr < fo && lr == 0)
+            *reinterpret_cast<float4*>(part + g.oB[l] + mr) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+// grad = sum of the splits' copies in order, loss[0] = sum of the blocks' parts
+__global__ __launch_bounds__(256) void grad_sum_kernel(size_t n, int splits, const float* __restrict__ part,
+                                                       float* __restrict__ grad, double* __restrict__ loss) {
+    const size_t i = 4 * (blockIdx.x * static_cast<size_t>(256) + threadIdx.x);
+    if (i < n) {   // n is a multiple of 4
+        float4 s = *reinterpret_cast<const float4*>(part + i);
+#pragma unroll 8
+        for (int z = 1; z < splits; z++) {
+            const float4 v = *reinterpret_cast<const float4*>(part + z * n + i);
+            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+        }
+        *reinterpret_cast<float4*>(grad + i) = s;
+    }
+    if (blockIdx.x) return;
+    __shared__ double p[kLossBlocks];
+    p[threadIdx.x] = loss[1 + threadIdx.x];
+    __syncthreads();
+    for (int h = kLossBlocks / 2; h > 0; h >>= 1) {
+        if (static_cast<int>(threadIdx.x) < h) p[threadIdx.x] += p[threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) loss[0] = p[0];
+}
+
 // Inference in one kernel: features, hidden layers and output layer for 64 rows
 // per workgroup, with the activations (BF16) in LDS from layer to layer.
 //
@@ -659,39 +833,23 @@ void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-template <bool TA, bool TB, int EPI>
-void gemm(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb, const EpiArgs& e,
-          hipStream_t s) {
-    if constexpr (!TA && !TB && (EPI == kFwdGelu || EPI == kFwdLinear)) {
-        const bool aligned = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0) &&
-                             lda % 8 == 0 && ldb % 8 == 0 && K % 32 == 0;
-        if (aligned && N % 128 == 0) {
-            hipLaunchKernelGGL((gemm_nt_bf16<128, EPI>), dim3((M + 127) / 128, N / 128), dim3(256), 0, s, M, N, K, A,
-                               lda, B, ldb, e);
-            check(hipGetLastError(), "surrogate GEMM launch");
-            return;
-        }
-        if (aligned && N % 64 == 0) {
-            hipLaunchKernelGGL((gemm_nt_bf16<64, EPI>), dim3((M + 127) / 128, N / 64), dim3(256), 0, s, M, N, K, A,
-                               lda, B, ldb, e);
-            check(hipGetLastError(), "surrogate GEMM launch");
-            return;
-        }
+// C = A B^T (kBwdGelu: A B) with A (M x K), every matrix contiguous.  Forward
+// layers go to gemm_nt_bf16 once its larger tiles make 128 workgroups (16,384
+// rows of 320: 93 us per prediction against 109 with gemm_direct; of 1,024: 175
+// against 391; 1,024 rows of 1,024, 64 workgroups: 106 against 87).
+template <int EPI>
+void gemm(int M, int N, int K, const uint16_t* A, const uint16_t* B, const EpiArgs& e, hipStream_t s) {
+    const int bn = N % 128 ? 64 : 128;
+    if (K % 32) {
+        hipLaunchKernelGGL((gemm_bf16<EPI>), dim3((M + kTM - 1) / kTM, (N + kTN - 1) / kTN), dim3(256), 0, s, M, N, K,
+                           A, B, e);
+    } else if (EPI == kBwdGelu || N % 64 || (M + 127) / 128 * (N / bn) < 128) {
+        auto* const k = K % 128 == 0 ? &gemm_direct<4, EPI> : K % 64 == 0 ? &gemm_direct<2, EPI> : &gemm_direct<1, EPI>;
+        hipLaunchKernelGGL(k, dim3((M + 63) / 64, (N + 63) / 64), dim3(256), 0, s, M, N, K, A, B, e);
+    } else if constexpr (EPI != kBwdGelu) {
+        auto* const k = bn == 128 ? &gemm_nt_bf16<128, EPI> : &gemm_nt_bf16<64, EPI>;
+        hipLaunchKernelGGL(k, dim3((M + 127) / 128, N / bn), dim3(256), 0, s, M, N, K, A, K, B, K, e);
     }
-    dim3 grid((M + kTM - 1) / kTM, (N + kTN - 1) / kTN);
-    int kchunk = K;
-    if (EPI == kStoreF32) {
-        // weight gradients: few output tiles and a long K (the batch rows);
-        // split K so that the grid has about 256 workgroups
-        const int tiles = static_cast<int>(grid.x * grid.y);
-        const int splits = std::max(1, std::min(256 / std::max(tiles, 1), K / 256));
-        if (splits > 1) {
-            kchunk = ((K + splits - 1) / splits + kTK - 1) / kTK * kTK;
-            grid.z = (K + kchunk - 1) / kchunk;
-            check(hipMemsetAsync(e.zf, 0, static_cast<size_t>(M) * e.ldc * sizeof(float), s), "hipMemsetAsync");
-        }
-    }
-    hipLaunchKernelGGL((gemm_bf16<TA, TB, EPI>), grid, dim3(256), 0, s, M, N, K, A, lda, B, ldb, e, kchunk);
     check(hipGetLastError(), "surrogate GEMM launch");
 }
 
@@ -739,7 +897,7 @@ SurrogateNet::SurrogateNet(int K, double dt, int hidden, int depth, uint64_t see
     check(hipMalloc(&m2_, n_par_ * 4), "hipMalloc(surrogate)");
     check(hipMalloc(&wb_, n_par_ * 2), "hipMalloc(surrogate)");
     check(hipMalloc(&norm_, norm_len() * sizeof(double)), "hipMalloc(surrogate)");
-    check(hipMalloc(&loss_, sizeof(double)), "hipMalloc(surrogate)");
+    check(hipMalloc(&loss_, (1 + kLossBlocks) * sizeof(double)), "hipMalloc(surrogate)");
     check(hipMemcpy(par_, h.data(), n_par_ * 4, hipMemcpyHostToDevice), "hipMemcpy");
     check(hipMemset(m1_, 0, n_par_ * 4), "hipMemset");
     check(hipMemset(m2_, 0, n_par_ * 4), "hipMemset");
@@ -755,9 +913,9 @@ SurrogateNet::SurrogateNet(int K, double dt, int hidden, int depth, uint64_t see
 SurrogateNet::~SurrogateNet() {
     for (void* p : {static_cast<void*>(par_), static_cast<void*>(grad_), static_cast<void*>(m1_),
                     static_cast<void*>(m2_), static_cast<void*>(wb_), static_cast<void*>(norm_),
-                    static_cast<void*>(loss_), static_cast<void*>(act_), static_cast<void*>(pre_),
-                    static_cast<void*>(out_), static_cast<void*>(tgt_), static_cast<void*>(g0_),
-                    static_cast<void*>(g1_), static_cast<void*>(idx_)})
+                    static_cast<void*>(loss_), static_cast<void*>(part_), static_cast<void*>(act_),
+                    static_cast<void*>(pre_), static_cast<void*>(out_), static_cast<void*>(g_),
+                    static_cast<void*>(idx_)})
         if (p) (void)hipFree(p);
 }
 
@@ -769,18 +927,14 @@ void SurrogateNet::sync_bf16(hipStream_t s) {
 void SurrogateNet::ensure_batch(int rows) {
     if (rows <= cap_) return;
     for (void* p : {static_cast<void*>(act_), static_cast<void*>(pre_), static_cast<void*>(out_),
-                    static_cast<void*>(tgt_), static_cast<void*>(g0_), static_cast<void*>(g1_),
-                    static_cast<void*>(idx_)})
+                    static_cast<void*>(g_), static_cast<void*>(idx_)})
         if (p) (void)hipFree(p);
     cap_ = rows;
     const size_t r = static_cast<size_t>(rows);
-    const size_t wmax = std::max({s_.in_p, s_.hidden, s_.out_p});
     check(hipMalloc(&act_, r * (s_.in_p + static_cast<size_t>(s_.depth) * s_.hidden) * 2), "hipMalloc(surrogate batch)");
     check(hipMalloc(&pre_, r * static_cast<size_t>(s_.depth) * s_.hidden * 4), "hipMalloc(surrogate batch)");
     check(hipMalloc(&out_, r * s_.out_p * 4), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&tgt_, r * s_.out_p * 4), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&g0_, r * wmax * 2), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&g1_, r * wmax * 2), "hipMalloc(surrogate batch)");
+    check(hipMalloc(&g_, r * (s_.out_p + static_cast<size_t>(s_.depth) * s_.hidden) * 2), "hipMalloc(surrogate batch)");
     check(hipMalloc(&idx_, r * 4), "hipMalloc(surrogate batch)");
 }
 
@@ -796,44 +950,61 @@ void SurrogateNet::forward(int rows, hipStream_t st) {
         if (l < s_.depth) {
             e.zf = pre_ + r * static_cast<size_t>(l) * s_.hidden;
             e.hb = act_ + r * (s_.in_p + static_cast<size_t>(l) * s_.hidden);
-            gemm<false, false, kFwdGelu>(rows, fo, fi, H, fi, wb_ + oW_[l], fi, e, st);
+            gemm<kFwdGelu>(rows, fo, fi, H, wb_ + oW_[l], e, st);
         } else {
             e.zf = out_;
-            gemm<false, false, kFwdLinear>(rows, fo, fi, H, fi, wb_ + oW_[l], fi, e, st);
+            gemm<kFwdLinear>(rows, fo, fi, H, wb_ + oW_[l], e, st);
         }
     }
 }
 
-// loss on out_/tgt_, gradient into grad_, optional Adam step
-double SurrogateNet::backward_and_loss(int rows, bool update, double lr, hipStream_t st) {
+// loss of out_ against the pairs (rows idx, or all), gradient into grad_,
+// optional Adam step
+double SurrogateNet::backward_and_loss(int rows, const int* idx, const double* y0, const double* y1, bool update,
+                                       double lr, hipStream_t st) {
     const size_t r = static_cast<size_t>(rows);
-    check(hipMemsetAsync(loss_, 0, sizeof(double), st), "hipMemsetAsync");
-    hipLaunchKernelGGL(loss_kernel, dim3(256), dim3(256), 0, st, rows, s_.n_out, s_.out_p, out_, tgt_, g0_, loss_);
+    // G_depth, then G_{depth-1} .. G_0
+    const auto G = [&](int l) {
+        return l == s_.depth ? g_ : g_ + r * (s_.out_p + static_cast<size_t>(s_.depth - 1 - l) * s_.hidden);
+    };
+    hipLaunchKernelGGL(loss_kernel, dim3(kLossBlocks), dim3(256), 0, st, rows, idx, s_.K + 2, s_.n_out, s_.in_p,
+                       s_.out_p, y0, y1, norm_, out_, G(s_.depth), loss_);
     check(hipGetLastError(), "surrogate loss");
-    uint16_t* G = g0_;
-    uint16_t* Gn = g1_;
-    for (int l = s_.depth; l >= 0; l--) {
-        const int fi = s_.fan_in(l), fo = s_.fan_out(l);
-        const uint16_t* H = (l == 0) ? act_ : act_ + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
-        // dW_l = G^T H  (fo x fi)
-        EpiArgs ew{};
-        ew.zf = grad_ + oW_[l];
-        ew.ldc = fi;
-        gemm<true, true, kStoreF32>(fo, fi, rows, G, fo, H, fi, ew, st);
-        check(hipMemsetAsync(grad_ + oB_[l], 0, static_cast<size_t>(fo) * sizeof(float), st), "hipMemsetAsync");
-        hipLaunchKernelGGL(colsum_kernel, dim3((fo + 63) / 64, (rows + kColsumRows - 1) / kColsumRows), dim3(256), 0, st,
-                           rows, fo, G, grad_ + oB_[l]);
-        check(hipGetLastError(), "surrogate bias gradient");
-        if (l > 0) {
-            // G_{l-1} = (G W_l) * gelu'(Z_{l-1})  (rows x fi)
-            EpiArgs eb{};
-            eb.hb = Gn;
-            eb.zin = pre_ + r * static_cast<size_t>(l - 1) * s_.hidden;
-            eb.ldc = fi;
-            gemm<false, true, kBwdGelu>(rows, fi, fo, G, fo, wb_ + oW_[l], fi, eb, st);
-            std::swap(G, Gn);
-        }
+    for (int l = s_.depth; l > 0; l--) {
+        // G_{l-1} = (G_l W_l) * gelu'(Z_{l-1})  (rows x fan_in)
+        EpiArgs e{};
+        e.hb = G(l - 1);
+        e.zin = pre_ + r * static_cast<size_t>(l - 1) * s_.hidden;
+        e.ldc = s_.fan_in(l);
+        gemm<kBwdGelu>(rows, s_.fan_in(l), s_.fan_out(l), G(l), wb_ + oW_[l], e, st);
     }
+    GradArgs g{};
+    g.rows = rows;
+    g.n_par = n_par_;
+    for (int l = 0; l < s_.layers(); l++) {
+        g.fo[l] = s_.fan_out(l);
+        g.fi[l] = s_.fan_in(l);
+        g.oW[l] = oW_[l];
+        g.oB[l] = oB_[l];
+        g.G[l] = G(l);
+        g.H[l] = (l == 0) ? act_ : act_ + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
+        g.first[l + 1] = g.first[l] + (g.fo[l] + 63) / 64 * ((g.fi[l] + 63) / 64);
+    }
+    // at most kGradTiles workgroups of at least 256 rows each (4,096 rows of
+    // 4 x 256: 131 us per gradient with 512, 139 with 1,024 or 2,048)
+    const int tiles = g.first[s_.layers()];
+    const int want = std::max(1, std::min(kGradTiles / tiles, (rows + 255) / 256));
+    g.chunk = ((rows + want - 1) / want + 127) / 128 * 128;
+    const int splits = (rows + g.chunk - 1) / g.chunk;
+    if (splits > 1 && !part_)
+        check(hipMalloc(&part_, n_par_ * 4 * std::max(1, kGradTiles / tiles)), "hipMalloc(surrogate gradient)");
+    g.part = splits > 1 ? part_ : grad_;
+    hipLaunchKernelGGL(wgrad_kernel, dim3(tiles, splits), dim3(256), 0, st, g);
+    check(hipGetLastError(), "surrogate weight gradient");
+    const size_t nsum = splits > 1 ? n_par_ : 0;
+    hipLaunchKernelGGL(grad_sum_kernel, dim3(static_cast<unsigned>((nsum + 1023) / 1024 + (nsum == 0))), dim3(256), 0, st,
+                       nsum, splits, part_, grad_, loss_);
+    check(hipGetLastError(), "surrogate gradient sum");
     if (update) {
         adam_t_ += 1;
         const float c1 = 1.f - std::pow(0.9f, static_cast<float>(adam_t_));
@@ -909,11 +1080,9 @@ double SurrogateNet::train_epoch(long n, const double* y0, const double* P, cons
         check(hipMemcpyAsync(idx_, perm.data() + b0, rows * 4, hipMemcpyHostToDevice, st), "hipMemcpyAsync(idx)");
         hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, idx_, N, s_.K, y0, P, norm_, s_.in_p,
                            act_);
-        hipLaunchKernelGGL(targets_kernel, dim3(rows), dim3(64), 0, st, rows, idx_, N, s_.K, y0, y1, norm_, s_.in_p,
-                           s_.out_p, tgt_);
         check(hipGetLastError(), "surrogate features");
         forward(rows, st);
-        total += backward_and_loss(rows, true, lr, st);
+        total += backward_and_loss(rows, idx_, y0, y1, true, lr, st);
         nb++;
     }
     return nb ? total / nb : 0.0;
@@ -926,11 +1095,9 @@ double SurrogateNet::loss_grad(long n, const double* y0, const double* P, const 
     const int N = s_.K + 2;
     hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0, P, norm_, s_.in_p,
                        act_);
-    hipLaunchKernelGGL(targets_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0, y1, norm_, s_.in_p,
-                       s_.out_p, tgt_);
     check(hipGetLastError(), "surrogate features");
     forward(rows, st);
-    const double loss = backward_and_loss(rows, false, 0.0, st);
+    const double loss = backward_and_loss(rows, nullptr, y0, y1, false, 0.0, st);
     if (grad_host) check(hipMemcpy(grad_host, grad_, n_par_ * 4, hipMemcpyDeviceToHost), "hipMemcpy(grad)");
     return loss;
 }
@@ -1048,12 +1215,12 @@ void SurrogateNet::predict_noalloc(long n, const double* y0, const double* P, do
             if (l < s_.depth) {
                 e.zf = nullptr;
                 e.hb = next;
-                gemm<false, false, kFwdGelu>(rows, fo, fi, H, fi, wb_ + oW_[l], fi, e, st);
+                gemm<kFwdGelu>(rows, fo, fi, H, wb_ + oW_[l], e, st);
                 H = next;
                 next = (next == ha) ? hb : ha;
             } else {
                 e.zf = out;
-                gemm<false, false, kFwdLinear>(rows, fo, fi, H, fi, wb_ + oW_[l], fi, e, st);
+                gemm<kFwdLinear>(rows, fo, fi, H, wb_ + oW_[l], e, st);
             }
         }
         launch_apply(rows, N, s_.K, y0 + c0 * N, out, norm_, s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N, st);

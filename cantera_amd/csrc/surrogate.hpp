@@ -77,7 +77,8 @@ private:
     void ensure_batch(int rows);
     void forward(int rows, hipStream_t stream);
     bool infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t stream) const;
-    double backward_and_loss(int rows, bool update, double lr, hipStream_t stream);
+    double backward_and_loss(int rows, const int* idx, const double* y0, const double* y1, bool update, double lr,
+                             hipStream_t stream);
     void sync_bf16(hipStream_t stream);
 
     SurrogateShape s_{};
@@ -100,11 +101,10 @@ private:
     uint16_t* act_ = nullptr;       // H_0..H_depth (bf16), rows x width each
     float* pre_ = nullptr;          // Z_0..Z_{depth-1} (fp32)
     float* out_ = nullptr;          // rows x out_p
-    float* tgt_ = nullptr;          // rows x out_p
-    uint16_t* g0_ = nullptr;        // gradient operands (bf16), ping-pong
-    uint16_t* g1_ = nullptr;
+    uint16_t* g_ = nullptr;         // gradient operands G_depth..G_0 (bf16), rows x width each
     int* idx_ = nullptr;
-    double* loss_ = nullptr;
+    double* loss_ = nullptr;        // the loss, then its parts
+    float* part_ = nullptr;         // gradient copies of the row splits (at most 16 MB, or one)
 };
 
 }  // namespace cg

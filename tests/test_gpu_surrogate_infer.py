@@ -9,10 +9,12 @@ them per row, |h| <= 2 and |w| <= 1 / sqrt(hidden) <= 1 / 6.9, an output moves b
 less than 4e-3; the increments follow through sinh, and the projection does not
 enlarge an error in its own norm (factor 2: its weights depend on the
 increments)."""
+import os
+
 import numpy as np
 import pytest
 
-from conftest import mech_file
+from conftest import GOLDEN, mech_file
 from test_gpu_surrogate import bf16, gelu, pad, synthetic_pairs
 
 pytestmark = pytest.mark.gpu
@@ -37,15 +39,29 @@ def network_output(params, norm, K, hidden, depth, y0, P):
     return h[:, :K + 1].astype(np.float64)
 
 
+def mech_126(path):
+    """The first 126 species of the merged mechanism with GRI-3.0's 325
+    reactions: the largest mechanism the network takes."""
+    with open(os.path.join(GOLDEN, "gri30_ndodecane.mech")) as f:
+        lines = f.read().splitlines()
+    head = [l for l in lines if l.split()[0] in ("CGMECH", "phase", "source", "elements")]
+    species = [l for l in lines if l.startswith("S ")][:126]
+    reactions = [l for l in lines if l[:2] in ("R ", "E ")][:2 * 325]
+    path.write_text("\n".join(head + ["species 126"] + species + ["reactions 325"] + reactions + ["end", ""]))
+    return str(path)
+
+
 @pytest.mark.parametrize("mech,hidden,depth,rows", [
     ("h2o2", 64, 1, 1), ("h2o2", 48, 2, 33), ("h2o2", 128, 2, 64), ("gri30", 192, 3, 65),
-    ("gri30", 256, 4, 31), ("gri30", 256, 1, 129), ("gri30", 320, 2, 97), ("nDodecane", 64, 2, 1000)])
-def test_predict_matches_reference(mech, hidden, depth, rows):
+    ("gri30", 256, 4, 31), ("gri30", 256, 1, 129), ("gri30", 320, 2, 97), ("nDodecane", 64, 2, 1000),
+    ("126 species", 64, 1, 70)])
+def test_predict_matches_reference(mech, hidden, depth, rows, tmp_path):
     import cantera_amd as ca
     from cantera_amd.surrogate import Surrogate
     from cantera_amd.workloads import MechInfo
-    info = MechInfo(mech_file(mech))
-    sol = ca.Solution(mech)
+    path = mech_126(tmp_path / "m126.mech") if mech == "126 species" else mech_file(mech)
+    info = MechInfo(path)
+    sol = ca.Solution(path)
     K = sol.n_species
     sur = Surrogate(sol, dt=1e-6, hidden=hidden, depth=depth, seed=hidden + depth)
     y0, P, y1 = synthetic_pairs(info, max(rows, 256), 11)
