@@ -399,7 +399,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // steps of 32 through LDS with 16-byte global loads and LDS accesses, the next
 // step's tile loaded into registers while the current one is multiplied.
 // Requires K % 32 == 0, N % BN == 0, lda, ldb % 8 == 0 and 16-byte aligned A,
-// B (checked by the launcher); rows >= M read zero and are not stored.
+// B (as every buffer here is); rows >= M read zero and are not stored.
 template <int BN, int EPI>
 __global__ __launch_bounds__(256) void gemm_nt_bf16(int M, int N, int K, const uint16_t* __restrict__ A, int lda,
                                                     const uint16_t* __restrict__ B, int ldb, EpiArgs e) {

@@ -1,8 +1,8 @@
 // Wavefront-cooperative gas kinetics for one state at a time: lanes over
 // species for thermo and concentrations, lanes over reactions for rate
-// constants, equilibrium constants and rates of progress, and a balanced
-// sub-row gather for the net production rates.  Shared by the batched rate
-// kernel and the per-reactor BDF integrator.
+// constants, equilibrium constants and rates of progress, which they add to the
+// species' net production rates in LDS.  Shared by the batched rate kernels and
+// the per-reactor BDF integrator.
 //
 // Reference algorithm (file:line in the Cantera sources):
 //   BulkKinetics::updateROP            src/kinetics/BulkKinetics.cpp:457-545
