@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void j
         double* const ckv = vec + kVec * (kTile + ts);        // (wdot_k - D_k) / C_tot
         double* const hjv = vec + kVec * (2 * kTile + ts);    // sum_k h_k JC_kj, then the T row
         double* const ftv = vec + kVec * (3 * kTile + ts);    // f(T + dT), then the T column
-            if (w < kTile) {
+        if (w < kTile) {
             hkv[lane] = lane < K ? hk : 0.0;
         } else {
             ftv[lane] = f;
@@ -321,11 +321,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void j
             } else if (lane < N) {   // the temperature row, then odd species rows
                 o[N] = static_cast<OT>(lane >= 2 ? hjv[cj] : (lane == 1 ? ftv[K] : 0.0));
             }
-            const double t01 = lane == 1 ? 1.0 : 0.0;   // column 0 is zero, column 1 d / dT
 #pragma unroll 4
             for (int k = w / kTile; k < K; k += kWaves / kTile) {
                 const double jc = wv[k] * wi * (A[k * K + cj] + ckv[k]);
-                const double jt1 = t01 * ftv[k];
+                const double jt1 = lane == 1 ? ftv[k] : 0.0;   // column 0 is zero at any state, column 1 d / dT
                 if (lane < N) o[(k + 2) * N] = static_cast<OT>(lane >= 2 ? jc : jt1);
             }
         }
