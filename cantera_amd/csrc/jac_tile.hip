@@ -75,9 +75,9 @@ __device__ __forceinline__ void deriv_pass(const DevMech& m, const JacTables& jt
         ex[0] = x.rd.y * g.logT - x.rd.z * g.recipT;
         ex[1] = std_kc_arg(x, g.logC0, v);
         ex[2] = fa.y * g.logT - fa.z * g.recipT;
-        ex[3] = fmax(-g.T * fb.x, -1e4);
-        ex[4] = fmax(-g.T * fb.y, -1e4);
-        ex[5] = fmin(fmax(-fb.z * g.recipT, -1e4), 1e4);
+        ex[3] = troe_arg(-g.T * fb.x);
+        ex[4] = troe_arg(-g.T * fb.y);
+        ex[5] = troe_arg(-fb.z * g.recipT);
         fast_exp_n(ex);
         ekc = ex[1];
         kf = x.rd.x * ex[0];

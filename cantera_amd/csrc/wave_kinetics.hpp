@@ -331,8 +331,9 @@ __device__ __forceinline__ void load_rxn(const DevMech& m, int p, RxnRegs& x) {
 // (both subtractions exact to the last bit through the fused multiply-adds),
 // exp(r) = 1 + r + r^2 q(r) with q the degree-9 minimax polynomial of the
 // relative error (3.7e-18, Remez exchange), scaled by v_ldexp, which gives
-// infinity, subnormals and zero by itself.  Error below 0.63 ulp.  Arguments
-// are finite (an infinite one gives NaN) and below 1e13 in magnitude.
+// infinity, subnormals and zero by itself.  Error below 0.92 ulp, below 0.62
+// for 99% of 4 million arguments in [-700, 700] against extended precision.
+// Arguments are finite (an infinite one gives NaN) and below 1e13 in magnitude.
 constexpr double kLog2e = 1.4426950408889634;
 constexpr double kLn2Hi = 0x1.62e42fefa39efp-1, kLn2Lo = 0x1.abc9e3b39803fp-56;
 constexpr double kExpC[10] = {0x1.ad7f3cdbe6745p-26, 0x1.28ad9ef903086p-22, 0x1.71df25b30699dp-19,
@@ -498,6 +499,17 @@ __device__ __forceinline__ double fast_exp10(double x) {
     const double e = fast_exp(h);
     return fma(e, l, e);
 }
+
+// Exponent of a Troe centre term, kept where fast_exp is defined: 1/T3 is
+// infinite for Tsang, T2 is 1e100 in some mechanisms, T3 and T1 may be tiny and
+// of either sign.  Beyond +-1e4 the exponential is infinite or 0 all the same.
+__device__ __forceinline__ double troe_arg(double x) { return fmin(fmax(x, -1e4), 1e4); }
+
+// Exponent of 1/K_c kept where fast_exp is defined (the NASA polynomials pass
+// 1e13 at 1e7 K, a vanishing pressure makes it infinite): beyond +-1e5 the
+// exponential is infinite or 0 all the same.  NaN goes to the upper end, that is
+// to the cap of 1/K_c.
+__device__ __forceinline__ double kc_arg(double x) { return fmax(fmin(x, 1e5), -1e5); }
 
 // Transcendentals of the rate constants.  kF32: evaluated in FP32 (hardware
 // exp2/log2 based) on FP64 arguments rounded to FP32, widened back to FP64;
@@ -667,11 +679,9 @@ __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const Gas
         double work = 0.0;
         if (type == kTroe && !sri) {
             // Troe (fo[7] = 0) and Tsang (Fcent = A + B T)
-            // (1/T3 is infinite for Tsang, and mechanisms use 1e100 for T2: the
-            // exponents are kept moderate)
-            double Fcent = (1.0 - fo[3]) * rate_exp<kF32>(fmax(-g.T * fo[4], -1e4)) +
-                           fo[3] * rate_exp<kF32>(fmax(-g.T * fo[5], -1e4));
-            if (fo[6] != 0.0) Fcent += rate_exp<kF32>(fmin(fmax(-fo[6] / g.T, -1e4), 1e4));
+            double Fcent = (1.0 - fo[3]) * rate_exp<kF32>(troe_arg(-g.T * fo[4])) +
+                           fo[3] * rate_exp<kF32>(troe_arg(-g.T * fo[5]));
+            if (fo[6] != 0.0) Fcent += rate_exp<kF32>(troe_arg(-fo[6] / g.T));
             Fcent += fo[7] * g.T;
             work = rate_log10<kF32>(fmax(Fcent, kSmallNumber));
         }
@@ -722,7 +732,7 @@ __device__ __forceinline__ void eval_reaction(const DevMech& m, int p, const Gas
             if (x.nr > 2) dr += MU[x.rk[2]];
             delta -= dr;
         }
-        rkcn = fmin(fast_exp(delta - rd.w * g.logC0), kBigNumber);
+        rkcn = fmin(fast_exp(kc_arg(delta - rd.w * g.logC0)), kBigNumber);
     }
     o.rkcn = rkcn;
     double ropf = kf * perturb;
@@ -818,7 +828,7 @@ struct StdRxn {
 __device__ __forceinline__ double std_kc_arg(const StdRxn& x, double logC0, const double2 (&v)[6]) {
     const double dr = (v[0].y + v[1].y) + v[2].y;
     const double dp = (v[3].y + v[4].y) + v[5].y;
-    return (dp - dr) - x.rd.w * logC0;
+    return kc_arg((dp - dr) - x.rd.w * logC0);
 }
 
 // net rate of progress from the forward constant kf (perturbed, times [M] for a
@@ -904,15 +914,14 @@ __device__ __forceinline__ void falloff_pass(const DevMech& m, const RxnS* rs, c
 #pragma unroll
     for (int e = 0; e < 6; e++) v[e] = lv.pair(x.slot(e));
     const double M = add_mul_rn(efficiency_sum(m, C, ia.w, ib.x), tbdef, g.ctot);
-    // the pass's six exponentials side by side (Troe exponents kept moderate:
-    // 1/T3 is infinite for Tsang, some T2 are 1e100)
+    // the pass's six exponentials side by side
     double ex[6];
     ex[0] = x.rd.y * g.logT - x.rd.z * g.recipT;
     ex[1] = std_kc_arg(x, g.logC0, v);
     ex[2] = fa.y * g.logT - fa.z * g.recipT;
-    ex[3] = fmax(-g.T * fb.x, -1e4);
-    ex[4] = fmax(-g.T * fb.y, -1e4);
-    ex[5] = fmin(fmax(-fb.z * g.recipT, -1e4), 1e4);
+    ex[3] = troe_arg(-g.T * fb.x);
+    ex[4] = troe_arg(-g.T * fb.y);
+    ex[5] = troe_arg(-fb.z * g.recipT);
     const bool falloff = __any(type >= kLindemann);
     if constexpr (kF32) {
         ex[1] = fast_exp(ex[1]);

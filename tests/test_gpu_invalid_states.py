@@ -40,3 +40,22 @@ def test_mass_row_and_column_are_zero(mech):
     scale = np.abs(clean[1::2]).max(axis=(1, 2), keepdims=True)
     assert np.abs(J[1::2] - clean[1::2]).max() <= 1e-12 * scale.max()
     assert np.all(np.abs(J[1::2] - clean[1::2]) <= 1e-12 * scale)
+
+
+@pytest.mark.parametrize("mech", ["gri30", "h2o2", "pdep-test", "chemically-activated-reaction"])
+@pytest.mark.parametrize("n", [20, 4100])
+def test_exponents_beyond_any_range(mech, n):
+    """Far outside the fits of the thermodynamics the exponent of an equilibrium
+    constant passes 1e13: exp is then 0 or infinite, of no other sign, as in the
+    oracle.  n on either side of the kernels' switch."""
+    import cantera_amd as ca
+    from conftest import mech_file
+    from oracle.oracle import Mech
+    sol, om = ca.Solution(mech), Mech(mech_file(mech))
+    T, P, Y = states(sol, n)
+    T[:10], T[10:20] = 1e10, 1e12
+    w = sol.net_production_rates(T, P, Y)
+    for s in range(20):
+        ref = om.rates(T[s], P[s], np.ascontiguousarray(Y[:, s]))["wdot"]
+        assert np.array_equal(np.isnan(w[:, s]), np.isnan(ref))
+        assert np.array_equal(np.where(np.isinf(w[:, s]), w[:, s], 0.0), np.where(np.isinf(ref), ref, 0.0))
