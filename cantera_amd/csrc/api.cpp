@@ -397,7 +397,7 @@ int32_t cg_jac_batch_device(int32_t h, int64_t n, const double* T, const double*
         const JacTables& jt = mo.dm->jac();
         const bool tile = jt.nd > 0 && jac_tile_lds_bytes(m, jt) <= kLdsPerCu;
         const size_t lds = tile ? jac_tile_lds_bytes(m, jt) : jac_lds_bytes(m, mo.ns);
-        const void* kp = tile ? jac_tile_kernel_ptr(f32) : jac_kernel_ptr(mo.ns, f32);
+        const void* kp = tile ? jac_tile_kernel_ptr(f32) : jac_kernel_ptr(m, mo.ns, f32);
         set_lds_limit(kp, lds);
         const int grid = tile ? grid_for(kp, lds, 0, jac_tile_items(n), 256) : grid_for(kp, lds, 0, n);
         hipStream_t s = static_cast<hipStream_t>(stream);
@@ -584,7 +584,7 @@ static int32_t create_batch(int32_t h, int64_t n, const double* T0, const double
         }
         check(hipMemcpy(b->rec, rec.data(), rec.size() * 8, hipMemcpyHostToDevice), "hipMemcpy(records)");
         b->lds = bdf_lds_bytes(m, b->ld, b->fp32, b->global_matrix);
-        set_lds_limit(bdf_kernel_ptr(m.N, b->fp32, b->global_matrix), b->lds);
+        set_lds_limit(bdf_kernel_ptr(m, b->fp32, b->global_matrix), b->lds);
         std::lock_guard<std::mutex> lk(g_mu);
         g_batches.push_back(std::move(b));
         return static_cast<int32_t>(g_batches.size() - 1);
@@ -757,7 +757,7 @@ int32_t cg_reactors_create_mole(int32_t h, int64_t n, const double* T0, const do
         }
         check(hipMemcpy(b->rec, rec.data(), rec.size() * 8, hipMemcpyHostToDevice), "hipMemcpy(records)");
         b->lds = lds;
-        set_lds_limit(bdf_mole_kernel_ptr(N), b->lds);
+        set_lds_limit(bdf_mole_kernel_ptr(m, N), b->lds);
         std::lock_guard<std::mutex> lk(g_mu);
         g_batches.push_back(std::move(b));
         return static_cast<int32_t>(g_batches.size() - 1);
@@ -815,7 +815,7 @@ int32_t cg_reactors_set_matrix_storage(int32_t h, int32_t storage) {
         b.drop_graph();
         const DevMech& m = b.mech->dm->view();
         b.lds = bdf_lds_bytes(m, b.ld, b.fp32, b.global_matrix);
-        set_lds_limit(bdf_kernel_ptr(m.N, b.fp32, b.global_matrix, b.nsens > 0), b.lds);
+        set_lds_limit(bdf_kernel_ptr(m, b.fp32, b.global_matrix, b.nsens > 0), b.lds);
         return 0;
     });
 }
@@ -865,7 +865,8 @@ static BdfArgs advance_args(Batch& b) {
 }
 
 static const void* batch_kernel_ptr(const Batch& b) {
-    return b.mole ? bdf_mole_kernel_ptr(b.N) : bdf_kernel_ptr(b.N, b.fp32, b.global_matrix, b.nsens > 0);
+    const DevMech& m = b.mech->dm->view();
+    return b.mole ? bdf_mole_kernel_ptr(m, b.N) : bdf_kernel_ptr(m, b.fp32, b.global_matrix, b.nsens > 0);
 }
 
 static hipError_t batch_launch(const Batch& b, const BdfArgs& a, int grid) {
@@ -994,7 +995,7 @@ int32_t cg_reactors_autotune(int32_t h, const double* t_probe_dev, int32_t* choi
             b.global_matrix = cand[c].first == 2;
             b.waves_per_cu = cand[c].second;
             b.lds = bdf_lds_bytes(m, b.ld, b.fp32, b.global_matrix);
-            const void* kp = bdf_kernel_ptr(m.N, b.fp32, b.global_matrix);
+            const void* kp = bdf_kernel_ptr(m, b.fp32, b.global_matrix);
             set_lds_limit(kp, b.lds);
             const int grid = advance_grid(b);
             double ms = -1.0;
@@ -1018,7 +1019,7 @@ int32_t cg_reactors_autotune(int32_t h, const double* t_probe_dev, int32_t* choi
         if (best < 0) { b.global_matrix = global0; b.waves_per_cu = wpc0; }
         else { b.global_matrix = cand[best].first == 2; b.waves_per_cu = cand[best].second; }
         b.lds = bdf_lds_bytes(m, b.ld, b.fp32, b.global_matrix);
-        set_lds_limit(bdf_kernel_ptr(m.N, b.fp32, b.global_matrix), b.lds);
+        set_lds_limit(bdf_kernel_ptr(m, b.fp32, b.global_matrix), b.lds);
         b.drop_graph();
         b.launched = launched0;
         if (choice) {
@@ -1058,7 +1059,7 @@ int32_t cg_reactors_add_sensitivity_reaction(int32_t h, int32_t rxn) {
         b.sens_rxn_orig[b.nsens] = rxn;
         b.nsens++;
         b.drop_graph();
-        set_lds_limit(bdf_kernel_ptr(b.N, false, b.global_matrix, true), b.lds);
+        set_lds_limit(bdf_kernel_ptr(b.mech->dm->view(), false, b.global_matrix, true), b.lds);
         return b.nsens - 1;
     });
 }
@@ -1356,7 +1357,7 @@ static void advance_surrogate_device(Batch& b, SurrogateObj& so, const double* t
                            b.stream), "surrogate gather");
     so.net->predict(n, b.sg_Y, b.sg_P, b.sg_Yn, b.stream);
     const size_t lds = guard_lds_bytes(m, b.ns);
-    const void* gk = guard_kernel_ptr(b.ns);
+    const void* gk = guard_kernel_ptr(m, b.ns);
     set_lds_limit(gk, lds);
     const int grid = grid_for(gk, lds, 0, n);
     check(surrogate_guard(m, b.ns, n, elig, b.sg_Y, b.sg_Yn, b.sg_F, fvalid, b.sg_P, b.rec, b.rec_stride, NP, b.tout,
@@ -1388,7 +1389,7 @@ int32_t cg_reactors_net_production_rates_device(int32_t bh, double* wdot_dev) {
         if (b.mole) throw std::runtime_error("rates at the states of a mole-based batch are not available");
         const DevMech& m = b.mech->dm->view();
         const size_t lds = reactor_rates_lds_bytes(m);
-        const void* kp = reactor_rates_kernel_ptr(b.ns);
+        const void* kp = reactor_rates_kernel_ptr(m, b.ns);
         set_lds_limit(kp, lds);
         const int grid = grid_for(kp, lds, 0, b.n);
         check(reactor_rates_launch(m, b.ns, b.n, b.rec, b.rec_stride, b.const_volume ? 1 : 0, wdot_dev, grid, lds,

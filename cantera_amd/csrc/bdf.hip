@@ -3,20 +3,13 @@
 
 namespace cg {
 
-const void* bdf_kernel_r16(bool, bool);
-const void* bdf_kernel_r32(bool, bool);
-const void* bdf_kernel_lr56(bool, bool);
-const void* bdf_kernel_lr64(bool, bool);
-const void* bdf_kernel_l2(bool, bool);
-const void* bdf_kernel_gr56(bool, bool);
-const void* bdf_kernel_gr64(bool, bool);
-hipError_t bdf_launch_r16(const BdfArgs&, bool, int, size_t, hipStream_t);
-hipError_t bdf_launch_r32(const BdfArgs&, bool, int, size_t, hipStream_t);
-hipError_t bdf_launch_lr56(const BdfArgs&, bool, int, size_t, hipStream_t);
-hipError_t bdf_launch_lr64(const BdfArgs&, bool, int, size_t, hipStream_t);
-hipError_t bdf_launch_l2(const BdfArgs&, bool, int, size_t, hipStream_t);
-hipError_t bdf_launch_gr56(const BdfArgs&, bool, int, size_t, hipStream_t);
-hipError_t bdf_launch_gr64(const BdfArgs&, bool, int, size_t, hipStream_t);
+const void* bdf_kernel_r16(bool, bool, bool);
+const void* bdf_kernel_r32(bool, bool, bool);
+const void* bdf_kernel_lr56(bool, bool, bool);
+const void* bdf_kernel_lr64(bool, bool, bool);
+const void* bdf_kernel_l2(bool, bool, bool);
+const void* bdf_kernel_gr56(bool, bool, bool);
+const void* bdf_kernel_gr64(bool, bool, bool);
 
 namespace {
 __global__ void reset_queue_kernel(int* q) { *q = 0; }
@@ -55,27 +48,24 @@ size_t bdf_lds_bytes(const DevMech& m, int ld, bool fp32, bool global) {
     return bytes;
 }
 
-const void* bdf_kernel_ptr(int N, bool fp32, bool global, bool sens) {
-    switch (bdf_variant(N)) {
-        case 16: return bdf_kernel_r16(fp32, sens);
-        case 32: return bdf_kernel_r32(fp32, sens);
-        case 56: return global ? bdf_kernel_gr56(fp32, sens) : bdf_kernel_lr56(fp32, sens);
-        case 64: return global ? bdf_kernel_gr64(fp32, sens) : bdf_kernel_lr64(fp32, sens);
-        case 2: return bdf_kernel_l2(fp32, sens);
+const void* bdf_kernel_ptr(const DevMech& m, bool fp32, bool global, bool sens) {
+    const bool gen = m.gen_end > 0;
+    switch (bdf_variant(m.N)) {
+        case 16: return bdf_kernel_r16(fp32, sens, gen);
+        case 32: return bdf_kernel_r32(fp32, sens, gen);
+        case 56: return global ? bdf_kernel_gr56(fp32, sens, gen) : bdf_kernel_lr56(fp32, sens, gen);
+        case 64: return global ? bdf_kernel_gr64(fp32, sens, gen) : bdf_kernel_lr64(fp32, sens, gen);
+        case 2: return bdf_kernel_l2(fp32, sens, gen);
         default: return nullptr;
     }
 }
 
-hipError_t bdf_launch(const BdfArgs& a, bool fp32, bool global, int grid, size_t lds, hipStream_t stream) {
+hipError_t bdf_launch(BdfArgs a, bool fp32, bool global, int grid, size_t lds, hipStream_t stream) {
+    const void* kernel = bdf_kernel_ptr(a.mech, fp32, global, a.nsens > 0);
+    if (!kernel) return hipErrorInvalidValue;
     hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(1), 0, stream, a.queue);
-    switch (bdf_variant(a.mech.N)) {
-        case 16: return bdf_launch_r16(a, fp32, grid, lds, stream);
-        case 32: return bdf_launch_r32(a, fp32, grid, lds, stream);
-        case 56: return global ? bdf_launch_gr56(a, fp32, grid, lds, stream) : bdf_launch_lr56(a, fp32, grid, lds, stream);
-        case 64: return global ? bdf_launch_gr64(a, fp32, grid, lds, stream) : bdf_launch_lr64(a, fp32, grid, lds, stream);
-        case 2: return bdf_launch_l2(a, fp32, grid, lds, stream);
-        default: return hipErrorInvalidValue;
-    }
+    void* args[] = {&a};
+    return hipLaunchKernel(kernel, dim3(grid), dim3(64), args, lds, stream);
 }
 
 }  // namespace cg

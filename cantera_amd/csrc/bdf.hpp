@@ -76,14 +76,14 @@ size_t bdf_lu_elems(int N, int ld);
 // global-memory factor slot instead of LDS
 size_t bdf_lds_bytes(const DevMech& m, int ld, bool fp32, bool global);
 // a.nsens > 0 selects the FP64 kernels that also integrate the sensitivities
-hipError_t bdf_launch(const BdfArgs& a, bool fp32, bool global, int grid, size_t lds, hipStream_t stream);
-const void* bdf_kernel_ptr(int N, bool fp32, bool global, bool sens = false);
+hipError_t bdf_launch(BdfArgs a, bool fp32, bool global, int grid, size_t lds, hipStream_t stream);
+const void* bdf_kernel_ptr(const DevMech& m, bool fp32, bool global, bool sens = false);
 
 // mole-reactor integrator: state [n_0..n_{K-1}, T], N = K + 1 <= 256
 int bdf_mole_ns(int N);
 size_t bdf_mole_lds_bytes(const DevMech& m, int N, int nnz);
-hipError_t bdf_mole_launch(const BdfArgs& a, int grid, size_t lds, hipStream_t stream);
-const void* bdf_mole_kernel_ptr(int N);
+hipError_t bdf_mole_launch(BdfArgs a, int grid, size_t lds, hipStream_t stream);
+const void* bdf_mole_kernel_ptr(const DevMech& m, int N);
 
 // Batched rate evaluation (species-major SoA in and out): kernel and launch
 // shape for n states.  f32: rate constants through FP32 transcendentals.
@@ -97,9 +97,9 @@ RatesPlan rates_plan(const DevMech& m, int ns, bool f32, long n);
 hipError_t rates_launch(const RatesPlan& p, DevMech m, long n, const double* T, const double* P, const double* Y,
                         double* wdot, int grid, hipStream_t stream);
 // rates at the output states of a reactor batch (records as the integrator's)
-hipError_t reactor_rates_launch(const DevMech& m, int ns, long n, const double* rec, size_t stride, int cv,
+hipError_t reactor_rates_launch(DevMech m, int ns, long n, const double* rec, size_t stride, int cv,
                                 double* wdot, int grid, size_t lds, hipStream_t stream);
-const void* reactor_rates_kernel_ptr(int ns);
+const void* reactor_rates_kernel_ptr(const DevMech& m, int ns);
 size_t reactor_rates_lds_bytes(const DevMech& m);
 
 // longest-first processing order for the integrator's work queue (kernels
@@ -115,7 +115,7 @@ hipError_t pack_rows(const double* src, size_t stride, int width, int rows, doub
 
 // guarded surrogate steps for reactor batches (all on the device)
 size_t guard_lds_bytes(const DevMech& m, int ns);
-const void* guard_kernel_ptr(int ns);
+const void* guard_kernel_ptr(const DevMech& m, int ns);
 hipError_t surrogate_clear(int* p, int n, hipStream_t s);
 // output states of all reactors, reference order [m, T, Y], n x N doubles
 hipError_t export_states(int n, const double* rec, size_t stride, int NP, int N, int K, double* Y, hipStream_t s);
@@ -132,9 +132,9 @@ hipError_t surrogate_guard(const DevMech& m, int ns, int n, int* elig, const dou
 // batched reactor Jacobians (inputs as the rates, output N x N per state)
 size_t jac_lds_bytes(const DevMech& m, int ns);
 // f32: FP32 output (the FP64 assembly rounded at the store; needs ns == 1)
-hipError_t jac_launch(const DevMech& m, int ns, bool f32, long n, const double* T, const double* P, const double* Y,
+hipError_t jac_launch(DevMech m, int ns, bool f32, long n, const double* T, const double* P, const double* Y,
                       void* J, int grid, size_t lds, hipStream_t stream);
-const void* jac_kernel_ptr(int ns, bool f32);
+const void* jac_kernel_ptr(const DevMech& m, int ns, bool f32);
 
 // the same without atomics, for mechanisms with JacTables
 size_t jac_tile_lds_bytes(const DevMech& m, const JacTables& jt);

@@ -105,7 +105,7 @@ struct has_jac_in_place : std::false_type {};
 template <class LS>
 struct has_jac_in_place<LS, std::void_t<decltype(&LS::form_in_place)>> : std::true_type {};
 
-template <int NS, class LS, typename MT, bool kSens = false, bool kMole = false>
+template <int NS, class LS, typename MT, bool kGen, bool kSens = false, bool kMole = false>
 struct Integrator {
     const DevMech& m;
     const BdfArgs& a;
@@ -211,8 +211,8 @@ struct Integrator {
         for (int s = 0; s < NS; s++)
             if (comp(s) < N) S.yb[comp(s)] = yy[s];
         wave_sync();
-        if constexpr (kMole) mole_rhs_call<NS>(kernarg_mech(), L, uni(c.P));
-        else rhs_call<NS>(kernarg_mech(), L, uni(c.P));
+        if constexpr (kMole) mole_rhs_call<NS, kGen>(kernarg_mech(), L, uni(c.P));
+        else rhs_call<NS, kGen>(kernarg_mech(), L, uni(c.P));
         int bad = 0;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
@@ -261,7 +261,7 @@ struct Integrator {
         for (int s = 0; s < NS; s++)
             if (comp(s) < N) S.yb[comp(s)] = yy[s];
         wave_sync();
-        rhs_pert_call<NS>(kernarg_mech(), L, uni(c.P), rx, v);
+        rhs_pert_call<NS, kGen>(kernarg_mech(), L, uni(c.P), rx, v);
         int bad = 0;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
@@ -576,7 +576,7 @@ struct Integrator {
                     if (comp(s) < N) S.Y0[comp(s)] = fmax(zn[0][s], 0.0);
                 wave_sync();
                 const SparseTables* sp = (const SparseTables*)&kernarg_args()->sp;
-                mole_jac_call<NS>(kernarg_mech(), L, uni(c.P), Js + sp_nnz(), Js, sp);
+                mole_jac_call<NS, kGen>(kernarg_mech(), L, uni(c.P), Js + sp_nnz(), Js, sp);
             } else {
 #pragma unroll
                 for (int s = 0; s < NS; s++)
@@ -587,12 +587,12 @@ struct Integrator {
                 wave_sync();
                 if constexpr (has_jac_in_place<LS>::value) {
                     if (ls.jac_in_place(N)) {
-                        jac_lds_call<NS>(kernarg_mech(), L, uni(c.P), ls.jac_offset(), Js);
+                        jac_lds_call<NS, kGen>(kernarg_mech(), L, uni(c.P), ls.jac_offset(), Js);
                         ls.form_in_place(N, gamma);
                         formed = true;
                     }
                 }
-                if (!formed) jac_call<NS>(kernarg_mech(), L, uni(c.P), Js);
+                if (!formed) jac_call<NS, kGen>(kernarg_mech(), L, uni(c.P), Js);
             }
         }
         if (!formed) ls.form(Js, N, gamma);
@@ -1415,7 +1415,7 @@ __host__ __device__ inline size_t bdf_scratch_doubles(int K, int ns, bool mole =
     return static_cast<size_t>(kWave) * ns * (mole ? 3 : 4) + species_doubles(K) + (mole ? 1 : 2) * K + kCtlDoubles;
 }
 
-template <int NS, class LS, typename MT, bool kSens = false, bool kMole = false>
+template <int NS, class LS, typename MT, bool kGen, bool kSens = false, bool kMole = false>
 __device__ __forceinline__ void bdf_advance_body(const BdfArgs& a) {
     const DevMech& m = a.mech;
     ScratchLayout L;
@@ -1429,8 +1429,8 @@ __device__ __forceinline__ void bdf_advance_body(const BdfArgs& a) {
     double* base = lds_base() + off;
     Ctl& c = *reinterpret_cast<Ctl*>(base);
     base += kCtlDoubles;
-    Integrator<NS, LS, MT, kSens, kMole> it(m, a, c);
-    it.S = scratch_view(L, kernarg_mech());
+    Integrator<NS, LS, MT, kGen, kSens, kMole> it(m, a, c);
+    it.S = scratch_view<kGen>(L, kernarg_mech());
     it.L = L;
     it.lane = lane_id();
     it.N = kMole ? m.K + 1 + (m.const_volume ? 1 : 0) : m.N;

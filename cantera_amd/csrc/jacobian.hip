@@ -32,8 +32,8 @@ namespace {
 // registers went to scratch memory.
 // OT: element type of the output (double, or float for CG_FP32: the FP64
 // assembly rounded once at the store, which halves the HBM bytes written).
-template <int NS, bool kLdsJ, typename OT>
-__global__ __launch_bounds__(64) void jac_batch_kernel(DevMech m, long n, const double* __restrict__ T,
+template <int NS, bool kLdsJ, typename OT, bool kGen>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void jac_batch_kernel(DevMech m, long n, const double* __restrict__ T,
                                                        const double* __restrict__ P, const double* __restrict__ Y,
                                                        OT* __restrict__ J) {
     const int lane = lane_id();
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(64) void jac_batch_kernel(DevMech m, long n, const 
     L.Y0 = off;  off += kWave * NS;
     L.F0 = off;  off += kWave * NS;
     L.W2 = off;  off += 2 * m.K;
-    const WaveScratch S = scratch_view(L, kernarg_mech());
+    const Scratch<kGen> S = scratch_view<kGen>(L, kernarg_mech());
     double* Jl = lds_base() + off;
     const int NN = m.N * m.N;
     const XcdStates xs(n);
@@ -88,25 +88,21 @@ size_t jac_lds_bytes(const DevMech& m, int ns) {
     return d * sizeof(double);
 }
 
-hipError_t jac_launch(const DevMech& m, int ns, bool f32, long n, const double* T, const double* P, const double* Y,
-                      void* J, int grid, size_t lds, hipStream_t stream) {
-    if (ns == 1 && f32)
-        hipLaunchKernelGGL((jac_batch_kernel<1, true, float>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y,
-                           static_cast<float*>(J));
-    else if (ns == 1)
-        hipLaunchKernelGGL((jac_batch_kernel<1, true, double>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y,
-                           static_cast<double*>(J));
-    else if (ns == 2 && !f32)
-        hipLaunchKernelGGL((jac_batch_kernel<2, false, double>), dim3(grid), dim3(64), lds, stream, m, n, T, P, Y,
-                           static_cast<double*>(J));
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+// up to 62 species: only mechanisms with general reactions come here
+const void* jac_kernel_ptr(const DevMech& m, int ns, bool f32) {
+    if (ns == 1) return f32 ? reinterpret_cast<const void*>(&jac_batch_kernel<1, true, float, true>)
+                            : reinterpret_cast<const void*>(&jac_batch_kernel<1, true, double, true>);
+    if (ns != 2 || f32) return nullptr;
+    return m.gen_end > 0 ? reinterpret_cast<const void*>(&jac_batch_kernel<2, false, double, true>)
+                         : reinterpret_cast<const void*>(&jac_batch_kernel<2, false, double, false>);
 }
 
-const void* jac_kernel_ptr(int ns, bool f32) {
-    if (ns == 1) return f32 ? reinterpret_cast<const void*>(&jac_batch_kernel<1, true, float>)
-                            : reinterpret_cast<const void*>(&jac_batch_kernel<1, true, double>);
-    return reinterpret_cast<const void*>(&jac_batch_kernel<2, false, double>);
+hipError_t jac_launch(DevMech m, int ns, bool f32, long n, const double* T, const double* P, const double* Y, void* J,
+                      int grid, size_t lds, hipStream_t stream) {
+    const void* kernel = jac_kernel_ptr(m, ns, f32);
+    if (!kernel) return hipErrorInvalidValue;
+    void* args[] = {&m, &n, &T, &P, &Y, &J};
+    return hipLaunchKernel(kernel, dim3(grid), dim3(64), args, lds, stream);
 }
 
 }  // namespace cg

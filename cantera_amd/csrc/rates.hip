@@ -18,8 +18,8 @@ namespace cg {
 
 // From this many states on, several states per wavefront.  Below, the tiles
 // leave SIMDs empty and one state per wavefront ends sooner (us, one state /
-// tiles: gri30 2,048 states 25 / 33, 4,096 35 / 35, 8,192 51 / 36; n-dodecane
-// 2,048 29 / 29, 4,096 42 / 32; h2o2 1,024 15 / 15, 4,096 21 / 15).
+// tiles: gri30 2,048 states 21 / 34, 4,095 28 / 34, 6,144 35 / 36; n-dodecane
+// 2,048 26 / 29, 4,095 38 / 31; h2o2 2,048 14 / 15, 4,095 17 / 15).
 constexpr long kRatesWideMin = 4096;
 // LDS of a wavefront with 8 states: 8 wavefronts share a CU (two per SIMD, as
 // their registers allow); larger mechanisms take 4 states
@@ -28,13 +28,15 @@ constexpr size_t kRatesWideLds = 160 * 1024 / 8;
 namespace {
 
 // At most 168 VGPRs, so that three wavefronts share a SIMD (latency-bound
-// kernel; without the bound the allocator settles at 169 for NS = 1).
-template <int NS, bool kF32>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void rates_kernel(
+// kernel; without the bound the allocator settles at 169 for NS = 1).  The
+// general code would spill 30 of them: two wavefronts there (7
+// pressure-dependent reactions, 2,048 states: 24 -> 20 us).
+template <int NS, bool kF32, bool kGen>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kGen ? 2 : 3))) void rates_kernel(
     DevMech m, long n, const double* __restrict__ T, const double* __restrict__ P, const double* __restrict__ Y,
     double* __restrict__ wdot) {
     const int lane = lane_id();
-    WaveScratch S{};
+    Scratch<kGen> S{};
     bind_species(S, kernarg_mech());
     const XcdStates xs(n);
     for (long st = xs.lo; st < xs.hi; st += xs.step) {
@@ -172,11 +174,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ra
 // Net production rates at the output states of a reactor batch (one record
 // per reactor: the interpolated state [Y, T, m] after the 6 Nordsieck columns,
 // then the control block with P, or V for a constant-volume reactor).
-template <int NS>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void reactor_rates_kernel(
+template <int NS, bool kGen>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kGen ? 2 : 3))) void reactor_rates_kernel(
     DevMech m, long n, const double* __restrict__ rec, size_t stride, int cv, double* __restrict__ wdot) {
     const int lane = lane_id();
-    WaveScratch S{};
+    Scratch<kGen> S{};
     bind_species(S, kernarg_mech());
     constexpr int NP = kWave * NS;
     const XcdStates xs(n);
@@ -206,22 +208,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void re
 
 }  // namespace
 
-hipError_t reactor_rates_launch(const DevMech& m, int ns, long n, const double* rec, size_t stride, int cv,
-                                double* wdot, int grid, size_t lds, hipStream_t stream) {
-    if (ns == 1)
-        hipLaunchKernelGGL((reactor_rates_kernel<1>), dim3(grid), dim3(64), lds, stream, m, n, rec, stride, cv, wdot);
-    else if (ns == 2)
-        hipLaunchKernelGGL((reactor_rates_kernel<2>), dim3(grid), dim3(64), lds, stream, m, n, rec, stride, cv, wdot);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+template <bool kGen>
+static const void* reactor_rates_kernel_of(int ns) {
+    if (ns == 1) return reinterpret_cast<const void*>(&reactor_rates_kernel<1, kGen>);
+    if (ns == 2) return reinterpret_cast<const void*>(&reactor_rates_kernel<2, kGen>);
+    return nullptr;
 }
 
-// state slots per lane of the rate kernels: 1, 2, or 4 for 128 < K + 2 <= 256
-static int rates_ns(int ns) { return ns <= 2 ? ns : 4; }
+const void* reactor_rates_kernel_ptr(const DevMech& m, int ns) {
+    return m.gen_end > 0 ? reactor_rates_kernel_of<true>(ns) : reactor_rates_kernel_of<false>(ns);
+}
 
-const void* reactor_rates_kernel_ptr(int ns) {
-    return ns == 1 ? reinterpret_cast<const void*>(&reactor_rates_kernel<1>)
-                   : reinterpret_cast<const void*>(&reactor_rates_kernel<2>);
+hipError_t reactor_rates_launch(DevMech m, int ns, long n, const double* rec, size_t stride, int cv, double* wdot,
+                                int grid, size_t lds, hipStream_t stream) {
+    const void* kernel = reactor_rates_kernel_ptr(m, ns);
+    if (!kernel) return hipErrorInvalidValue;
+    void* args[] = {&m, &n, &rec, &stride, &cv, &wdot};
+    return hipLaunchKernel(kernel, dim3(grid), dim3(64), args, lds, stream);
+}
+
+// state slots per lane: 1, 2, or 4 for 128 < K + 2 <= 256
+template <bool kF32, bool kGen>
+static const void* rates_kernel_of(int ns) {
+    if (ns == 1) return reinterpret_cast<const void*>(&rates_kernel<1, kF32, kGen>);
+    return ns == 2 ? reinterpret_cast<const void*>(&rates_kernel<2, kF32, kGen>)
+                   : reinterpret_cast<const void*>(&rates_kernel<4, kF32, kGen>);
+}
+
+template <bool kF32>
+static const void* rates_kernel_of(bool gen, int ns, int wide) {
+    if (wide == 8) return reinterpret_cast<const void*>(&rates_wide_kernel<8, kF32>);
+    if (wide == 4) return reinterpret_cast<const void*>(&rates_wide_kernel<4, kF32>);
+    return gen ? rates_kernel_of<kF32, true>(ns) : rates_kernel_of<kF32, false>(ns);
 }
 
 size_t reactor_rates_lds_bytes(const DevMech& m) { return static_cast<size_t>(species_doubles(m.K)) * sizeof(double); }
@@ -230,9 +248,7 @@ static size_t wide_lds(int K, int S) { return static_cast<size_t>(24) * S * (K +
 
 RatesPlan rates_plan(const DevMech& m, int ns, bool f32, long n) {
     RatesPlan p{};
-    if (n >= kRatesWideMin) {
-        p.wide = wide_lds(m.K, 8) <= kRatesWideLds ? 8 : 4;
-    }
+    if (n >= kRatesWideMin) p.wide = wide_lds(m.K, 8) <= kRatesWideLds ? 8 : 4;
     if (p.wide) {
         p.lds = wide_lds(m.K, p.wide);
         p.items = (n + p.wide - 1) / p.wide;
@@ -240,13 +256,8 @@ RatesPlan rates_plan(const DevMech& m, int ns, bool f32, long n) {
         p.lds = reactor_rates_lds_bytes(m);
         p.items = n;
     }
-    switch (p.wide ? 10 * p.wide : rates_ns(ns)) {
-        case 1: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_kernel<1, true>) : reinterpret_cast<const void*>(&rates_kernel<1, false>); break;
-        case 2: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_kernel<2, true>) : reinterpret_cast<const void*>(&rates_kernel<2, false>); break;
-        case 4: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_kernel<4, true>) : reinterpret_cast<const void*>(&rates_kernel<4, false>); break;
-        case 80: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_wide_kernel<8, true>) : reinterpret_cast<const void*>(&rates_wide_kernel<8, false>); break;
-        default: p.kernel = f32 ? reinterpret_cast<const void*>(&rates_wide_kernel<4, true>) : reinterpret_cast<const void*>(&rates_wide_kernel<4, false>); break;
-    }
+    const bool gen = m.gen_end > 0;
+    p.kernel = f32 ? rates_kernel_of<true>(gen, ns, p.wide) : rates_kernel_of<false>(gen, ns, p.wide);
     return p;
 }
 

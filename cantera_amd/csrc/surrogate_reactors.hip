@@ -117,7 +117,7 @@ struct GuardArgs {
 
 static_assert(offsetof(GuardArgs, m) == 0, "GuardArgs must begin with the mechanism");
 
-template <int NS>
+template <int NS, bool kGen>
 __global__ __launch_bounds__(64) void guard_kernel(GuardArgs a) {
     const DevMech& m = a.m;
     const int lane = lane_id();
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64) void guard_kernel(GuardArgs a) {
     L.Y0 = off;  off += kWave * NS;
     L.F0 = off;  off += kWave * NS;
     L.W2 = off;
-    const WaveScratch S = scratch_view(L, kernarg_mech());
+    const Scratch<kGen> S = scratch_view<kGen>(L, kernarg_mech());
     const int N = m.N, K = m.K;
     for (int i = blockIdx.x; i < a.n; i += gridDim.x) {
         if (uni(a.elig[i]) != 1) continue;
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(64) void guard_kernel(GuardArgs a) {
                     if (c < N) S.yb[c] = y0[s];
                 }
                 wave_sync();
-                rhs_call<NS>(kernarg_mech(), L, P);
+                rhs_call<NS, kGen>(kernarg_mech(), L, P);
 #pragma unroll
                 for (int s = 0; s < NS; s++) {
                     const int c = lane + kWave * s;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(64) void guard_kernel(GuardArgs a) {
                 if (c < N) S.yb[c] = y1[s];
             }
             wave_sync();
-            rhs_call<NS>(kernarg_mech(), L, P);
+            rhs_call<NS, kGen>(kernarg_mech(), L, P);
 #pragma unroll
             for (int s = 0; s < NS; s++) {
                 const int c = lane + kWave * s;
@@ -286,8 +286,14 @@ size_t guard_lds_bytes(const DevMech& m, int ns) {
     return d * sizeof(double);
 }
 
-const void* guard_kernel_ptr(int ns) {
-    return ns == 1 ? reinterpret_cast<const void*>(&guard_kernel<1>) : reinterpret_cast<const void*>(&guard_kernel<2>);
+template <bool kGen>
+static const void* guard_kernel_of(int ns) {
+    return ns == 1 ? reinterpret_cast<const void*>(&guard_kernel<1, kGen>)
+                   : reinterpret_cast<const void*>(&guard_kernel<2, kGen>);
+}
+
+const void* guard_kernel_ptr(const DevMech& m, int ns) {
+    return m.gen_end > 0 ? guard_kernel_of<true>(ns) : guard_kernel_of<false>(ns);
 }
 
 hipError_t export_states(int n, const double* rec, size_t stride, int NP, int N, int K, double* Y, hipStream_t s) {
@@ -330,9 +336,8 @@ hipError_t surrogate_guard(const DevMech& m, int ns, int n, int* elig, const dou
     a.gate_T = gate_T;
     for (int j = 0; j < 3; j++) a.rad[j] = rad[j];
     a.counters = counters;
-    if (ns == 1) hipLaunchKernelGGL((guard_kernel<1>), dim3(grid), dim3(64), lds, s, a);
-    else hipLaunchKernelGGL((guard_kernel<2>), dim3(grid), dim3(64), lds, s, a);
-    return hipGetLastError();
+    void* args[] = {&a};
+    return hipLaunchKernel(guard_kernel_ptr(m, ns), dim3(grid), dim3(64), args, lds, s);
 }
 
 }  // namespace cg

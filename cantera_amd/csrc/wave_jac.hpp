@@ -176,8 +176,8 @@ __device__ __forceinline__ void scatter_reaction_derivs(const DevMech& m, int p,
 // the temperature difference, which saves the caller an RHS evaluation.
 // The per-reaction derivatives are accumulated with FP64 global atomics, so
 // their summation order is not fixed.
-template <int NS, bool kRefOrder = false, bool kBaseF0 = false>
-__device__ __forceinline__ void reactor_jacobian(const DevMech& m, const WaveScratch& S, double P, const double (&y)[NS],
+template <int NS, bool kRefOrder = false, bool kBaseF0 = false, bool kGen>
+__device__ __forceinline__ void reactor_jacobian(const DevMech& m, const Scratch<kGen>& S, double P, const double (&y)[NS],
                                  const double (&f0)[NS], double* __restrict__ J) {
     const int lane = lane_id();
     const int K = m.K, N = m.N;
@@ -292,10 +292,10 @@ __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const WaveScr
 }
 
 // Out-of-line Jacobian: expansion point in S.Y0, its RHS in S.F0.
-template <int NS>
+template <int NS, bool kGen>
 __device__ __noinline__ void jac_call(KernargMech* mech, ScratchLayout L, double P, double* J) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const Scratch<kGen> S = scratch_view<kGen>(L, mech);
     const int lane = lane_id();
     double y[NS], f0[NS];
 #pragma unroll
@@ -311,10 +311,10 @@ __device__ __noinline__ void jac_call(KernargMech* mech, ScratchLayout L, double
 // copying the result to Jsave (global, the copy reused while the Jacobian is
 // current).  The LDS pointer is formed here, so the assembly's accesses and
 // atomics are LDS instructions.
-template <int NS>
+template <int NS, bool kGen>
 __device__ __noinline__ void jac_lds_call(KernargMech* mech, ScratchLayout L, double P, int offJ, double* Jsave) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const Scratch<kGen> S = scratch_view<kGen>(L, mech);
     const int lane = lane_id();
     double y[NS], f0[NS];
 #pragma unroll

@@ -203,6 +203,15 @@ struct LaneView {
     }
 };
 
+// The scratch of a kernel for mechanisms with reactions that need the general
+// code (PLOG, Chebyshev, SRI, chemically activated, power-law orders): kGen.
+// The kernels for the others hold none of that code.  With one kernel for both,
+// the general passes a call behind a test of the mechanism, every kernel saved
+// registers around a call that gri30, h2o2 and n-dodecane never make, and the
+// Jacobian kernel of large mechanisms fell to one wavefront per SIMD.
+template <bool kGen>
+struct Scratch : WaveScratch {};
+
 __host__ __device__ __forceinline__ int species_doubles(int K) { return 3 * (K + kDummy); }
 
 // The same scratch as offsets (in doubles) from the start of dynamic LDS, for
@@ -229,9 +238,10 @@ __device__ __forceinline__ void bind_species(WaveScratch& S, KernargMech* mech) 
     S.WD = lds_base() + 2 * (mech->K + kDummy);
 }
 
-__device__ __forceinline__ WaveScratch scratch_view(const ScratchLayout& L, KernargMech* mech) {
+template <bool kGen>
+__device__ __forceinline__ Scratch<kGen> scratch_view(const ScratchLayout& L, KernargMech* mech) {
     double* b = lds_base();
-    WaveScratch S;
+    Scratch<kGen> S;
     bind_species(S, mech);
     S.yb = b + L.yb; S.W2 = b + L.W2; S.F = b + L.F; S.Y0 = b + L.Y0; S.F0 = b + L.F0;
     return S;
@@ -1045,18 +1055,10 @@ __device__ __forceinline__ void species_pass(const DevMech& m, const WaveScratch
 }
 
 // The passes of 64 reactions that hold non-standard reactions (PLOG,
-// Chebyshev, SRI, chemically activated, power-law orders): the general code,
-// out of line so that its registers and hoisted constants burden only the
-// mechanisms that have such reactions.
+// Chebyshev, SRI, chemically activated, power-law orders), by the general code.
 template <bool kF32, bool kPert>
-__device__ __noinline__ void general_passes(KernargMech* mech, double T, double logT,
-                                            double recipT, double logC0, double ctot, double pressure, int pert_rxn,
-                                            double pert_v) {
-    const DevMech m = *(const DevMech*)mech;
-    WaveScratch S{};
-    bind_species(S, mech);
-    GasState g{};
-    g.T = T; g.logT = logT; g.recipT = recipT; g.logC0 = logC0; g.ctot = ctot; g.pressure = pressure;
+__device__ __forceinline__ void general_passes(const DevMech& m, const WaveScratch& S, const GasState& g,
+                                               int pert_rxn, double pert_v) {
     const int lane = lane_id();
     const double kpd = pdep_rate_lane(m, g);
     for (int p = lane; p < min(kWave * m.gen_end, m.I); p += kWave) {
@@ -1085,8 +1087,8 @@ __device__ __noinline__ void general_passes(KernargMech* mech, double T, double 
 // species' terms is the hardware's, not the reference's reaction order.
 // kPert: reaction pert_rxn (permuted index) runs with rate multiplier pert_v.
 // kBlock: elementary passes evaluated side by side.
-template <int NS, bool kF32 = false, bool kPert = false, int kBlock = 3>
-__device__ __forceinline__ void production_rates(const DevMech& m, const WaveScratch& S, const GasState& g,
+template <int NS, bool kF32 = false, bool kPert = false, int kBlock = 3, bool kGen>
+__device__ __forceinline__ void production_rates(const DevMech& m, const Scratch<kGen>& S, const GasState& g,
                                                  SpeciesRegs<NS>& sr, int pert_rxn = -1, double pert_v = 1.0) {
     const int lane = lane_id();
 #pragma unroll
@@ -1095,10 +1097,8 @@ __device__ __forceinline__ void production_rates(const DevMech& m, const WaveScr
         if (k < m.K) S.WD[k] = 0.0;
     }
     wave_sync();
-    if (m.gen_end > 0)
-        general_passes<kF32, kPert>(S.mech, g.T, g.logT, g.recipT, g.logC0, g.ctot,
-                                    g.pressure, pert_rxn, pert_v);
-    standard_passes<kBlock, kF32, kPert, 1>(m, m.rs, LaneView<1>{0u, S.WD}, S.C, g, lane, kWave * m.gen_end,
+    if constexpr (kGen) general_passes<kF32, kPert>(m, S, g, pert_rxn, pert_v);
+    standard_passes<kBlock, kF32, kPert, 1>(m, m.rs, LaneView<1>{0u, S.WD}, S.C, g, lane, kGen ? kWave * m.gen_end : 0,
                                             kWave * m.tb_end, m.I, pert_rxn, pert_v);
     wave_sync();
 #pragma unroll
@@ -1119,8 +1119,8 @@ struct RhsScalars {
 // divided by the left-hand sides as ReactorNet::eval does: ydot for the lane's
 // components (internal order).  y holds [Y_0..Y_{K-1}, T, m] distributed; P is
 // the pressure, or the volume of a constant-volume reactor.
-template <int NS, bool kPert = false>
-__device__ __forceinline__ void reactor_rhs(const DevMech& m, const WaveScratch& S, double P, const double (&y)[NS],
+template <int NS, bool kPert = false, bool kGen>
+__device__ __forceinline__ void reactor_rhs(const DevMech& m, const Scratch<kGen>& S, double P, const double (&y)[NS],
                                             double (&f)[NS], GasState& g, SpeciesRegs<NS>& sr, RhsScalars& rs,
                                             int pert_rxn = -1, double pert_v = 1.0) {
     const int lane = lane_id();
@@ -1168,10 +1168,10 @@ __device__ __forceinline__ void reactor_rhs(const DevMech& m, const WaveScratch&
 // Out-of-line reactor RHS: state taken from S.yb (written by the caller),
 // ydot written to S.F.  One copy of the kinetics code serves every call site of
 // the integrator (smaller code, and the caller keeps little live across it).
-template <int NS>
+template <int NS, bool kGen>
 __device__ __noinline__ void rhs_call(KernargMech* mech, ScratchLayout L, double P) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const Scratch<kGen> S = scratch_view<kGen>(L, mech);
     const int lane = lane_id();
     double y[NS], f[NS];
 #pragma unroll
@@ -1193,10 +1193,10 @@ __device__ __noinline__ void rhs_call(KernargMech* mech, ScratchLayout L, double
 
 // rhs_call with reaction pert_rxn (permuted index) at rate multiplier pert_v:
 // the perturbed right-hand sides of the sensitivity difference quotients.
-template <int NS>
+template <int NS, bool kGen>
 __device__ __noinline__ void rhs_pert_call(KernargMech* mech, ScratchLayout L, double P, int pert_rxn, double pert_v) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const Scratch<kGen> S = scratch_view<kGen>(L, mech);
     const int lane = lane_id();
     double y[NS], f[NS];
 #pragma unroll
@@ -1224,7 +1224,7 @@ __device__ __noinline__ void rhs_pert_call(KernargMech* mech, ScratchLayout L, d
 template <int NS>
 __device__ __noinline__ void loss_frequency_call(KernargMech* mech, ScratchLayout L, double P) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const WaveScratch S = scratch_view<true>(L, mech);
     const int lane = lane_id();
     double y[NS];
 #pragma unroll

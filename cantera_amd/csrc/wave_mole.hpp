@@ -17,8 +17,8 @@ namespace cg {
 // dT/dt = -sum_k wdot_k h_k V / (mass c_p).  Constant volume
 // (IdealGasMoleReactor::updateState / eval, IdealGasMoleReactor.cpp:97-166):
 // rho = mass / V, u_k = h_k - R T and c_v in the energy equation, dV/dt = 0.
-template <int NS>
-__device__ __forceinline__ void mole_rhs(const DevMech& m, const WaveScratch& S, double P, const double (&y)[NS],
+template <int NS, bool kGen>
+__device__ __forceinline__ void mole_rhs(const DevMech& m, const Scratch<kGen>& S, double P, const double (&y)[NS],
                                          double (&f)[NS], GasState& g, SpeciesRegs<NS>& sr, double& vol,
                                          double& totcp) {
     const int lane = lane_id();
@@ -71,10 +71,10 @@ __device__ __forceinline__ void mole_rhs(const DevMech& m, const WaveScratch& S,
 }
 
 // Out-of-line mole RHS: state from S.yb, ydot to S.F (as rhs_call).
-template <int NS>
+template <int NS, bool kGen>
 __device__ __noinline__ void mole_rhs_call(KernargMech* mech, ScratchLayout L, double P) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const Scratch<kGen> S = scratch_view<kGen>(L, mech);
     const int lane = lane_id();
     const int N = m.K + 1 + (m.const_volume ? 1 : 0);
     double y[NS], f[NS];
@@ -107,11 +107,11 @@ __device__ __noinline__ void mole_rhs_call(KernargMech* mech, ScratchLayout L, d
 // efficiency part of d[M]/dC per row in LDS (S.WD); the entries are then
 // written into the value slots of the preconditioner's fill pattern (Js,
 // zero at fill-only slots).
-template <int NS>
+template <int NS, bool kGen>
 __device__ __noinline__ void mole_jac_call(KernargMech* mech, ScratchLayout L, double P, double* __restrict__ Jd,
                                            double* __restrict__ Js, const SparseTables* sp) {
     const DevMech m = *(const DevMech*)mech;
-    const WaveScratch S = scratch_view(L, mech);
+    const Scratch<kGen> S = scratch_view<kGen>(L, mech);
     const int lane = lane_id();
     const int K = m.K, N = K + 1 + (m.const_volume ? 1 : 0);
     const double hshift = m.const_volume ? 1.0 : 0.0;
