@@ -13,7 +13,10 @@
 //
 // One wavefront per state: the Jacobian assembly (two RHS evaluations, at the
 // state and with T + dT, then the per-reaction derivatives), in LDS when it
-// fits, else in the state's output block.
+// fits, else in the state's output block.  Two wavefronts per SIMD: the
+// elementary passes go two side by side (three spill 19 registers).  One
+// n-dodecane state 147 -> 100 us and 12,000 of them 4.59 -> 4.18 ms with the
+// passes over the matrix in blocks (reactor_jacobian).
 #include <hip/hip_runtime.h>
 
 #include "bdf.hpp"
@@ -67,12 +70,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ja
         for (int s = 0; s < NS; s++) f[s] = 0.0;   // not read: the Jacobian takes its own base RHS
         OT* Jg = J + static_cast<size_t>(st) * NN;
         if constexpr (kLdsJ) {
-            reactor_jacobian<NS, true, true>(m, S, Ps, y, f, Jl);
+            reactor_jacobian<NS, true, true, 2>(m, S, Ps, y, f, Jl);
             for (int e = lane; e < NN; e += kWave) Jg[e] = static_cast<OT>(Jl[e]);
             wave_sync();
         } else {
             static_assert(sizeof(OT) == sizeof(double), "in-place assembly needs a double output");
-            reactor_jacobian<NS, true, true>(m, S, Ps, y, f, Jg);
+            reactor_jacobian<NS, true, true, 2>(m, S, Ps, y, f, Jg);
         }
     }
 }

@@ -176,7 +176,7 @@ __device__ __forceinline__ void scatter_reaction_derivs(const DevMech& m, int p,
 // the temperature difference, which saves the caller an RHS evaluation.
 // The per-reaction derivatives are accumulated with FP64 global atomics, so
 // their summation order is not fixed.
-template <int NS, bool kRefOrder = false, bool kBaseF0 = false, bool kGen>
+template <int NS, bool kRefOrder = false, bool kBaseF0 = false, int kBlock = 3, bool kGen>
 __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const Scratch<kGen>& S, double P, const double (&y)[NS],
                                  const double (&f0)[NS], double* __restrict__ J) {
     const int lane = lane_id();
@@ -202,10 +202,10 @@ __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const Scratch
 #pragma unroll
     for (int s = 0; s < NS; s++)
         if (lane + kWave * s == K) y1[s] = Tval + dT;
-    reactor_rhs<NS>(m, S, P, y1, f1, g, sr, rs);
+    reactor_rhs<NS, false, kBlock>(m, S, P, y1, f1, g, sr, rs);
     // base state (species scratch, wdot)
     double fb[NS];
-    reactor_rhs<NS>(m, S, P, y, fb, g, sr, rs);
+    reactor_rhs<NS, false, kBlock>(m, S, P, y, fb, g, sr, rs);
 #pragma unroll
     for (int s = 0; s < NS; s++) dfdT[s] = (f1[s] - (kBaseF0 ? fb[s] : f0[s])) / dT;
 #pragma unroll
@@ -226,17 +226,32 @@ __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const Scratch
     for (int p = lane; p < m.I; p += kWave) scatter_reaction_derivs(m, p, g, S.C, S.MU, kpd, JC, N, acc);
     __threadfence();
     wave_sync();
-    // D_k = sum_l JC[k][l] C_l ; keep wdot and D in W2, h_k in MU
+    // D_k = sum_l JC[k][l] C_l; keep (wdot_k - D_k) / C_tot and W_k in W2, h_k in
+    // MU.  This pass over the matrix and the one below wait once per block of
+    // kRow entries; left to itself the compiler waited for each pair of LDS
+    // reads, and for each entry below
+    constexpr int kRow = 8;
     double hD = 0.0, H = 0.0;
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         int k = lane + kWave * s;
         if (k < K) {
             double d = 0.0;
-            for (int l = 0; l < K; l++) d += JC[k * N + l] * S.C[l];
+            const double* row = JC + k * N;
+            int l = 0;
+            for (; l + kRow <= K; l += kRow) {
+                double a[kRow], c[kRow];
+#pragma unroll
+                for (int b = 0; b < kRow; b++) a[b] = row[l + b];
+#pragma unroll
+                for (int b = 0; b < kRow; b++) c[b] = opaque(S.C[l + b]);
+#pragma unroll
+                for (int b = 0; b < kRow; b++) d += opaque(a[b]) * c[b];
+            }
+            for (; l < K; l++) d += row[l] * S.C[l];
             const double hk = (sr.hrt[s] - hshift) * g.RT;
-            S.W2[k] = sr.wdot[s];
-            S.W2[K + k] = d;
+            S.W2[k] = (sr.wdot[s] - d) / g.ctot;
+            S.W2[K + k] = m.mw[k];
             hD += hk * d;
             H += hk * sr.wdot[s];
         }
@@ -250,7 +265,7 @@ __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const Scratch
         if (k < K) S.MU[k] = (sr.hrt[s] - hshift) * g.RT;
     }
     wave_sync();
-    const double rho = g.dens, Ct = g.ctot, Wbar = g.mmw, cp = rs.cp_mass;
+    const double rho = g.dens, Wbar = g.mmw, cp = rs.cp_mass;
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         int j = lane + kWave * s;
@@ -267,11 +282,24 @@ __device__ __forceinline__ void reactor_jacobian(const DevMech& m, const Scratch
                 const double cvj = kGasConstant * (sr.cpr[s] - 1.0) / wj;
                 rowT[j] = -1.0 / (rho * cp) * (rho * hJ / wj - H * cvj / cp);
             } else {
-                for (int k = 0; k < K; k++) hJ += S.MU[k] * JC[k * N + j];
-                for (int k = 0; k < K; k++) {
-                    const double jc = JC[k * N + j];
-                    JC[k * N + j] = m.mw[k] / wj * (jc + (S.W2[k] - S.W2[K + k]) / Ct);
+                // column j: entry k to W_k / W_j (J_kj + (wdot_k - D_k) / C_tot)
+                const double rwj = 1.0 / wj;
+                auto entry = [&](int k, double jc) {
+                    hJ += S.MU[k] * jc;
+                    const double t = jc + S.W2[k];
+                    return kBaseF0 ? S.W2[K + k] * rwj * t : S.W2[K + k] / wj * t;
+                };
+                int k = 0;
+                for (; k + kRow <= K; k += kRow) {
+                    double v[kRow];
+#pragma unroll
+                    for (int b = 0; b < kRow; b++) v[b] = JC[(k + b) * N + j];
+#pragma unroll
+                    for (int b = 0; b < kRow; b++) v[b] = entry(k + b, opaque(v[b]));
+#pragma unroll
+                    for (int b = 0; b < kRow; b++) JC[(k + b) * N + j] = v[b];
                 }
+                for (; k < K; k++) JC[k * N + j] = entry(k, JC[k * N + j]);
                 const double cpj = kGasConstant * sr.cpr[s] / wj;
                 rowT[j] = -1.0 / (rho * cp) * ((rho * hJ - Wbar * hD + Wbar * H) / wj - H * cpj / cp);
             }

@@ -1119,7 +1119,7 @@ struct RhsScalars {
 // divided by the left-hand sides as ReactorNet::eval does: ydot for the lane's
 // components (internal order).  y holds [Y_0..Y_{K-1}, T, m] distributed; P is
 // the pressure, or the volume of a constant-volume reactor.
-template <int NS, bool kPert = false, bool kGen>
+template <int NS, bool kPert = false, int kBlock = 3, bool kGen>
 __device__ __forceinline__ void reactor_rhs(const DevMech& m, const Scratch<kGen>& S, double P, const double (&y)[NS],
                                             double (&f)[NS], GasState& g, SpeciesRegs<NS>& sr, RhsScalars& rs,
                                             int pert_rxn = -1, double pert_v = 1.0) {
@@ -1134,7 +1134,7 @@ __device__ __forceinline__ void reactor_rhs(const DevMech& m, const Scratch<kGen
     const double mass = uni(S.yb[m.K + 1]);
     const bool cv = m.const_volume;
     species_pass<NS>(m, S, T, P, y, g, sr, cv ? mass / P : 0.0);
-    production_rates<NS, false, kPert>(m, S, g, sr, pert_rxn, pert_v);
+    production_rates<NS, false, kPert, kBlock>(m, S, g, sr, pert_rxn, pert_v);
     const double vol = cv ? P : mass / g.dens;
     const double hshift = cv ? 1.0 : 0.0;   // u_k / RT = h_k / RT - 1
     double e = 0.0, inner = 0.0;

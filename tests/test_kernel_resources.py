@@ -58,7 +58,7 @@ def pick(kernels, pattern):
     (r"\d+rates_kernelILi[12]ELb0ELb0E", 0, 168),
     (r"reactor_rates_kernelILi[12]ELb0E", 0, 168),
     # Jacobians: two wavefronts per SIMD (512 registers of a lane)
-    (r"jac_batch_kernelI", 128, 256),
+    (r"jac_batch_kernelI", 64, 256),
     # integrators of h2o2, gri30 and n-dodecane (their own frames)
     (r"bdf_advance_r16IdLb0ELb0E", 240, 512),
     (r"bdf_advance_lr56IdLb0ELb0E", 280, 512),
