@@ -19,8 +19,13 @@ namespace cg {
 // From this many states on, several states per wavefront.  Below, the tiles
 // leave SIMDs empty and one state per wavefront ends sooner (us, one state /
 // tiles: gri30 2,048 states 21 / 34, 4,095 28 / 34, 6,144 35 / 36; n-dodecane
-// 2,048 26 / 29, 4,095 38 / 31; h2o2 2,048 14 / 15, 4,095 17 / 15).
-constexpr long kRatesWideMin = 4096;
+// 2,048 26 / 29, 4,095 38 / 31).  A mechanism of one pass of reactions has
+// nothing to gain from 64 lanes a state and is past that point once two
+// wavefronts per SIMD, all that the general code's registers allow, are full
+// (h2o2 2,048 14 / 15, 3,072 16 / 15; 7 pressure-dependent reactions 2,048
+// 20 / 19, 3,072 28 / 19).
+constexpr long kRatesWideMin = 4096, kRatesWideMinSmall = 2049;
+constexpr int kRatesSmall = 64;   // reactions
 // LDS of a wavefront with 8 states: 8 wavefronts share a CU (two per SIMD, as
 // their registers allow); larger mechanisms take 4 states
 constexpr size_t kRatesWideLds = 160 * 1024 / 8;
@@ -248,7 +253,8 @@ static size_t wide_lds(int K, int S) { return static_cast<size_t>(24) * S * (K +
 
 RatesPlan rates_plan(const DevMech& m, int ns, bool f32, long n) {
     RatesPlan p{};
-    if (n >= kRatesWideMin) p.wide = wide_lds(m.K, 8) <= kRatesWideLds ? 8 : 4;
+    if (n >= (m.I <= kRatesSmall ? kRatesWideMinSmall : kRatesWideMin))
+        p.wide = wide_lds(m.K, 8) <= kRatesWideLds ? 8 : 4;
     if (p.wide) {
         p.lds = wide_lds(m.K, p.wide);
         p.items = (n + p.wide - 1) / p.wide;
