@@ -14,15 +14,17 @@
 //
 // Layout: inputs and outputs species-major as the batched rates (T[n], P[n],
 // Y[k*n + s]).  One wavefront per state: lane k owns species k (slot s for
-// k = lane + 64 s), with its NASA coefficients and element counts in registers
-// for the whole kernel.  The Newton matrix and right-hand side are entries of
+// k = lane + 64 s), with its element counts and, for one slot, its NASA
+// coefficients in registers for the whole kernel.  The Newton matrix and right-hand side are entries of
 // one contraction G = V^T diag(n) V over the species with V's columns the
 // element counts, 1, h/RT, mu/RT and cp/R (E + 4 <= 12): V goes to LDS and
 // v_mfma_f64_16x16x4f64 sums four species at a time.  The (E+2) x (E+2)
 // system is solved row per lane in registers (RegLinSys).  (As wavefront
 // sums, 36 per iteration for 5 elements, with the system eliminated by one
 // lane in LDS, 20,011 gri30 states took 3.7 ms; HBM traffic is the state in
-// and out.)
+// and out.)  Two wavefronts per SIMD in both registers and LDS: 12,000
+// n-dodecane states TP 1.34 ms, HP 1.51 (one per SIMD 1.85 and 2.08, wavefront
+// sums 1.53 and 2.03).
 #include <hip/hip_runtime.h>
 
 #include "bdf.hpp"
@@ -42,27 +44,33 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
                                                    const double* __restrict__ Pin, const double* __restrict__ Yin,
                                                    double* __restrict__ Tout, double* __restrict__ Yout,
                                                    int* __restrict__ info, int max_iter) {
-    // columns of V: elements 0 .. E-1, then 1, h, mu, cp; odd strides, so that
-    // a column of lanes and a row of columns are both free of bank conflicts
-    constexpr int kCols = 17;
+    // NASA coefficients in registers for one species per lane; for two they come
+    // from L1 each time (28 registers a slot that made it one wavefront per SIMD)
+    constexpr bool kHold = NS == 1;
+    // columns of V: elements 0 .. E-1, then 1, h, mu, cp, then zero; odd strides,
+    // so that a column of lanes and a row of columns are both free of bank
+    // conflicts.  With 15.7 KB for two slots (20.6 with all 16 columns of the
+    // product) LDS leaves room for two wavefronts per SIMD, as the registers do.
+    constexpr int kCols = 13;
     __shared__ double Vs[kWave * NS * kCols];
     __shared__ double ns[kWave * NS];
-    __shared__ double Gs[16 * kCols];
+    __shared__ double Gs[kCols * kCols];
     const int lane = lane_id();
     const int K = m.K, E = m.E;
     const int cOne = E, cH = E + 1, cMu = E + 2, cCp = E + 3;
     const int nu = E + 1 + (hp ? 1 : 0);
     // the lane's species
-    double cl[NS][7], ch[NS][7], tmid[NS], el[NS][kEqMaxE], rmw[NS];
+    double cl[kHold ? NS : 1][7], ch[kHold ? NS : 1][7], tmid[NS], el[NS][kEqMaxE], rmw[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         const int k = lane + kWave * s, kc = min(k, K - 1);
         const double* c16 = m.nasa + 16 * kc;
+        if constexpr (kHold)
 #pragma unroll
-        for (int j = 0; j < 7; j++) {
-            cl[s][j] = c16[j];
-            ch[s][j] = c16[8 + j];
-        }
+            for (int j = 0; j < 7; j++) {
+                cl[s][j] = c16[j];
+                ch[s][j] = c16[8 + j];
+            }
         tmid[s] = c16[7];
         rmw[s] = m.rmw[kc];
 #pragma unroll
@@ -79,8 +87,12 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
     auto thermo = [&](int s, double T, double recipT, double logT, double& cp, double& h, double& g) {
         const bool low = T <= tmid[s];
         double c[7];
+        const double* c7 = m.nasa + 16 * min(lane + kWave * s, K - 1) + (low ? 0 : 8);
 #pragma unroll
-        for (int j = 0; j < 7; j++) c[j] = low ? cl[s][j] : ch[s][j];
+        for (int j = 0; j < 7; j++) {
+            if constexpr (kHold) c[j] = low ? cl[s][j] : ch[s][j];
+            else c[j] = c7[j];
+        }
         const double ct1 = c[1] * T, ct2 = c[2] * (T * T), ct3 = c[3] * (T * T * T), ct4 = c[4] * (T * T * T * T);
         cp = c[0] + ct1 + ct2 + ct3 + ct4;
         h = c[0] + 0.5 * ct1 + 1.0 / 3.0 * ct2 + 0.25 * ct3 + 0.2 * ct4 + c[5] * recipT;
@@ -166,7 +178,7 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
             // n_k, as right operand; two accumulators break the chain
             mfma_d4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
             {
-                const int kq = lane >> 4, lr = lane & 15;
+                const int kq = lane >> 4, lr = min(lane & 15, kCols - 1);   // spare lanes: a zero column
                 for (int k0 = 0; k0 < K; k0 += 8) {   // rows past K are zero
                     const int ka = k0 + kq, kb = k0 + 4 + kq;
                     const double va = Vs[ka * kCols + lr], na = ns[ka], vb = Vs[kb * kCols + lr], nb = ns[kb];
@@ -174,7 +186,8 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
                     acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(vb, nb * vb, acc1, 0, 0, 0);
                 }
 #pragma unroll
-                for (int r = 0; r < 4; r++) Gs[(kq + 4 * r) * kCols + lr] = acc0[r] + acc1[r];
+                for (int r = 0; r < 4; r++)
+                    if (kq + 4 * r < kCols) Gs[(kq + 4 * r) * kCols + lr] = acc0[r] + acc1[r];
             }
             wave_sync();
             RegLinSys<kEqMaxNu, double> ls;

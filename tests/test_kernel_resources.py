@@ -68,3 +68,10 @@ def test_no_general_code(kernels, pattern, scratch, vgprs):
     for k in pick(kernels, pattern):
         assert k[".private_segment_fixed_size"] <= scratch, k[".name"]
         assert k[".vgpr_count"] <= vgprs, k[".name"]
+
+
+def test_equilibrium_two_wavefronts_per_simd(kernels):
+    """Eight wavefronts of a CU in its 160 KB of LDS and 512 registers a lane."""
+    for k in pick(kernels, r"equil_kernelILi[12]E"):
+        assert k[".vgpr_count"] <= 256, k[".name"]
+        assert k[".group_segment_fixed_size"] <= 160 * 1024 // 8, k[".name"]
