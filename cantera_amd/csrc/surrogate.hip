@@ -246,92 +246,126 @@ __global__ void to_bf16_kernel(size_t n, const float* __restrict__ w, uint16_t* 
 // the correction of least D^-1-weighted norm, so species near zero hardly move
 // and sum_k dY_k = 0 follows from element conservation.
 //
-// A wavefront takes 32 rows, two lanes per row, each with every other species:
-// the E x E Gram matrix B D B^T and B dY are sums in the lane's registers, the
-// two halves are added once, and each lane solves its row's (symmetric positive
-// definite) system by elimination (an element absent from the mechanism's
-// species has a zero row and gets lambda = 0).  Rows of y0 and of the output go
-// through LDS, so HBM sees whole lines; the network output is FP32, so the
-// decode is too (sinhf), the increments and the projection are FP64.  (One row
-// per wavefront with E (E + 3) / 2 wavefront sums and the elimination repeated
-// by all 64 lanes took 217 us per 65,536 gri30 rows; this takes 65, of which the
-// 90 MB of rows are 18 at a copy's rate and the rest the FP64 sums and sinhf at
-// a few wavefronts per SIMD.)
-constexpr int kMaxK = 128, kMaxE = 8, kApplyRows = 32;
-template <int EM>   // elements, padded with zero rows
+// A wavefront takes R rows, 64 / R lanes per row: the E x E Gram matrix B D B^T
+// and B dY are sums over the species in the lane's registers, added over a row's
+// lanes, and each lane solves its row's (symmetric positive definite) system by
+// elimination (an element absent from the mechanism's species has a zero row and
+// gets lambda = 0).  Rows of y0 and of the output go through LDS, so HBM sees
+// whole lines; the network output is FP32, so the decode is too (sinhf), the
+// increments and the projection are FP64.
+//
+// R = 8: 65,536 gri30 rows in 38 us (with two lanes per row 65, with a wavefront
+// per row 217), of which the 90 MB of rows are 18 at a copy's rate, one row in 6
+// us instead of the 19 that two lanes need for 53 species.  R = 32 where 8 lanes
+// have fewer than two species each (see launch_apply).  The loads of rows,
+// outputs and tables are in flight together, and sinhf is spread over the 64
+// lanes whatever the number of rows.  A row's result does not depend on R: the
+// species form 8 classes, k mod 8, each summed in order, and the classes are
+// added pairwise, ((0 + 1) + (2 + 3)) + ((4 + 5) + (6 + 7)), by one lane or
+// across lanes.
+constexpr int kMaxK = 128, kMaxE = 8, kClasses = 8;
+template <int EM, int R>   // EM: elements, padded with zero rows
 __global__ __launch_bounds__(64) void apply_kernel(int rows, int N, int K, const double* __restrict__ y0,
                                                    const float* __restrict__ out, const double* __restrict__ norm,
                                                    int in_p, int out_p, const double* __restrict__ comp,
                                                    const double* __restrict__ rmw, int E, double* __restrict__ y1) {
+    constexpr int C = kClasses * R / 64;           // classes per lane: 1 or 4
+    static_assert(C == 1 || C == 4, "rows per wavefront");
     extern __shared__ __attribute__((aligned(16))) double apply_lds[];
-    const int os = out_p + 1;                      // odd row stride
+    const int ds = (K + 1) | 1;                    // odd row stride
     double* const ly = apply_lds;                  // rows of y0
-    double* const lB = ly + kApplyRows * N;        // B_ek, species-major, EM each
-    double* const ld = lB + EM * K;                // mu, sd, sc of each output
-    float* const lo = reinterpret_cast<float*>(ld + 3 * (K + 1));
-    const int lane = threadIdx.x, half = lane / kApplyRows;
-    const int r0 = blockIdx.x * kApplyRows, nr = min(kApplyRows, rows - r0);
+    double* const lB = ly + R * N;                 // B_ek, species-major, EM each
+    double* const ld = lB + EM * K;                // increments of T and Y before the projection
+    const int lane = threadIdx.x, part = lane / R;
+    const int r0 = blockIdx.x * R, nr = min(R, rows - r0);
     const bool project = comp && E >= 1 && E <= kMaxE;
-    // everything through LDS, 8 loads per lane in flight
-    auto stage = [&](int count, auto&& load, auto&& store) {
-        for (int i = lane; i < count; i += 8 * 64) {
-            decltype(load(0)) v[8];
-#pragma unroll
-            for (int b = 0; b < 8; b++) v[b] = load(min(i + 64 * b, count - 1));
-#pragma unroll
-            for (int b = 0; b < 8; b++)
-                if (i + 64 * b < count) store(i + 64 * b, v[b]);
-        }
-    };
+    // the loads of all that goes to LDS are in flight together
+    constexpr int kY = 8, kB = 8;
     const double* yr = y0 + static_cast<size_t>(r0) * N;
+    const int ny = nr * N, nb = project ? K * EM : 0;
+    auto b_entry = [&](int i) { return i % EM < E ? comp[i / EM * E + i % EM] * rmw[i / EM] : 0.0; };
+    double vy[kY], vb[kB];
+#pragma unroll
+    for (int b = 0; b < kY; b++) vy[b] = yr[min(lane + 64 * b, ny - 1)];
+#pragma unroll
+    for (int b = 0; b < kB; b++) vb[b] = nb ? b_entry(min(lane + 64 * b, nb - 1)) : 0.0;
     const float* orow = out + static_cast<size_t>(r0) * out_p;
-    stage(nr * N, [&](int i) { return yr[i]; }, [&](int i, double v) { ly[i] = v; });
-    stage(nr * out_p, [&](int i) { return orow[i]; },
-          [&](int i, float v) { lo[i / out_p * os + i % out_p] = v; });
     const double* par = norm + 2 * in_p;           // mu, sd, sc
-    stage(3 * (K + 1), [&](int i) { return par[(i % 3) * out_p + i / 3]; }, [&](int i, double v) { ld[i] = v; });
-    if (project)
-        stage(K * EM, [&](int i) { return i % EM < E ? comp[i / EM * E + i % EM] * rmw[i / EM] : 0.0; },
-              [&](int i, double v) { lB[i] = v; });
-    __syncthreads();
-    const int row = min(lane % kApplyRows, nr - 1);   // spare lanes repeat the last row
-    double* const y = ly + row * N;
-    float* const o = lo + row * os;
-    double G[EM][EM + 1];
+    const int n_out = K + 1, no = nr * n_out;      // output 0 is T, 1 + k species k
+    for (int i0 = lane; i0 < no; i0 += 64 * 8) {
+        float v[8];
+        double mu[8], sd[8], sc[8];
+        int at[8];
 #pragma unroll
-    for (int a = 0; a < EM; a++)
-#pragma unroll
-        for (int b = 0; b <= EM; b++) G[a][b] = 0.0;
-    // output j = 0 is T, 1 + k species k; half 0 takes the even ones
-    for (int j = half; j <= K; j += 2) {
-        const float sh = sinhf(static_cast<float>(o[j] * ld[3 * j + 1] + ld[3 * j]));
-        o[j] = sh;
-        if (j == 0 || !project) continue;
-        const int k = j - 1;
-        const double dY = ld[3 * j + 2] * static_cast<double>(sh);
-        const double D = fmax(fabs(y[2 + k]), fabs(y[2 + k] + dY)) + 1e-12;
-        double B[EM];
-#pragma unroll
-        for (int a = 0; a < EM; a++) B[a] = lB[k * EM + a];
-#pragma unroll
-        for (int a = 0; a < EM; a++) {
-            const double bd = B[a] * D;
-#pragma unroll
-            for (int b = a; b < EM; b++) G[a][b] += bd * B[b];
-            G[a][EM] += B[a] * dY;
+        for (int b = 0; b < 8; b++) {
+            const int i = min(i0 + 64 * b, no - 1);
+            const int r = static_cast<int>(static_cast<unsigned>(i) / static_cast<unsigned>(n_out)), c = i - r * n_out;
+            v[b] = orow[r * out_p + c];
+            mu[b] = par[c];
+            sd[b] = par[out_p + c];
+            sc[b] = par[2 * out_p + c];
+            at[b] = r * ds + c;
         }
+#pragma unroll
+        for (int b = 0; b < 8; b++)
+            if (i0 + 64 * b < no)
+                ld[at[b]] = sc[b] * static_cast<double>(sinhf(static_cast<float>(v[b] * sd[b] + mu[b])));
     }
+#pragma unroll
+    for (int b = 0; b < kY; b++)
+        if (lane + 64 * b < ny) ly[lane + 64 * b] = vy[b];
+    for (int i = lane + 64 * kY; i < ny; i += 64 * kY) {
+#pragma unroll
+        for (int b = 0; b < kY; b++) vy[b] = yr[min(i + 64 * b, ny - 1)];
+#pragma unroll
+        for (int b = 0; b < kY; b++)
+            if (i + 64 * b < ny) ly[i + 64 * b] = vy[b];
+    }
+#pragma unroll
+    for (int b = 0; b < kB; b++)
+        if (lane + 64 * b < nb) lB[lane + 64 * b] = vb[b];
+    for (int i = lane + 64 * kB; i < nb; i += 64) lB[i] = b_entry(i);
+    __syncthreads();
+    const int row = min(lane % R, nr - 1);         // spare lanes repeat the last row
+    double* const y = ly + row * N;
+    const double* const dy = ld + row * ds;
+    auto weight = [&](int k, double d) { return fmax(fabs(y[2 + k]), fabs(y[2 + k] + d)) + 1e-12; };
     double lam[EM];
 #pragma unroll
     for (int a = 0; a < EM; a++) lam[a] = 0.0;
     if (project) {
+        double G[EM][EM + 1], H[EM][EM + 1];
+        auto each = [&](auto&& f) {
 #pragma unroll
-        for (int a = 0; a < EM; a++)
+            for (int a = 0; a < EM; a++)
 #pragma unroll
-            for (int b = a; b <= EM; b++) {
-                G[a][b] += __shfl_xor(G[a][b], kApplyRows);
-                if (b < EM) G[b][a] = G[a][b];
+                for (int b = a; b <= EM; b++) f(a, b);
+        };
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            double S[EM][EM + 1];
+            each([&](int a, int b) { S[a][b] = 0.0; });
+            for (int k = part * C + c; k < K; k += kClasses) {
+                const double dY = dy[1 + k], D = weight(k, dY);
+                double B[EM];
+#pragma unroll
+                for (int a = 0; a < EM; a++) B[a] = lB[k * EM + a];
+#pragma unroll
+                for (int a = 0; a < EM; a++) {
+                    const double bd = B[a] * D;
+#pragma unroll
+                    for (int b = a; b < EM; b++) S[a][b] += bd * B[b];
+                    S[a][EM] += B[a] * dY;
+                }
             }
+            if (c == 0) each([&](int a, int b) { G[a][b] = S[a][b]; });
+            if (c == 1) each([&](int a, int b) { G[a][b] += S[a][b]; });
+            if (c == 2) each([&](int a, int b) { H[a][b] = S[a][b]; });
+            if (c == 3) each([&](int a, int b) { G[a][b] += H[a][b] + S[a][b]; });
+        }
+#pragma unroll
+        for (int d = R; d < 64; d *= 2) each([&](int a, int b) { G[a][b] += __shfl_xor(G[a][b], d); });
+        each([&](int a, int b) { if (b < EM) G[b][a] = G[a][b]; });
         // elimination without pivoting (SPD); zero rows give lambda = 0
         double rp[EM];
 #pragma unroll
@@ -353,39 +387,34 @@ __global__ __launch_bounds__(64) void apply_kernel(int rows, int N, int K, const
         }
     }
     __syncthreads();   // the spare lanes have read the last row
-    if (lane % kApplyRows < nr)
-        for (int j = half; j <= K; j += 2) {
-            const double d = ld[3 * j + 2] * static_cast<double>(o[j]);
-            if (j == 0) {
-                y[1] += d;
-                continue;
-            }
-            const int k = j - 1;
-            double c = 0.0;
-            if (project) {
+    if (lane % R < nr) {
+        if (part == 0) y[1] += dy[0];
+        for (int c = 0; c < C; c++)
+            for (int k = part * C + c; k < K; k += kClasses) {
+                const double d = dy[1 + k];
+                double s = 0.0;
+                if (project)
 #pragma unroll
-                for (int a = 0; a < EM; a++) c += lB[k * EM + a] * lam[a];
+                    for (int a = 0; a < EM; a++) s += lB[k * EM + a] * lam[a];
+                y[2 + k] += d - weight(k, d) * s;
             }
-            const double D = fmax(fabs(y[2 + k]), fabs(y[2 + k] + d)) + 1e-12;
-            y[2 + k] += d - D * c;
-        }
+    }
     __syncthreads();
     double* const yo = y1 + static_cast<size_t>(r0) * N;
     for (int i = lane; i < nr * N; i += 64) yo[i] = ly[i];
 }
 
+// 32 rows per wavefront for small mechanisms (us per prediction of h2o2, 8 / 32
+// rows: 8,192 rows 26 / 27, 11,904 28 / 28, 32,768 36 / 32, 65,536 51 / 42; gri30
+// and n-dodecane the same with both at 65,536)
+constexpr int kApplySmallK = 16, kApplyMany = 12288;
 void launch_apply(int rows, int N, int K, const double* y0, const float* out, const double* norm, int in_p, int out_p,
                   const double* comp, const double* rmw, int E, double* y1, hipStream_t st) {
-    const int em = E <= 5 ? 5 : kMaxE;
-    const size_t lds = static_cast<size_t>(kApplyRows * N + em * K + 3 * (K + 1)) * sizeof(double) +
-                       static_cast<size_t>(kApplyRows) * (out_p + 1) * sizeof(float);
-    const dim3 grid((rows + kApplyRows - 1) / kApplyRows);
-    if (em == 5)
-        hipLaunchKernelGGL(apply_kernel<5>, grid, dim3(64), lds, st, rows, N, K, y0, out, norm, in_p, out_p, comp, rmw,
-                           E, y1);
-    else
-        hipLaunchKernelGGL(apply_kernel<kMaxE>, grid, dim3(64), lds, st, rows, N, K, y0, out, norm, in_p, out_p, comp, rmw,
-                           E, y1);
+    const int em = E <= 5 ? 5 : kMaxE, R = em == 5 && K <= kApplySmallK && rows > kApplyMany ? 32 : 8;
+    const size_t lds = static_cast<size_t>(R * N + em * K + R * ((K + 1) | 1)) * sizeof(double);
+    auto* const k = R == 32 ? &apply_kernel<5, 32> : em == 5 ? &apply_kernel<5, 8> : &apply_kernel<kMaxE, 8>;
+    hipLaunchKernelGGL(k, dim3((rows + R - 1) / R), dim3(64), lds, st, rows, N, K, y0, out, norm, in_p, out_p, comp,
+                       rmw, E, y1);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw std::runtime_error(std::string("surrogate apply: ") + hipGetErrorString(e));
 }
