@@ -798,9 +798,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, lr = lane & 15, lq = lane >> 4;
     const int r0 = blockIdx.x * kMlpRows;
     // features (see features_kernel): column c of a state gives feature 0 (T,
-    // c = 1), 1 (ln P, in the place of the mass) or c; rows past the end repeat
-    // the last one
-    const int total = kMlpRows * g.N;
+    // c = 1), 1 (ln P, in the place of the mass) or c.  Rows past the end keep
+    // what LDS holds: a row of the operand reaches only its own row of the
+    // result, and theirs are not stored (the features of 64 rows for a single row
+    // of n-dodecane took 10 us)
+    const int nr = min(kMlpRows, g.rows - r0), total = nr * g.N;
     for (int e0 = t; e0 < total; e0 += 4 * 256) {
         double x[4];
         int row[4], col[4];
@@ -810,7 +812,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             row[b] = e / g.N;
             const int c = e - row[b] * g.N;
             col[b] = c < 2 ? 1 - c : c;
-            const size_t s = static_cast<size_t>(min(r0 + row[b], g.rows - 1));
+            const size_t s = static_cast<size_t>(r0 + row[b]);
             x[b] = c == 0 ? g.P[s] : g.y[s * g.N + c];
         }
 #pragma unroll
@@ -821,7 +823,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             act[row[b] * ls + col[b]] = f2bf(static_cast<float>(fmin(fmax(z, -8.0), 8.0)));
         }
     }
-    for (int i = t; i < kMlpRows * (g.in_p - g.N); i += 256) {
+    for (int i = t; i < nr * (g.in_p - g.N); i += 256) {
         const int r = i / (g.in_p - g.N), c = i - r * (g.in_p - g.N);
         act[r * ls + g.N + c] = 0;
     }
