@@ -161,6 +161,7 @@ int32_t guarded(F&& f) {
     } catch (...) {
         g_error = "unknown error";
     }
+    (void)hipGetLastError();   // reported here: not the error of the next call's launches
     return CG_ERR;
 }
 
@@ -241,7 +242,7 @@ void* cg_dev_alloc(int64_t bytes) {
     void* p = nullptr;
     if (bytes <= 0) { g_error = "cg_dev_alloc: size must be positive"; return nullptr; }
     hipError_t e = hipMalloc(&p, static_cast<size_t>(bytes));
-    if (e != hipSuccess) { g_error = std::string("hipMalloc: ") + hipGetErrorString(e); return nullptr; }
+    if (e != hipSuccess) { g_error = std::string("hipMalloc: ") + hipGetErrorString(e); (void)hipGetLastError(); return nullptr; }
     return p;
 }
 int32_t cg_dev_free(void* p) {

@@ -20,7 +20,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // round to nearest even (v_cvt_pk_bf16_f32); NaN stays NaN
 __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(static_cast<uint32_t>(h) << 16); }
 
 // GELU, tanh form (Hendrycks & Gimpel 2016), and its derivative.
 constexpr float kGeluC = 0.7978845608028654f;   // sqrt(2/pi)
@@ -944,9 +943,7 @@ SurrogateNet::SurrogateNet(int K, double dt, int hidden, int depth, uint64_t see
 SurrogateNet::~SurrogateNet() {
     for (void* p : {static_cast<void*>(par_), static_cast<void*>(grad_), static_cast<void*>(m1_),
                     static_cast<void*>(m2_), static_cast<void*>(wb_), static_cast<void*>(norm_),
-                    static_cast<void*>(loss_), static_cast<void*>(part_), static_cast<void*>(act_),
-                    static_cast<void*>(pre_), static_cast<void*>(out_), static_cast<void*>(g_),
-                    static_cast<void*>(idx_)})
+                    static_cast<void*>(loss_)})
         if (p) (void)hipFree(p);
 }
 
@@ -955,35 +952,45 @@ void SurrogateNet::sync_bf16(hipStream_t s) {
     check(hipGetLastError(), "surrogate bf16 copy");
 }
 
-void SurrogateNet::ensure_batch(int rows) {
-    if (rows <= cap_) return;
-    for (void* p : {static_cast<void*>(act_), static_cast<void*>(pre_), static_cast<void*>(out_),
-                    static_cast<void*>(g_), static_cast<void*>(idx_)})
-        if (p) (void)hipFree(p);
-    cap_ = rows;
-    const size_t r = static_cast<size_t>(rows);
-    check(hipMalloc(&act_, r * (s_.in_p + static_cast<size_t>(s_.depth) * s_.hidden) * 2), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&pre_, r * static_cast<size_t>(s_.depth) * s_.hidden * 4), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&out_, r * s_.out_p * 4), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&g_, r * (s_.out_p + static_cast<size_t>(s_.depth) * s_.hidden) * 2), "hipMalloc(surrogate batch)");
-    check(hipMalloc(&idx_, r * 4), "hipMalloc(surrogate batch)");
+DeviceBuffer::~DeviceBuffer() {
+    if (p_) (void)hipFree(p_);
+}
+
+void DeviceBuffer::reserve(size_t bytes) {
+    if (bytes <= bytes_) return;
+    void* old = p_;
+    p_ = nullptr;
+    bytes_ = 0;
+    if (old) check(hipFree(old), "hipFree(surrogate)");
+    check(hipMalloc(&p_, bytes), "hipMalloc(surrogate)");
+    bytes_ = bytes;
+}
+
+void SurrogateNet::reserve_training(int rows) {
+    const size_t r = static_cast<size_t>(rows), deep = static_cast<size_t>(s_.depth) * s_.hidden;
+    act_.reserve(r * (s_.in_p + deep) * 2);
+    pre_.reserve(r * deep * 4);
+    out_.reserve(r * s_.out_p * 4);
+    g_.reserve(r * (s_.out_p + deep) * 2);
+    idx_.reserve(r * 4);
 }
 
 // H_0 = features (already in act_), H_{l+1} = gelu(H_l W_l^T + b_l), out = H_depth W^T + b
 void SurrogateNet::forward(int rows, hipStream_t st) {
     const size_t r = static_cast<size_t>(rows);
+    uint16_t* const act = act_.as<uint16_t>();
     for (int l = 0; l <= s_.depth; l++) {
         const int fi = s_.fan_in(l), fo = s_.fan_out(l);
-        const uint16_t* H = (l == 0) ? act_ : act_ + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
+        const uint16_t* H = (l == 0) ? act : act + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
         EpiArgs e{};
         e.bias = par_ + oB_[l];
         e.ldc = fo;
         if (l < s_.depth) {
-            e.zf = pre_ + r * static_cast<size_t>(l) * s_.hidden;
-            e.hb = act_ + r * (s_.in_p + static_cast<size_t>(l) * s_.hidden);
+            e.zf = pre_.as<float>() + r * static_cast<size_t>(l) * s_.hidden;
+            e.hb = act + r * (s_.in_p + static_cast<size_t>(l) * s_.hidden);
             gemm<kFwdGelu>(rows, fo, fi, H, wb_ + oW_[l], e, st);
         } else {
-            e.zf = out_;
+            e.zf = out_.as<float>();
             gemm<kFwdLinear>(rows, fo, fi, H, wb_ + oW_[l], e, st);
         }
     }
@@ -996,16 +1003,17 @@ double SurrogateNet::backward_and_loss(int rows, const int* idx, const double* y
     const size_t r = static_cast<size_t>(rows);
     // G_depth, then G_{depth-1} .. G_0
     const auto G = [&](int l) {
-        return l == s_.depth ? g_ : g_ + r * (s_.out_p + static_cast<size_t>(s_.depth - 1 - l) * s_.hidden);
+        uint16_t* const g = g_.as<uint16_t>();
+        return l == s_.depth ? g : g + r * (s_.out_p + static_cast<size_t>(s_.depth - 1 - l) * s_.hidden);
     };
     hipLaunchKernelGGL(loss_kernel, dim3(kLossBlocks), dim3(256), 0, st, rows, idx, s_.K + 2, s_.n_out, s_.in_p,
-                       s_.out_p, y0, y1, norm_, out_, G(s_.depth), loss_);
+                       s_.out_p, y0, y1, norm_, out_.as<float>(), G(s_.depth), loss_);
     check(hipGetLastError(), "surrogate loss");
     for (int l = s_.depth; l > 0; l--) {
         // G_{l-1} = (G_l W_l) * gelu'(Z_{l-1})  (rows x fan_in)
         EpiArgs e{};
         e.hb = G(l - 1);
-        e.zin = pre_ + r * static_cast<size_t>(l - 1) * s_.hidden;
+        e.zin = pre_.as<float>() + r * static_cast<size_t>(l - 1) * s_.hidden;
         e.ldc = s_.fan_in(l);
         gemm<kBwdGelu>(rows, s_.fan_in(l), s_.fan_out(l), G(l), wb_ + oW_[l], e, st);
     }
@@ -1018,7 +1026,8 @@ double SurrogateNet::backward_and_loss(int rows, const int* idx, const double* y
         g.oW[l] = oW_[l];
         g.oB[l] = oB_[l];
         g.G[l] = G(l);
-        g.H[l] = (l == 0) ? act_ : act_ + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
+        const uint16_t* act = act_.as<uint16_t>();
+        g.H[l] = (l == 0) ? act : act + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
         g.first[l + 1] = g.first[l] + (g.fo[l] + 63) / 64 * ((g.fi[l] + 63) / 64);
     }
     // at most kGradTiles workgroups of at least 256 rows each (4,096 rows of
@@ -1027,14 +1036,13 @@ double SurrogateNet::backward_and_loss(int rows, const int* idx, const double* y
     const int want = std::max(1, std::min(kGradTiles / tiles, (rows + 255) / 256));
     g.chunk = ((rows + want - 1) / want + 127) / 128 * 128;
     const int splits = (rows + g.chunk - 1) / g.chunk;
-    if (splits > 1 && !part_)
-        check(hipMalloc(&part_, n_par_ * 4 * std::max(1, kGradTiles / tiles)), "hipMalloc(surrogate gradient)");
-    g.part = splits > 1 ? part_ : grad_;
+    if (splits > 1) part_.reserve(n_par_ * 4 * std::max(1, kGradTiles / tiles));
+    g.part = splits > 1 ? part_.as<float>() : grad_;
     hipLaunchKernelGGL(wgrad_kernel, dim3(tiles, splits), dim3(256), 0, st, g);
     check(hipGetLastError(), "surrogate weight gradient");
     const size_t nsum = splits > 1 ? n_par_ : 0;
     hipLaunchKernelGGL(grad_sum_kernel, dim3(static_cast<unsigned>((nsum + 1023) / 1024 + (nsum == 0))), dim3(256), 0, st,
-                       nsum, splits, part_, grad_, loss_);
+                       nsum, splits, part_.as<float>(), grad_, loss_);
     check(hipGetLastError(), "surrogate gradient sum");
     if (update) {
         adam_t_ += 1;
@@ -1098,7 +1106,7 @@ void SurrogateNet::fit_normalization(long n, const double* y0, const double* P, 
 double SurrogateNet::train_epoch(long n, const double* y0, const double* P, const double* y1, int batch, double lr,
                                  hipStream_t st) {
     if (batch < 1) throw std::runtime_error("surrogate: batch must be positive");
-    ensure_batch(batch);
+    reserve_training(batch);
     std::vector<int> perm(n);
     for (long i = 0; i < n; i++) perm[i] = static_cast<int>(i);
     std::mt19937_64 g(rng_++);
@@ -1108,12 +1116,12 @@ double SurrogateNet::train_epoch(long n, const double* y0, const double* P, cons
     long nb = 0;
     for (long b0 = 0; b0 < n; b0 += batch) {
         const int rows = static_cast<int>(std::min<long>(batch, n - b0));
-        check(hipMemcpyAsync(idx_, perm.data() + b0, rows * 4, hipMemcpyHostToDevice, st), "hipMemcpyAsync(idx)");
-        hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, idx_, N, s_.K, y0, P, norm_, s_.in_p,
-                           act_);
+        check(hipMemcpyAsync(idx_.as<int>(), perm.data() + b0, rows * 4, hipMemcpyHostToDevice, st), "hipMemcpyAsync(idx)");
+        hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, idx_.as<int>(), N, s_.K, y0, P,
+                           norm_, s_.in_p, act_.as<uint16_t>());
         check(hipGetLastError(), "surrogate features");
         forward(rows, st);
-        total += backward_and_loss(rows, idx_, y0, y1, true, lr, st);
+        total += backward_and_loss(rows, idx_.as<int>(), y0, y1, true, lr, st);
         nb++;
     }
     return nb ? total / nb : 0.0;
@@ -1122,10 +1130,10 @@ double SurrogateNet::train_epoch(long n, const double* y0, const double* P, cons
 double SurrogateNet::loss_grad(long n, const double* y0, const double* P, const double* y1, float* grad_host,
                                hipStream_t st) {
     const int rows = static_cast<int>(n);
-    ensure_batch(rows);
+    reserve_training(rows);
     const int N = s_.K + 2;
     hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0, P, norm_, s_.in_p,
-                       act_);
+                       act_.as<uint16_t>());
     check(hipGetLastError(), "surrogate features");
     forward(rows, st);
     const double loss = backward_and_loss(rows, nullptr, y0, y1, false, 0.0, st);
@@ -1133,10 +1141,11 @@ double SurrogateNet::loss_grad(long n, const double* y0, const double* P, const 
     return loss;
 }
 
-// The fused kernel for hidden widths of 64, 128, 192 and 256 (weights 16-byte
-// aligned: every width and offset is a multiple of 8 elements); false: not taken.
-bool SurrogateNet::infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t st) const {
-    if (s_.hidden % 64 || s_.hidden > 256 || reinterpret_cast<uintptr_t>(wb_) % 16) return false;
+// The fused kernel takes hidden widths of 64, 128, 192 and 256 (weights are
+// 16-byte aligned: every width and offset is a multiple of 8 elements).
+bool SurrogateNet::fused_shape() const { return s_.hidden % 64 == 0 && s_.hidden <= 256; }
+
+void SurrogateNet::infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t st) const {
     MlpArgs g{};
     g.rows = rows; g.N = s_.K + 2; g.K = s_.K; g.in_p = s_.in_p; g.out_p = s_.out_p; g.depth = s_.depth;
     g.y = y0; g.P = P; g.norm = norm_; g.W = wb_; g.par = par_; g.out = out;
@@ -1152,28 +1161,62 @@ bool SurrogateNet::infer_fused(int rows, const double* y0, const double* P, floa
         case 3: kp = reinterpret_cast<const void*>(&mlp_kernel<3>); break;
         default: kp = reinterpret_cast<const void*>(&mlp_kernel<4>);
     }
-    if (lds > 65536)
-        check(hipFuncSetAttribute(kp, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
-              "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
     void* args[] = {&g};
     check(hipLaunchKernel(kp, dim3((rows + kMlpRows - 1) / kMlpRows), dim3(256), args, lds, st), "surrogate MLP launch");
-    return true;
+}
+
+// Workspace of a row: the FP32 output (out_p) and, layer by layer, features (in_p
+// BF16) and two hidden activations (BF16, ping-pong).
+size_t SurrogateNet::infer_row_bytes() const {
+    return static_cast<size_t>(s_.out_p) * 4 +
+           (fused_shape() ? 0 : static_cast<size_t>(s_.in_p) * 2 + 4 * static_cast<size_t>(s_.hidden));
+}
+
+// y1 of `rows` rows through a workspace for `capacity` of them (every array of it
+// starts at a multiple of 16 bytes: widths are multiples of 16).
+void SurrogateNet::infer(int rows, const double* y0, const double* P, double* y1, unsigned char* workspace,
+                         int capacity, hipStream_t st) const {
+    const int N = s_.K + 2;
+    const size_t r = static_cast<size_t>(capacity);
+    float* const out = reinterpret_cast<float*>(workspace);
+    if (fused_shape()) {
+        infer_fused(rows, y0, P, out, st);
+    } else {
+        uint16_t* const feat = reinterpret_cast<uint16_t*>(out + r * s_.out_p);
+        uint16_t* const ha = feat + r * s_.in_p;
+        uint16_t* const hb = ha + r * s_.hidden;
+        hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0, P, norm_, s_.in_p,
+                           feat);
+        check(hipGetLastError(), "surrogate features");
+        const uint16_t* H = feat;
+        uint16_t* next = ha;
+        for (int l = 0; l <= s_.depth; l++) {
+            const int fi = s_.fan_in(l), fo = s_.fan_out(l);
+            EpiArgs e{};
+            e.bias = par_ + oB_[l];
+            e.ldc = fo;
+            if (l < s_.depth) {
+                e.hb = next;
+                gemm<kFwdGelu>(rows, fo, fi, H, wb_ + oW_[l], e, st);
+                H = next;
+                next = (next == ha) ? hb : ha;
+            } else {
+                e.zf = out;
+                gemm<kFwdLinear>(rows, fo, fi, H, wb_ + oW_[l], e, st);
+            }
+        }
+    }
+    launch_apply(rows, N, s_.K, y0, out, norm_, s_.in_p, s_.out_p, comp_, rmw_, E_, y1, st);
 }
 
 void SurrogateNet::predict(long n, const double* y0, const double* P, double* y1, hipStream_t st) {
     const int N = s_.K + 2;
     const long chunk = 65536;
-    for (long c0 = 0; c0 < n; c0 += chunk) {
-        const int rows = static_cast<int>(std::min(chunk, n - c0));
-        ensure_batch(rows);
-        if (!infer_fused(rows, y0 + c0 * N, P + c0, out_, st)) {
-            hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0 + c0 * N,
-                               P + c0, norm_, s_.in_p, act_);
-            check(hipGetLastError(), "surrogate features");
-            forward(rows, st);
-        }
-        launch_apply(rows, N, s_.K, y0 + c0 * N, out_, norm_, s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N, st);
-    }
+    const int cap = static_cast<int>(std::min(chunk, n));
+    ws_.reserve(cap * infer_row_bytes());
+    for (long c0 = 0; c0 < n; c0 += chunk)
+        infer(static_cast<int>(std::min(chunk, n - c0)), y0 + c0 * N, P + c0, y1 + c0 * N, ws_.as<unsigned char>(), cap,
+              st);
 }
 
 // ---- inference without allocation ------------------------------------------
@@ -1222,40 +1265,9 @@ void SurrogateNet::predict_noalloc(long n, const double* y0, const double* P, do
     if (R < 128)
         throw std::runtime_error("surrogate: network too wide for the 16 MiB inference workspace (fewer than 128 rows)");
     unsigned char* base = static_cast<unsigned char*>(scratch_on_current_device());
-    const size_t r = static_cast<size_t>(R);
-    uint16_t* feat = reinterpret_cast<uint16_t*>(base);
-    uint16_t* ha = reinterpret_cast<uint16_t*>(base + r * s_.in_p * 2);
-    uint16_t* hb = ha + r * s_.hidden;
-    float* out = reinterpret_cast<float*>(base + r * s_.in_p * 2 + 4 * r * s_.hidden);
     const int N = s_.K + 2;
-    for (long c0 = 0; c0 < n; c0 += R) {
-        const int rows = static_cast<int>(std::min<long>(R, n - c0));
-        const bool fused = infer_fused(rows, y0 + c0 * N, P + c0, out, st);
-        if (!fused) {
-            hipLaunchKernelGGL(features_kernel, dim3(rows), dim3(64), 0, st, rows, nullptr, N, s_.K, y0 + c0 * N,
-                               P + c0, norm_, s_.in_p, feat);
-            check(hipGetLastError(), "surrogate features");
-        }
-        const uint16_t* H = feat;
-        uint16_t* next = ha;
-        for (int l = 0; !fused && l <= s_.depth; l++) {
-            const int fi = s_.fan_in(l), fo = s_.fan_out(l);
-            EpiArgs e{};
-            e.bias = par_ + oB_[l];
-            e.ldc = fo;
-            if (l < s_.depth) {
-                e.zf = nullptr;
-                e.hb = next;
-                gemm<kFwdGelu>(rows, fo, fi, H, wb_ + oW_[l], e, st);
-                H = next;
-                next = (next == ha) ? hb : ha;
-            } else {
-                e.zf = out;
-                gemm<kFwdLinear>(rows, fo, fi, H, wb_ + oW_[l], e, st);
-            }
-        }
-        launch_apply(rows, N, s_.K, y0 + c0 * N, out, norm_, s_.in_p, s_.out_p, comp_, rmw_, E_, y1 + c0 * N, st);
-    }
+    for (long c0 = 0; c0 < n; c0 += R)
+        infer(static_cast<int>(std::min<long>(R, n - c0)), y0 + c0 * N, P + c0, y1 + c0 * N, base, R, st);
 }
 
 void SurrogateNet::set_elements(const double* comp, const double* rmw, int E) {

@@ -5,7 +5,8 @@
 // stays the fallback whenever the FP64 guard rejects a surrogate step.
 //
 // Arithmetic: BF16 weights and activations, FP32 accumulation on the matrix
-// cores (v_mfma_f32_16x16x16_bf16), FP32 master weights and Adam moments.
+// cores (v_mfma_f32_16x16x32_bf16; 16x16x16 where a width is no multiple of
+// 32), FP32 master weights and Adam moments.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -27,6 +28,22 @@ struct SurrogateShape {
     int layers() const { return depth + 1; }
     int fan_in(int l) const { return l == 0 ? in_p : hidden; }
     int fan_out(int l) const { return l == depth ? out_p : hidden; }
+};
+
+// Device memory that grows to the largest request.  A request that fails leaves
+// it empty, and the next one allocates anew.
+class DeviceBuffer {
+public:
+    DeviceBuffer() = default;
+    ~DeviceBuffer();
+    DeviceBuffer(const DeviceBuffer&) = delete;
+    DeviceBuffer& operator=(const DeviceBuffer&) = delete;
+    void reserve(size_t bytes);
+    template <class T> T* as() const { return static_cast<T*>(p_); }
+
+private:
+    void* p_ = nullptr;
+    size_t bytes_ = 0;
 };
 
 class SurrogateNet {
@@ -74,9 +91,13 @@ public:
     void set_normalization(const double* host);
 
 private:
-    void ensure_batch(int rows);
+    void reserve_training(int rows);
     void forward(int rows, hipStream_t stream);
-    bool infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t stream) const;
+    bool fused_shape() const;
+    void infer_fused(int rows, const double* y0, const double* P, float* out, hipStream_t stream) const;
+    size_t infer_row_bytes() const;
+    void infer(int rows, const double* y0, const double* P, double* y1, unsigned char* workspace, int capacity,
+               hipStream_t stream) const;
     double backward_and_loss(int rows, const int* idx, const double* y0, const double* y1, bool update, double lr,
                              hipStream_t stream);
     void sync_bf16(hipStream_t stream);
@@ -96,15 +117,15 @@ private:
     const double* rmw_ = nullptr;
     int E_ = 0;
     uint64_t rng_ = 0;
-    // batch workspace
-    int cap_ = 0;
-    uint16_t* act_ = nullptr;       // H_0..H_depth (bf16), rows x width each
-    float* pre_ = nullptr;          // Z_0..Z_{depth-1} (fp32)
-    float* out_ = nullptr;          // rows x out_p
-    uint16_t* g_ = nullptr;         // gradient operands G_depth..G_0 (bf16), rows x width each
-    int* idx_ = nullptr;
     double* loss_ = nullptr;        // the loss, then its parts
-    float* part_ = nullptr;         // gradient copies of the row splits (at most 16 MB, or one)
+    // training batch
+    DeviceBuffer act_;              // H_0..H_depth (bf16), rows x width each
+    DeviceBuffer pre_;              // Z_0..Z_{depth-1} (fp32)
+    DeviceBuffer out_;              // rows x out_p
+    DeviceBuffer g_;                // gradient operands G_depth..G_0 (bf16), rows x width each
+    DeviceBuffer idx_;
+    DeviceBuffer part_;             // gradient copies of the row splits (at most 16 MB, or one)
+    DeviceBuffer ws_;               // inference: infer_row_bytes() per row
 };
 
 }  // namespace cg
