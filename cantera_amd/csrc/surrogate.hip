@@ -611,6 +611,7 @@ __global__ __launch_bounds__(256) void gemm_direct(int M, int N, int K, const ui
 constexpr int kGradTiles = 512;   // workgroups aimed at
 struct GradArgs {
     int rows, chunk;
+    int layer0;                        // the first layer of this launch
     size_t n_par;
     float* part;
     int first[18];                     // first tile of each layer, and their number
@@ -622,7 +623,7 @@ struct GradArgs {
 __global__ __launch_bounds__(256) void wgrad_kernel(GradArgs g) {
     __shared__ float sum[4][16][64];   // one row of tiles of each wavefront
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
-    int l = 0;
+    int l = g.layer0;
     while (static_cast<int>(blockIdx.x) >= g.first[l + 1]) l++;
     const int fo = g.fo[l], fi = g.fi[l], tile = blockIdx.x - g.first[l], tn = (fi + 63) / 64;
     const int m0 = tile / tn * 64, n0 = tile % tn * 64, m = m0 + 4 * lr, n = n0 + 4 * lr;
@@ -966,12 +967,23 @@ void DeviceBuffer::reserve(size_t bytes) {
     bytes_ = bytes;
 }
 
+// Gradient operands held at a time: one launch computes the weight gradients of
+// as many layers as 256 MB of operands hold (all of them up to 123,361 rows of 4 x
+// 256), at least two, for a layer's operand is made from the next one's.  With
+// every layer's operand held, 1,048,576 rows of 16 x 1,024 had 30 GB more to find
+// than with two.
+constexpr size_t kHeldBytes = size_t{256} << 20;
+int SurrogateNet::held_operands(int rows) const {
+    const size_t n = kHeldBytes / (static_cast<size_t>(rows) * std::max(s_.out_p, s_.hidden) * 2);
+    return static_cast<int>(std::min(std::max<size_t>(n, 2), static_cast<size_t>(s_.layers())));
+}
+
 void SurrogateNet::reserve_training(int rows) {
     const size_t r = static_cast<size_t>(rows), deep = static_cast<size_t>(s_.depth) * s_.hidden;
     act_.reserve(r * (s_.in_p + deep) * 2);
     pre_.reserve(r * deep * 4);
     out_.reserve(r * s_.out_p * 4);
-    g_.reserve(r * (s_.out_p + deep) * 2);
+    g_.reserve(held_operands(rows) * r * std::max(s_.out_p, s_.hidden) * 2);
     idx_.reserve(r * 4);
 }
 
@@ -996,16 +1008,52 @@ void SurrogateNet::forward(int rows, hipStream_t st) {
     }
 }
 
+// Weight and bias gradients of layers l0 .. l1 into grad_ (and loss_[0]); G(l): the
+// gradient operand of layer l's outputs.
+template <class F>
+void SurrogateNet::weight_gradients(int rows, int l0, int l1, F&& G, hipStream_t st) {
+    const size_t r = static_cast<size_t>(rows);
+    GradArgs g{};
+    g.rows = rows;
+    g.layer0 = l0;
+    const size_t base = oW_[l0];
+    g.n_par = (l1 == s_.depth ? n_par_ : oW_[l1 + 1]) - base;
+    for (int l = l0; l <= l1; l++) {
+        g.fo[l] = s_.fan_out(l);
+        g.fi[l] = s_.fan_in(l);
+        g.oW[l] = oW_[l] - base;
+        g.oB[l] = oB_[l] - base;
+        g.G[l] = G(l);
+        const uint16_t* act = act_.as<uint16_t>();
+        g.H[l] = (l == 0) ? act : act + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
+        g.first[l + 1] = g.first[l] + (g.fo[l] + 63) / 64 * ((g.fi[l] + 63) / 64);
+    }
+    // at most kGradTiles workgroups of at least 256 rows each (4,096 rows of
+    // 4 x 256: 131 us per gradient with 512, 139 with 1,024 or 2,048)
+    const int tiles = g.first[l1 + 1];
+    const int want = std::max(1, std::min(kGradTiles / tiles, (rows + 255) / 256));
+    g.chunk = ((rows + want - 1) / want + 127) / 128 * 128;
+    const int splits = (rows + g.chunk - 1) / g.chunk;
+    if (splits > 1) part_.reserve(g.n_par * 4 * std::max(1, kGradTiles / tiles));
+    g.part = splits > 1 ? part_.as<float>() : grad_ + base;
+    hipLaunchKernelGGL(wgrad_kernel, dim3(tiles, splits), dim3(256), 0, st, g);
+    check(hipGetLastError(), "surrogate weight gradient");
+    const size_t nsum = splits > 1 ? g.n_par : 0;
+    hipLaunchKernelGGL(grad_sum_kernel, dim3(static_cast<unsigned>((nsum + 1023) / 1024 + (nsum == 0))), dim3(256), 0, st,
+                       nsum, splits, part_.as<float>(), grad_ + base, loss_);
+    check(hipGetLastError(), "surrogate gradient sum");
+}
+
 // loss of out_ against the pairs (rows idx, or all), gradient into grad_,
 // optional Adam step
 double SurrogateNet::backward_and_loss(int rows, const int* idx, const double* y0, const double* y1, bool update,
                                        double lr, hipStream_t st) {
     const size_t r = static_cast<size_t>(rows);
-    // G_depth, then G_{depth-1} .. G_0
-    const auto G = [&](int l) {
-        uint16_t* const g = g_.as<uint16_t>();
-        return l == s_.depth ? g : g + r * (s_.out_p + static_cast<size_t>(s_.depth - 1 - l) * s_.hidden);
+    const int held = held_operands(rows);
+    const auto G = [&](int l) {   // in turn, from G_depth to G_0
+        return g_.as<uint16_t>() + static_cast<size_t>((s_.depth - l) % held) * r * std::max(s_.out_p, s_.hidden);
     };
+    int top = s_.depth;           // the layers above are done
     hipLaunchKernelGGL(loss_kernel, dim3(kLossBlocks), dim3(256), 0, st, rows, idx, s_.K + 2, s_.n_out, s_.in_p,
                        s_.out_p, y0, y1, norm_, out_.as<float>(), G(s_.depth), loss_);
     check(hipGetLastError(), "surrogate loss");
@@ -1016,34 +1064,13 @@ double SurrogateNet::backward_and_loss(int rows, const int* idx, const double* y
         e.zin = pre_.as<float>() + r * static_cast<size_t>(l - 1) * s_.hidden;
         e.ldc = s_.fan_in(l);
         gemm<kBwdGelu>(rows, s_.fan_in(l), s_.fan_out(l), G(l), wb_ + oW_[l], e, st);
+        // the operand of layer `top` makes place for that of l - 2
+        if (top - (l - 1) + 1 == held && l > 1) {
+            weight_gradients(rows, l - 1, top, G, st);
+            top = l - 2;
+        }
     }
-    GradArgs g{};
-    g.rows = rows;
-    g.n_par = n_par_;
-    for (int l = 0; l < s_.layers(); l++) {
-        g.fo[l] = s_.fan_out(l);
-        g.fi[l] = s_.fan_in(l);
-        g.oW[l] = oW_[l];
-        g.oB[l] = oB_[l];
-        g.G[l] = G(l);
-        const uint16_t* act = act_.as<uint16_t>();
-        g.H[l] = (l == 0) ? act : act + r * (s_.in_p + static_cast<size_t>(l - 1) * s_.hidden);
-        g.first[l + 1] = g.first[l] + (g.fo[l] + 63) / 64 * ((g.fi[l] + 63) / 64);
-    }
-    // at most kGradTiles workgroups of at least 256 rows each (4,096 rows of
-    // 4 x 256: 131 us per gradient with 512, 139 with 1,024 or 2,048)
-    const int tiles = g.first[s_.layers()];
-    const int want = std::max(1, std::min(kGradTiles / tiles, (rows + 255) / 256));
-    g.chunk = ((rows + want - 1) / want + 127) / 128 * 128;
-    const int splits = (rows + g.chunk - 1) / g.chunk;
-    if (splits > 1) part_.reserve(n_par_ * 4 * std::max(1, kGradTiles / tiles));
-    g.part = splits > 1 ? part_.as<float>() : grad_;
-    hipLaunchKernelGGL(wgrad_kernel, dim3(tiles, splits), dim3(256), 0, st, g);
-    check(hipGetLastError(), "surrogate weight gradient");
-    const size_t nsum = splits > 1 ? n_par_ : 0;
-    hipLaunchKernelGGL(grad_sum_kernel, dim3(static_cast<unsigned>((nsum + 1023) / 1024 + (nsum == 0))), dim3(256), 0, st,
-                       nsum, splits, part_.as<float>(), grad_, loss_);
-    check(hipGetLastError(), "surrogate gradient sum");
+    if (top >= 0) weight_gradients(rows, 0, top, G, st);
     if (update) {
         adam_t_ += 1;
         const float c1 = 1.f - std::pow(0.9f, static_cast<float>(adam_t_));

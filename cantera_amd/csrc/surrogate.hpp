@@ -91,6 +91,7 @@ public:
     void set_normalization(const double* host);
 
 private:
+    int held_operands(int rows) const;
     void reserve_training(int rows);
     void forward(int rows, hipStream_t stream);
     bool fused_shape() const;
@@ -100,6 +101,8 @@ private:
                hipStream_t stream) const;
     double backward_and_loss(int rows, const int* idx, const double* y0, const double* y1, bool update, double lr,
                              hipStream_t stream);
+    template <class F>
+    void weight_gradients(int rows, int l0, int l1, F&& G, hipStream_t stream);
     void sync_bf16(hipStream_t stream);
 
     SurrogateShape s_{};
@@ -122,7 +125,7 @@ private:
     DeviceBuffer act_;              // H_0..H_depth (bf16), rows x width each
     DeviceBuffer pre_;              // Z_0..Z_{depth-1} (fp32)
     DeviceBuffer out_;              // rows x out_p
-    DeviceBuffer g_;                // gradient operands G_depth..G_0 (bf16), rows x width each
+    DeviceBuffer g_;                // gradient operands G_depth..G_0 (bf16), rows x the larger width each, in turn
     DeviceBuffer idx_;
     DeviceBuffer part_;             // gradient copies of the row splits (at most 16 MB, or one)
     DeviceBuffer ws_;               // inference: infer_row_bytes() per row

@@ -62,3 +62,46 @@ def test_a_failed_request_leaves_the_net_usable(gri30):
         assert again == loss
         np.testing.assert_array_equal(g, grad)
     np.testing.assert_array_equal(sur.predict(y0, P), pred)
+
+
+def test_gradient_of_more_layers_than_are_held():
+    """Above 256 MB the layers' gradient operands take turns.  Twice the rows:
+    the mean loss and its gradient are the means over the halves, which are below
+    that size; factors of 2 are exact in BF16, so only the order of FP32 sums of
+    16,384 terms differs (random signs: 128 roundings, 8e-6 of the terms' norm,
+    within a factor of 10 of the sum's)."""
+    import cantera_amd as ca
+    from cantera_amd.surrogate import Surrogate
+    from cantera_amd.workloads import MechInfo
+    sol = ca.Solution("h2o2")
+    hidden, depth, n = 512, 16, 16384
+    y0, P, y1 = synthetic_pairs(MechInfo(mech_file("h2o2")), n, 5)
+    sur = Surrogate(sol, dt=1e-6, hidden=hidden, depth=depth, seed=1)
+    sur.fit_normalization(y0, P, y1)
+    halves = [sur.loss_grad(y0[s], P[s], y1[s]) for s in (slice(0, n // 2), slice(n // 2, n))]
+    loss, grad = sur.loss_grad(y0, P, y1)
+    assert abs(loss - (halves[0][0] + halves[1][0]) / 2) <= 1e-6 * loss
+    mean = (halves[0][1].astype(np.float64) + halves[1][1]) / 2
+    widths = [64] + [hidden] * depth + [64]
+    off = 0
+    for fi, fo in zip(widths, widths[1:]):
+        a, b = grad[off:off + fo * fi + fo].astype(np.float64), mean[off:off + fo * fi + fo]
+        assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b)
+        off += fo * fi + fo
+
+
+def test_gradient_operands_are_bounded(gri30):
+    """Activations and pre-activations of every layer, outputs, and at most 256
+    MB of gradient operands, not one of every layer (1.1 GB here)."""
+    from cantera_amd._lib import check, lib
+    from cantera_amd.surrogate import DeviceArray, Surrogate
+    sol, (y0, P, y1) = gri30
+    hidden, depth, n = 512, 16, 65536
+    sur = Surrogate(sol, dt=1e-6, hidden=hidden, depth=depth, seed=1)
+    sur.fit_normalization(y0, P, y1)
+    sur.loss_grad(y0[:64], P[:64], y1[:64])   # code objects loaded
+    d0, dP, d1 = (DeviceArray(np.tile(x, (16,) + (1,) * (x.ndim - 1))) for x in (y0, P, y1))
+    before = free_bytes()
+    check(lib().cg_surrogate_loss_grad(sur.handle, n, d0.ptr, dP.ptr, d1.ptr, None, None))
+    partial = 3 * 4 * sur.n_params            # gradient copies of row splits, few at this size
+    assert before - free_bytes() <= n * (6 * depth * hidden + 2 * 64 + 8 * 64) + (256 << 20) + partial + (32 << 20)
