@@ -10,7 +10,7 @@ from conftest import mech_file
 
 pytestmark = pytest.mark.gpu
 
-WIDE = 4096     # states from which the wide kernel runs
+WIDE = 4096     # from here every mechanism's states go several to a wavefront, below 2,049 none's
 MECHS = ["h2o2", "gri30", "nDodecane", "noxNeg", "pdep-test", "sri-falloff", "tsang-falloff",
          "chemically-activated-reaction", "frac", "gri30_ndodecane"]
 
