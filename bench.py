@@ -564,7 +564,7 @@ def surrogate_block(a, sol, wl, steps):
         "inference_roofline": {"bound": "mfma", "pipe": "BF16 MFMA (dense 2.5 PFLOP/s)", "achieved": achieved,
                                "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / BF16_PEAK_TFLOPS,
                                "avg_launch_ms": inf_s * 1e3, "flops_per_launch": n * flop_fwd,
-                               "kernel": "gemm_nt_bf16 (features, 5 GEMMs, decode + element projection)"},
+                               "kernel": "mlp_kernel (features and layers), apply_kernel (decode + element projection)"},
     }
 
 
@@ -638,13 +638,13 @@ def batch_kernel_result(a, kind, precision, n=None, steps=None, warmup=None, cpu
         alg_bytes = n * (8 * (2 + K) + es * N * N)
         roof = {"bound": "hbm", "achieved": alg_bytes / avg_s / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": alg_bytes / avg_s / 1e9 / HBM_PEAK_GBS, "traffic": measured_traffic(name, n),
-                "kernel": "jac_batch_kernel", "avg_launch_ms": avg_s * 1e3, "bytes_per_launch": alg_bytes}
+                "kernel": "jac_tile_kernel", "avg_launch_ms": avg_s * 1e3, "bytes_per_launch": alg_bytes}
         metric = f"gri30 reactor Jacobians/s ({'FP32' if f32 else 'FP64'} output, 55x55 dense per state)"
     else:
         flops = n * F_rates
         roof = {"bound": "valu", "pipe": VALU_PIPE, "achieved": flops / avg_s / 1e12, "peak": FP64_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": flops / avg_s / 1e12 / FP64_PEAK_TFLOPS,
-                "traffic": measured_traffic(name, n), "kernel": "rates_kernel", "avg_launch_ms": avg_s * 1e3,
+                "traffic": measured_traffic(name, n), "kernel": "rates_wide_kernel", "avg_launch_ms": avg_s * 1e3,
                 "flops_per_launch": flops, "hbm_bytes_algorithmic": n * 8 * (2 + 2 * K),
                 "hbm_frac": n * 8 * (2 + 2 * K) / avg_s / 1e9 / HBM_PEAK_GBS}
         metric = "gri30 net production rates, states/s (" + ("FP32 rate constants" if f32 else "FP64") + ")"

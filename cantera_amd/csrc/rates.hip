@@ -76,7 +76,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kGen ? 2 : 3
 // 64 lanes to serve 29.  With S = 8 only 8 lanes share an accumulator, 50
 // falloff and three-body reactions take 7 passes of 8 states instead of one of
 // each, and a tile reads and writes whole 64-byte lines.  1,048,576 gri30
-// states: 4.50 -> 2.40 ms (FP64 VALU at 60% of its issue rate: 855
+// states: 4.50 -> 2.44 ms (FP64 VALU at 62% of its issue rate: 872
 // instructions a state); S = 16 leaves room for 7 wavefronts per CU (3.02 ms),
 // S = 4 has more lanes per accumulator (2.83 ms).  30,011 n-dodecane states,
 // FP32 constants: 213 -> 138 us with S = 4, 141 us with S = 8.  1/W_bar and [M]
