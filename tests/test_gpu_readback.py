@@ -30,3 +30,30 @@ def test_readback_is_exact_around_a_pass(n):
     np.testing.assert_array_equal(ctl[:, 45], P)
     assert not rb.status.any()
     assert not rb.stats["steps"].any()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 300])
+def test_reads_wait_for_a_queued_advance(n):
+    """State, status and counters read right behind an asynchronous advance (one
+    row is copied as it lies, more are packed first)."""
+    sol = ca.Solution("h2o2")
+    X = np.tile([2.0 if s == "H2" else 1.0 if s == "O2" else 0.0 for s in sol.species_names], (n, 1))
+    T, P, Y = np.linspace(1000.0, 1300.0, n), np.full(n, 101325.0), sol.mass_fractions_from_moles(X)
+    want = ca.ReactorBatch(sol, T, P, Y)
+    want.advance(np.full(n, 1e-4))
+    assert ca.lib().cg_device_synchronize() == 0
+    steps, y = want.stats["steps"], want.state
+    assert (steps > 0).all() and not want.status.any()
+    t = DeviceArray(np.full(n, 1e-4))
+    for read, ref in (("state", y), ("stats", steps), ("status", np.zeros(n))):
+        rb = ca.ReactorBatch(sol, T, P, Y)
+        rb.advance_device(t)
+        got = getattr(rb, read)
+        np.testing.assert_array_equal(got["steps"] if read == "stats" else got, ref)
+    ctl = np.empty((n, 64))
+    assert ca.lib().cg_reactors_get_control(want.handle, ctl) == 0
+    np.testing.assert_array_equal(ctl[:, 45], P)
+    dev = DeviceArray.empty((n, want.neq))
+    want.state_to_device(dev)
+    assert ca.lib().cg_device_synchronize() == 0
+    np.testing.assert_array_equal(dev.get(), y)
