@@ -19,16 +19,16 @@
 // one contraction G = V^T diag(n) V over the species with V's columns the
 // element counts, 1, h/RT, mu/RT and cp/R (E + 4 <= 12): V goes to LDS and
 // v_mfma_f64_16x16x4f64 sums four species at a time.  The (E+2) x (E+2)
-// system is solved row per lane in registers (RegLinSys).  (As wavefront
+// system is solved row per lane in registers (solve_rows).  (As wavefront
 // sums, 36 per iteration for 5 elements, with the system eliminated by one
 // lane in LDS, 20,011 gri30 states took 3.7 ms; HBM traffic is the state in
 // and out.)  Two wavefronts per SIMD in both registers and LDS: 12,000
-// n-dodecane states TP 1.34 ms, HP 1.51 (one per SIMD 1.85 and 2.08, wavefront
+// n-dodecane states TP 1.36 ms, HP 1.54 (one per SIMD 1.85 and 2.08, wavefront
 // sums 1.53 and 2.03).
 #include <hip/hip_runtime.h>
 
 #include "bdf.hpp"
-#include "linsys.hpp"
+#include "wave_linalg.hpp"
 
 namespace cg {
 
@@ -38,6 +38,57 @@ constexpr int kEqMaxE = 8;
 constexpr int kEqMaxNu = kEqMaxE + 2;
 constexpr double kSize = 18.420681;       // ln(1e8): trace-species threshold of eq. 3.2
 constexpr double kTraceLn = 9.2103404;    // ln(1e4)
+
+// x <- A^-1 x, row q of A and of x in lane q < nu; false where A is singular.
+// Gaussian elimination with the exact largest pivot of a column (the first of
+// equal ones, counted along the rows as exchanged) and with quotients by it: an
+// iterate of almost one species makes element rows multiples of each other, and
+// a quotient keeps the zero that they cancel to.  With products by 1 / pivot and
+// pivots compared in 58 bits that zero became a pivot of rounding noise or not
+// as it fell, and 0.07% of hydrogen mixtures at 200 to 500 K were refused that
+// are not now.  20,011 gri30 states 1.99 -> 2.04 ms for it.
+__device__ __forceinline__ bool solve_rows(double (&a)[kEqMaxNu], double& x, int nu) {
+    const int lane = lane_id();
+    int pos = lane;   // where the exchanges have brought this lane's row
+    double pivot = 1.0;
+    int owner[kEqMaxNu];
+#pragma unroll
+    for (int c = 0; c < kEqMaxNu; c++) {
+        owner[c] = 0;
+        if (c >= nu) continue;
+        const double v = (lane < nu && pos >= c) ? fabs(a[c]) : -1.0;
+        double top = fmax(v, dpp_f64<0xB1>(v));
+        top = fmax(top, dpp_f64<0x4E>(top));
+        top = fmax(top, dpp_f64<0x124>(top));
+        top = readlane_f64(fmax(top, dpp_f64<0x128>(top)), 0);
+        unsigned long long same = __ballot(v == top);
+        if (!(top > 0.0) || same == 0) return false;
+        int p = __builtin_ctzll(same), pp = __builtin_amdgcn_readlane(pos, p);
+        for (same &= same - 1; same; same &= same - 1) {
+            const int q = __builtin_ctzll(same), qp = __builtin_amdgcn_readlane(pos, q);
+            if (qp < pp) { p = q; pp = qp; }
+        }
+        pos = lane == p ? c : (pos == c ? pp : pos);
+        owner[c] = p;
+        pivot = lane == p ? a[c] : pivot;
+        const double q = a[c] / readlane_f64(a[c], p);
+        const double f = lane < nu && pos > c ? q : 0.0;
+#pragma unroll
+        for (int j = c + 1; j < kEqMaxNu; j++) a[j] -= f * readlane_f64(a[j], p);
+        x -= f * readlane_f64(x, p);
+    }
+    const double rdiag = 1.0 / pivot;
+    double y = 0.0;
+#pragma unroll
+    for (int c = kEqMaxNu - 1; c >= 0; c--) {
+        if (c >= nu) continue;
+        const double xc = readlane_f64(x * rdiag, owner[c]);
+        x -= (pos < c ? a[c] : 0.0) * xc;
+        y = lane == c ? xc : y;
+    }
+    x = y;
+    return true;
+}
 
 template <int NS>
 __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, const double* __restrict__ Tin,
@@ -190,7 +241,7 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
                     if (kq + 4 * r < kCols) Gs[(kq + 4 * r) * kCols + lr] = acc0[r] + acc1[r];
             }
             wave_sync();
-            RegLinSys<kEqMaxNu, double> ls;
+            double a[kEqMaxNu];
             const int row = min(lane, nu - 1);
             const double sumn = uni(Gs[cOne * kCols + cOne]);
 #pragma unroll
@@ -201,7 +252,7 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
                     v += (lane == cH) ? Gs[cOne * kCols + cCp] : 0.0;
                 }
                 // an element that the state lacks: 1 on the diagonal, 0 elsewhere
-                ls.a[j] = (lane < nu && j < nu) ? (row_on ? v : (j == lane ? 1.0 : 0.0)) : 0.0;
+                a[j] = (lane < nu && j < nu) ? (row_on ? v : (j == lane ? 1.0 : 0.0)) : 0.0;
             }
             double x;
             {
@@ -209,8 +260,7 @@ __global__ __launch_bounds__(64) void equil_kernel(DevMech m, long n, int hp, co
                 const double lead = elem ? bq0 : (lane == cOne ? ntot : h0 / (kGasConstant * T));
                 x = row_on ? lead - gone + gmu : 0.0;
             }
-            const bool ok = ls.factor(nu);
-            if (ok) x = ls.solve(x, nu);
+            const bool ok = solve_rows(a, x, nu);
             if (!ok || __any(lane < nu && !(x == x))) { status = -3; break; }
             const double dlnN = readlane_f64(x, cOne), dlnT = hp ? readlane_f64(x, cH) : 0.0;
             double pi[kEqMaxE];

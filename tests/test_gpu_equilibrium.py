@@ -104,3 +104,34 @@ def test_bad_mode_and_inputs():
         sol.equilibrate([1000.0, 1000.0], ONE_ATM, Y, mode="UV")
     with pytest.raises(ca.CanteraGpuError, match="temperature"):
         sol.equilibrate([1000.0, -5.0], ONE_ATM, Y)
+
+
+def test_cold_hydrogen_states_that_the_oracle_accepts(oracle_mod):
+    """Iterates of almost one species make element rows multiples of each other:
+    the zeros they cancel to have to stay zeros, or states are refused as the
+    rounding falls (a few in ten thousand).  Major species to 1e-10."""
+    import cantera_amd as ca
+    from cantera_amd.surrogate import DeviceArray
+    n, sol = 16384, ca.Solution("h2o2")
+    g = np.random.default_rng(11)
+    T, P = g.uniform(200.0, 500.0, n), ONE_ATM * np.exp(g.uniform(np.log(0.1), np.log(50.0), n))
+    X = 10.0 ** g.uniform(-12.0, -2.0, (sol.n_species, n))
+    for name, x in (("H2", 2.0 * g.uniform(0.3, 3.0, n)), ("O2", 1.0), ("N2", 3.76)):
+        X[sol.species_index(name)] = x
+    Y = X * sol.molecular_weights[:, None]
+    Y /= Y.sum(axis=0)
+    d = [DeviceArray(v) for v in (T, P, Y, np.zeros(n), np.zeros_like(Y), np.zeros(n, dtype=np.int32))]
+    assert ca.lib().cg_equilibrate_batch_device(sol.handle, n, b"TP", *(v.ptr for v in d), 500, None) == 0
+    assert ca.lib().cg_device_synchronize() == 0
+    Ye, info = d[4].get(), d[5].get()
+    om = oracle_mod.Mech(mech_file("h2o2"))
+    accepted = 0
+    for i in range(n):
+        try:
+            _, Yo, _ = om.equilibrate(T[i], P[i], np.ascontiguousarray(Y[:, i]), mode="TP")
+        except RuntimeError:
+            continue
+        accepted += 1
+        assert info[i] >= 0, (i, T[i], P[i])
+        np.testing.assert_allclose(Ye[:, i], Yo, rtol=0.0, atol=1e-10)
+    assert accepted > n // 2
