@@ -23,7 +23,7 @@
 // sums, 36 per iteration for 5 elements, with the system eliminated by one
 // lane in LDS, 20,011 gri30 states took 3.7 ms; HBM traffic is the state in
 // and out.)  Two wavefronts per SIMD in both registers and LDS: 12,000
-// n-dodecane states TP 1.36 ms, HP 1.54 (one per SIMD 1.85 and 2.08, wavefront
+// n-dodecane states TP 1.29 ms, HP 1.45 (one per SIMD 1.85 and 2.08, wavefront
 // sums 1.53 and 2.03).
 #include <hip/hip_runtime.h>
 
@@ -40,50 +40,53 @@ constexpr double kSize = 18.420681;       // ln(1e8): trace-species threshold of
 constexpr double kTraceLn = 9.2103404;    // ln(1e4)
 
 // x <- A^-1 x, row q of A and of x in lane q < nu; false where A is singular.
-// Gaussian elimination with the exact largest pivot of a column (the first of
-// equal ones, counted along the rows as exchanged) and with quotients by it: an
-// iterate of almost one species makes element rows multiples of each other, and
-// a quotient keeps the zero that they cancel to.  With products by 1 / pivot and
-// pivots compared in 58 bits that zero became a pivot of rounding noise or not
-// as it fell, and 0.07% of hydrogen mixtures at 200 to 500 K were refused that
-// are not now.  20,011 gri30 states 1.99 -> 2.04 ms for it.
+// Gaussian elimination with the exact largest pivot of a column and with
+// quotients by it (a product by the reciprocal and a correction by its
+// remainder, so exact where the quotient is): an iterate of almost one species
+// makes element rows multiples of each other, and a quotient keeps the zero that
+// they cancel to.  With bare products by 1 / pivot and pivots compared in 58
+// bits that zero became a pivot of rounding noise or not as it fell, and 0.07%
+// of hydrogen mixtures at 200 to 500 K were refused that are not now.  20,011
+// gri30 states 1.99 -> 1.93 ms (2.04 with divisions).
 __device__ __forceinline__ bool solve_rows(double (&a)[kEqMaxNu], double& x, int nu) {
     const int lane = lane_id();
-    int pos = lane;   // where the exchanges have brought this lane's row
-    double pivot = 1.0;
+    bool open = lane < nu;   // not a pivot row yet
+    int step = kEqMaxNu;     // the column that this lane's row is the pivot of
+    double rdiag = 0.0;
     int owner[kEqMaxNu];
 #pragma unroll
     for (int c = 0; c < kEqMaxNu; c++) {
         owner[c] = 0;
         if (c >= nu) continue;
-        const double v = (lane < nu && pos >= c) ? fabs(a[c]) : -1.0;
+        const double v = open ? fabs(a[c]) : -1.0;
         double top = fmax(v, dpp_f64<0xB1>(v));
         top = fmax(top, dpp_f64<0x4E>(top));
         top = fmax(top, dpp_f64<0x124>(top));
         top = readlane_f64(fmax(top, dpp_f64<0x128>(top)), 0);
-        unsigned long long same = __ballot(v == top);
+        const unsigned long long same = __ballot(v == top);
         if (!(top > 0.0) || same == 0) return false;
-        int p = __builtin_ctzll(same), pp = __builtin_amdgcn_readlane(pos, p);
-        for (same &= same - 1; same; same &= same - 1) {
-            const int q = __builtin_ctzll(same), qp = __builtin_amdgcn_readlane(pos, q);
-            if (qp < pp) { p = q; pp = qp; }
+        const int p = owner[c] = __builtin_ctzll(same);
+        const double piv = readlane_f64(a[c], p);
+        double rp = __builtin_amdgcn_rcp(piv);
+        rp = fma(fma(-piv, rp, 1.0), rp, rp);
+        rp = fma(fma(-piv, rp, 1.0), rp, rp);
+        if (lane == p) {
+            open = false;
+            step = c;
+            rdiag = rp;
         }
-        pos = lane == p ? c : (pos == c ? pp : pos);
-        owner[c] = p;
-        pivot = lane == p ? a[c] : pivot;
-        const double q = a[c] / readlane_f64(a[c], p);
-        const double f = lane < nu && pos > c ? q : 0.0;
+        const double q0 = a[c] * rp, q = fma(fma(-q0, piv, a[c]), rp, q0);
+        const double f = open ? q : 0.0;
 #pragma unroll
         for (int j = c + 1; j < kEqMaxNu; j++) a[j] -= f * readlane_f64(a[j], p);
         x -= f * readlane_f64(x, p);
     }
-    const double rdiag = 1.0 / pivot;
     double y = 0.0;
 #pragma unroll
     for (int c = kEqMaxNu - 1; c >= 0; c--) {
         if (c >= nu) continue;
         const double xc = readlane_f64(x * rdiag, owner[c]);
-        x -= (pos < c ? a[c] : 0.0) * xc;
+        x -= (step < c ? a[c] : 0.0) * xc;
         y = lane == c ? xc : y;
     }
     x = y;
